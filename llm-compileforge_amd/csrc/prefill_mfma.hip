@@ -46,7 +46,12 @@
 //
 // Items come from a list the plan kernel sorts longest first (counting
 // sort on the tile count), so the persistent workgroups finish together
-// without splitting an item: there are no partials and no merge pass.
+// without splitting an item.  Calls with fewer items than resident
+// workgroups (a short chunk behind a long prefix is a handful of items of
+// hundreds of tiles) take the direct path instead: no plan launch, long items
+// cut along the KV range into one piece per workgroup; a piece leaves its
+// columns' (m, l, o) in a workspace slot and prefill_merge_kernel combines
+// them (direct_piece below).
 // The longest items, up to 75 % of the tiles, form eight per-XCD lists
 // (list x: sorted positions x, x + 8, ...; with Hkv a multiple of 8 these
 // are the items of heads x, x + 8, ..., so all row blocks of a (chunk, KV
@@ -55,6 +60,7 @@
 // items.  The shared tail keeps the XCDs finishing together: they do not
 // run equally fast (on the measured part the odd XCDs took ~6 % longer per
 // tile), which fully static per-XCD lists turned into a 10 % longer launch.
+#include <algorithm>
 #include <type_traits>
 
 #include "cf_device.hpp"
@@ -71,6 +77,10 @@ constexpr int kPlanThreads = 1024;
 constexpr int kCostBins = 2048;   // tile counts at or above share the last bin
 constexpr int kXcds = 8;          // workgroup g runs on XCD g % 8, each with its own L2
 constexpr int kAffinePct = 75;    // share of the tiles taken from per-XCD lists
+constexpr int kPlanChunks = 1024; // chunk records the plan kernel keeps in LDS
+constexpr int kDirectItems = 512; // most items of a direct launch (one piece per workgroup)
+constexpr int kDirectCandidates = 16;
+constexpr int kMinPieceTiles = 6; // shortest piece an item is cut into: a piece costs its (m, l, o) record and the merge
 
 __device__ __forceinline__ float wave_incl_scanf(float v, int lane) {
 #pragma unroll
@@ -86,57 +96,202 @@ __device__ __forceinline__ int item_kvlen(int pos0, int rb, int RB, int L, int c
   return max(0, min(pos0 + rb * RB + rows, cap));
 }
 
-// ---- plan: chunk rows, work items, longest-first order -------------------
+// ---- chunk rows --------------------------------------------------------------
 // Chunks are taken in order and made disjoint: chunk n covers q rows
 // [max(q_start[n], end of chunk n-1), max(q_start[n+1], that)), clamped to
-// [0, Tq).  Its rows sit at positions seq_lens[n] - L + i.
+// [0, Tq).  Its rows sit at positions seq_lens[n] - L + i.  One wave; put(n,
+// {first row, L, position of the first row, row blocks of the chunks before})
+// is called for every chunk, and the row blocks of all chunks are returned.
+template <class Put>
+__device__ __forceinline__ int chunk_rows(const PrefillParams& p, int lane, Put put) {
+  int rend = 0, nrb_run = 0;
+  for (int n0 = 0; n0 < p.N; n0 += 64) {
+    const int n = n0 + lane;
+    int a = 0, b = 0, S = 0;
+    if (n < p.N) {
+      a = min(max(p.q_start[(int64_t)n * p.qs_s], 0), p.Tq);
+      b = min(max(p.q_start[(int64_t)(n + 1) * p.qs_s], 0), p.Tq);
+      S = p.seq_lens[(int64_t)n * p.sl_s];
+    }
+    const int row1 = max(wave_incl_max(max(a, b), lane), rend);
+    int prev_end = __shfl_up(row1, 1, 64);
+    if (lane == 0) prev_end = rend;
+    const int row0 = n < p.N ? max(a, prev_end) : row1;
+    const int L = n < p.N ? row1 - row0 : 0;
+    const int nrb = (L + p.RB - 1) / p.RB;
+    const int incl = wave_incl_scan(nrb, lane) + nrb_run;
+    if (n < p.N) put(n, make_int4(row0, L, S - L, incl - nrb));
+    rend = __shfl(row1, 63, 64);
+    nrb_run = __shfl(incl, 63, 64);
+  }
+  return nrb_run;
+}
+
+// The chunk holding row block f (flattened over chunks): binary search on .w.
+template <class At>
+__device__ __forceinline__ int chunk_of(At chunk_at, int N, int f) {
+  int lo = 0, hi = N - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (chunk_at(mid).w <= f) lo = mid;
+    else hi = mid - 1;
+  }
+  return lo;
+}
+
+__device__ __forceinline__ int block_tiles(const PrefillParams& p, const int4& c, int f) {
+  return (item_kvlen(c.z, f - c.w, p.RB, c.y, p.Mb * 16) + 31) >> 5;
+}
+
+// ---- direct launches: one piece per workgroup ------------------------------
+// Calls of at most one item per resident workgroup W (every short chunk, most
+// single prompts) need no queue: each workgroup works out its own piece from
+// the chunk table, and there is no plan launch.  With T tiles in all, a
+// workgroup's share is T / W; items longer than P tiles are cut along the KV
+// range into equal pieces, P the shortest of share * (1 + k / 8), at least
+// kMinPieceTiles, for which all pieces fit the W workgroups at once.  Piece
+// number i of row block f for head h is workgroup (first piece of f + i) *
+// Hkv + h (heads fastest, so with Hkv a multiple of 8 the pieces of a head
+// read its K/V through one XCD's L2), and so is its workspace slot.
+//
+// Measured, whole calls (e4m3, 32 query / 8 KV heads of 128): 100 rows behind
+// 12,001 cached tokens 354 us (32 workgroups walking 380 tiles each) -> 46 us;
+// a 1,237-row prompt (bf16, 32 / 4 heads of 64) 50.6 -> 36.2 us.  Above W items
+// the longest-first queue is within a few percent of even shares, and cutting
+// them only adds records and a merge launch (eight 512-row chunks behind
+// 0-4,096 tokens, cut in the queue's plan: 123 us against 114 us uncut).
+struct DirectPlan {
+  int4 chunks[kDirectItems];
+  int tiles[kDirectItems];
+  int red[3][4];
+  float sum[4];
+  int pieces[kDirectCandidates];
+};
+struct DirectPiece {
+  int4 chunk;
+  int n, rb, h, jt0, nt, slot;  // chunk, row block, KV head, tiles [jt0, nt), workspace slot (-1: a whole item)
+};
+
+// Equal pieces of an item of t tiles cut at P (t, P < 2^24; every caller gets
+// the same count, whatever the rounding).
+__device__ __forceinline__ int piece_count(int t, int P) {
+  return max(1, (int)ceilf((float)t / (float)P));
+}
+
+__device__ bool direct_piece(const PrefillParams& p, DirectPlan* s, DirectPiece* out, int tid) {
+  const int lane = tid & 63, wave = uniform(tid >> 6);
+  if (wave == 0) {
+    const int nrb = chunk_rows(p, lane, [&](int n, const int4& c) { s->chunks[n] = c; });
+    if (lane == 0) s->red[0][0] = nrb;
+  }
+  if (tid < kDirectCandidates) s->pieces[tid] = 0;
+  if (tid == 0) out->n = -1;
+  __syncthreads();
+  const int nblocks = s->red[0][0];
+  __syncthreads();
+  auto chunk_at = [&](int n) { return s->chunks[n]; };
+  float sum = 0.0f;
+  int most = 0;
+  for (int f = tid; f < nblocks; f += 256) {
+    const int t = min(block_tiles(p, s->chunks[chunk_of(chunk_at, p.N, f)], f), (1 << 24) - 1);
+    s->tiles[f] = t;
+    sum += (float)t;
+    most = max(most, t);
+  }
+  sum = wave_sum(sum);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o, 64));
+  if (lane == 0) {
+    s->sum[wave] = sum;
+    s->red[1][wave] = most;
+  }
+  __syncthreads();
+  most = max(max(s->red[1][0], s->red[1][1]), max(s->red[1][2], s->red[1][3]));
+  const float share = (s->sum[0] + s->sum[1] + s->sum[2] + s->sum[3]) * (float)p.Hkv / (float)p.workers;
+  auto candidate = [&](int k) {
+    return max(kMinPieceTiles, (int)fminf(ceilf(share * (1.0f + 0.125f * k)), 16777216.0f));
+  };
+  int P = 1 << 24;
+  if (most > candidate(0)) {  // uniform
+    for (int k = wave; k < kDirectCandidates; k += 4) {
+      const int Pk = candidate(k);
+      int n = 0;
+      for (int f = lane; f < nblocks; f += 64) n += piece_count(s->tiles[f], Pk);
+      n = wave_sum_i(n);
+      if (lane == 0) s->pieces[k] = n;
+    }
+    __syncthreads();
+    for (int k = kDirectCandidates - 1; k >= 0; --k)
+      if (s->pieces[k] * p.Hkv <= p.workers) P = candidate(k);
+  }
+  // this workgroup's piece: an exclusive scan of the row blocks' piece counts
+  const int want = (int)blockIdx.x / p.Hkv;
+  int carry = 0;
+  for (int f0 = 0; f0 < nblocks; f0 += 256) {
+    const int f = f0 + tid;
+    const int n = f < nblocks ? piece_count(s->tiles[f], P) : 0;
+    const int incl = wave_incl_scan(n, lane);
+    if (lane == 63) s->red[2][wave] = incl;
+    __syncthreads();
+    int before = carry;
+    for (int w = 0; w < 4; ++w) {
+      if (w < wave) before += s->red[2][w];
+      carry += s->red[2][w];
+    }
+    const int at = before + incl - n;  // first piece of f
+    if (want >= at && want < at + n) {
+      const int i = want - at, t = s->tiles[f], q = t / n, more = t - q * n;
+      const int lo = chunk_of(chunk_at, p.N, f);
+      const int h = (int)blockIdx.x - want * p.Hkv;
+      out->chunk = s->chunks[lo];
+      out->n = lo;
+      out->rb = f - s->chunks[lo].w;
+      out->h = h;
+      out->jt0 = i * q + min(i, more);
+      out->nt = out->jt0 + q + (i < more ? 1 : 0);
+      out->slot = n > 1 ? (int)blockIdx.x : -1;
+      // what the merge needs of this item
+      if (i == 0 && p.splits != nullptr) {
+        p.splits[2 * (f * p.Hkv + h)] = make_int4(out->chunk.x + out->rb * p.RB, min(p.RB, out->chunk.y - out->rb * p.RB), h, n);
+        p.splits[2 * (f * p.Hkv + h) + 1] = make_int4(at, 0, 0, 0);
+      }
+    }
+    __syncthreads();
+  }
+  if (blockIdx.x == 0 && tid == 0 && p.splits != nullptr) p.header[11] = nblocks * p.Hkv;
+  return out->n >= 0;  // false: fewer pieces than workgroups
+}
+
+// ---- plan: chunk rows, work items, longest-first order -------------------
 __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PrefillParams p) {
   __shared__ int hist[kCostBins];
+  __shared__ int4 s_chunks[kPlanChunks];
   __shared__ int wave_tot[kPlanThreads / 64];
   __shared__ float wave_tiles[kPlanThreads / 64];
   __shared__ int s_aff;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int cap = p.Mb * 16;
+  const bool in_lds = p.N <= kPlanChunks;
   if (wave == 0) {
-    // chunk rows, and in .w the row blocks of the chunks before this one
-    int rend = 0, nrb_run = 0;
-    for (int n0 = 0; n0 < p.N; n0 += 64) {
-      const int n = n0 + lane;
-      int a = 0, b = 0, S = 0;
-      if (n < p.N) {
-        a = min(max(p.q_start[(int64_t)n * p.qs_s], 0), p.Tq);
-        b = min(max(p.q_start[(int64_t)(n + 1) * p.qs_s], 0), p.Tq);
-        S = p.seq_lens[(int64_t)n * p.sl_s];
-      }
-      const int row1 = max(wave_incl_max(max(a, b), lane), rend);
-      int prev_end = __shfl_up(row1, 1, 64);
-      if (lane == 0) prev_end = rend;
-      const int row0 = n < p.N ? max(a, prev_end) : row1;
-      const int L = n < p.N ? row1 - row0 : 0;
-      const int nrb = (L + p.RB - 1) / p.RB;
-      const int incl = wave_incl_scan(nrb, lane) + nrb_run;
-      if (n < p.N) p.chunks[n] = make_int4(row0, L, S - L, incl - nrb);
-      rend = __shfl(row1, 63, 64);
-      nrb_run = __shfl(incl, 63, 64);
-    }
-    if (lane == 0) wave_tot[0] = nrb_run;
+    const int nrb = chunk_rows(p, lane, [&](int n, const int4& c) {
+      p.chunks[n] = c;
+      if (in_lds) s_chunks[n] = c;
+    });
+    if (lane == 0) wave_tot[0] = nrb;
   }
   for (int i = tid; i < kCostBins; i += kPlanThreads) hist[i] = 0;
   if (tid == 0) s_aff = 0x7fffffff;
   __syncthreads();
   const int nblocks = wave_tot[0];  // row blocks of all chunks
   __syncthreads();
+  // (two code paths: one pointer to either would make every read a flat load)
+  auto chunk_at = [&](int n) { return in_lds ? s_chunks[n] : p.chunks[n]; };
   // Row block f (flattened over chunks): its chunk by binary search on .w;
   // items (f, h) for every KV head.  Bin kCostBins-1-tiles puts the longest
   // items first.
   for (int f = tid; f < nblocks; f += kPlanThreads) {
-    int lo = 0, hi = p.N - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (p.chunks[mid].w <= f) lo = mid;
-      else hi = mid - 1;
-    }
-    const int4 c = p.chunks[lo];
+    const int lo = chunk_of(chunk_at, p.N, f);
+    const int4 c = chunk_at(lo);
     const int tiles = (item_kvlen(c.z, f - c.w, p.RB, c.y, cap) + 31) >> 5;
     atomicAdd(&hist[kCostBins - 1 - min(tiles, kCostBins - 1)], p.Hkv);
   }
@@ -175,13 +330,8 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PrefillParam
   hist[2 * tid + 1] = excl + h0;
   __syncthreads();
   for (int f = tid; f < nblocks; f += kPlanThreads) {
-    int lo = 0, hi = p.N - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (p.chunks[mid].w <= f) lo = mid;
-      else hi = mid - 1;
-    }
-    const int4 c = p.chunks[lo];
+    const int lo = chunk_of(chunk_at, p.N, f);
+    const int4 c = chunk_at(lo);
     const int rb = f - c.w;
     const int tiles = (item_kvlen(c.z, rb, p.RB, c.y, cap) + 31) >> 5;
     const int at = atomicAdd(&hist[kCostBins - 1 - min(tiles, kCostBins - 1)], p.Hkv);
@@ -450,7 +600,10 @@ __device__ __forceinline__ void mask_staged_v(uint4* vr, const TileIds& t, int v
   }
 }
 
-template <int QT, int KT, int D, int G, bool VTOK>
+// DIRECT: one piece per workgroup (direct_piece), otherwise the queue's items;
+// a template so that the queue's loop keeps the registers it needs (as a
+// run-time flag it cost 10 VGPRs and 4 % of a queued launch).
+template <int QT, int KT, int D, int G, bool VTOK, bool DIRECT>
 __global__ __launch_bounds__(256, 2) void prefill_item_kernel(PrefillParams p, const int32_t* __restrict__ tables,
                                                               const int4* __restrict__ items,
                                                               const int4* __restrict__ chunks, int* header,
@@ -468,34 +621,50 @@ __global__ __launch_bounds__(256, 2) void prefill_item_kernel(PrefillParams p, c
   const int li = lane & 15, lq = lane >> 4;
   // list x is drained by the workgroups with blockIdx.x % 8 == x (wherever
   // they run), so a grid of fewer than 8 takes every item from the queue
-  const int n_items = header[0], n_aff = gridDim.x >= kXcds ? header[2] : 0;
+  const int n_items = DIRECT ? 0 : header[0], n_aff = DIRECT ? 0 : (gridDim.x >= kXcds ? header[2] : 0);
   const int cap = p.Mb * 16;
   // Beside the memory-bound decode kernel (a mixed step's two streams), a
-  // SIMD holds one wave of each; the prefill's, on the step's critical path,
-  // issues first.  Among the prefill's own waves the priorities are equal.
-  __builtin_amdgcn_s_setprio(2);
+  // SIMD holds one wave of each.  A queued launch outlives the decode and is
+  // the step's critical path: its waves issue first (1.7 % off a step of
+  // eight 512-row chunks and 248 decodes).  A direct launch ends first and
+  // leaves the decode its issue slots (two 512-row chunks and 61 decodes:
+  // 126 us against 138 us).  Among the prefill's own waves priorities are equal.
+  if constexpr (!DIRECT) __builtin_amdgcn_s_setprio(2);
 
   for (;;) {
-    if (tid == 0) {
-      int it = n_items;
-      if (own_list) {
-        const int pos = kXcds * atomicAdd(&header[3 + xcd], 1) + xcd;
-        if (pos < n_aff) it = pos;
-        else own_list = false;
+    // tiles [jt0, nt) of the item; slot >= 0: a piece, its columns' (m, l, o)
+    // go to that workspace slot
+    int n, rb, h, jt0 = 0, nt, slot = -1;
+    int4 ch;
+    if constexpr (DIRECT) {
+      __shared__ DirectPiece s_piece;
+      static_assert(sizeof(DirectPlan) <= sizeof(lds), "the direct plan shares the tiles' LDS");
+      if (!direct_piece(p, (DirectPlan*)lds, &s_piece, tid)) return;
+      n = uniform(s_piece.n), rb = uniform(s_piece.rb), h = uniform(s_piece.h);
+      jt0 = uniform(s_piece.jt0), nt = uniform(s_piece.nt), slot = uniform(s_piece.slot);
+      ch = s_piece.chunk;
+    } else {
+      if (tid == 0) {
+        int it = n_items;
+        if (own_list) {
+          const int pos = kXcds * atomicAdd(&header[3 + xcd], 1) + xcd;
+          if (pos < n_aff) it = pos;
+          else own_list = false;
+        }
+        if (!own_list) {
+          const int pos = n_aff + atomicAdd(&header[1], 1);
+          it = pos < n_items ? pos : n_items;
+        }
+        s_item = it;
       }
-      if (!own_list) {
-        const int pos = n_aff + atomicAdd(&header[1], 1);
-        it = pos < n_items ? pos : n_items;
-      }
-      s_item = it;
+      __syncthreads();
+      const int it = uniform(s_item);
+      __syncthreads();
+      if (it >= n_items) break;
+      const int4 item = items[it];
+      n = uniform(item.x), rb = uniform(item.y), h = uniform(item.z), nt = uniform(item.w);
+      ch = chunks[n];
     }
-    __syncthreads();
-    const int it = uniform(s_item);
-    __syncthreads();
-    if (it >= n_items) break;
-    const int4 item = items[it];
-    const int n = uniform(item.x), rb = uniform(item.y), h = uniform(item.z), nt = uniform(item.w);
-    const int4 ch = chunks[n];
     const int row0 = uniform(ch.x + rb * RB);
     const int rows = uniform(min(RB, ch.y - rb * RB));
     const int pos0 = uniform(ch.z + rb * RB);
@@ -565,15 +734,15 @@ __global__ __launch_bounds__(256, 2) void prefill_item_kernel(PrefillParams p, c
     const int32_t* trow = tables + (int64_t)n * p.t_sb;
     const int nblk = (kvlen + 15) >> 4, nfull = kvlen >> 5;
     const int64_t tsm = p.t_sm;
-    const int32_t* tp = trow + 6 * tsm;  // table entry of tile 3's first block, advanced every step
-    TileIds id0 = tile_ids(p, trow, 0, kvlen);
-    TileIds id1 = nt > 1 ? tile_ids(p, trow, 1, kvlen) : id0;
-    TileIds id2 = nt > 2 ? tile_ids(p, trow, 2, kvlen) : id1;
-    if (nt > 0) {
+    const int32_t* tp = trow + 2 * (jt0 + 3) * tsm;  // table entry of tile jt0 + 3's first block, advanced every step
+    TileIds id0 = tile_ids(p, trow, jt0, kvlen);
+    TileIds id1 = jt0 + 1 < nt ? tile_ids(p, trow, jt0 + 1, kvlen) : id0;
+    TileIds id2 = jt0 + 2 < nt ? tile_ids(p, trow, jt0 + 2, kvlen) : id1;
+    if (jt0 < nt) {
       stage_load<KT, D, VTOK>(kr, vr, p, id0, h, tid);
-      stage_write<QT, KT, D, VTOK>(lds[0], kr, vr, id0, kvlen, tid);
+      stage_write<QT, KT, D, VTOK>(lds[0], kr, vr, id0, kvlen - 32 * jt0, tid);
     }
-    if (nt > 1) stage_load<KT, D, VTOK>(kr, vr, p, id1, h, tid);
+    if (jt0 + 1 < nt) stage_load<KT, D, VTOK>(kr, vr, p, id1, h, tid);
     __syncthreads();
 
     // P in fp16 against fp16 V operands (e4m3 V converts exactly; fp16 V as
@@ -770,11 +939,25 @@ __global__ __launch_bounds__(256, 2) void prefill_item_kernel(PrefillParams p, c
       id1 = id2;
       id2 = id3;
     };
-    for (int j = 0; j < nt; j += 2) {
+    for (int j = jt0; j < nt; j += 2) {
       step(std::integral_constant<int, 0>{}, j);
       if (j + 1 < nt) step(std::integral_constant<int, 1>{}, j + 1);
     }
 
+    // ---- a piece: its used columns' (m, l) and o, in register order ---------
+    if (DIRECT && slot >= 0) {
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        if ((32 * wave + 16 * k + li) / G < rows) {
+          const int64_t ck = (int64_t)slot * 8 + 2 * wave + k;  // 16-column group of the slot
+          if (lq == 0) p.ws_ml[ck * 16 + li] = make_float2(m[k], ol[k][0]);
+          float4* os = p.ws_o + ck * NV * 64 + lane;
+#pragma unroll
+          for (int t = 0; t < NV; ++t) os[t * 64] = make_float4(o[k][t][0], o[k][t][1], o[k][t][2], o[k][t][3]);
+        }
+      }
+      break;
+    }
     // ---- normalized output --------------------------------------------------
     const float vs = vscale ? vscale[h * p.vs_s] : 1.0f;
 #pragma unroll
@@ -794,6 +977,91 @@ __global__ __launch_bounds__(256, 2) void prefill_item_kernel(PrefillParams p, c
         }
       }
     }
+    if constexpr (DIRECT) break;
+  }
+}
+
+// Combines the pieces of a direct launch's cut items: O = sum_i w_i o_i /
+// sum_i w_i l_i per column, w_i = 2^(m_i - max m) (m in log2 units).  A unit
+// is one 16-column group of one item; thread (wave, lane) holds channels
+// 16 t + 4 lq .. + 3 of column li for its wave's quarter of the t, the order
+// the pieces were written in (1 KiB runs).  It is bound by one round trip and
+// the 64 * D bytes a piece's group holds: (m, l) and o are read side by side,
+// kMergeBatch pieces at a time.
+constexpr int kMergeBatch = 4;
+
+template <int QT, int D, int G>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p, const int* __restrict__ header,
+                                                            const int4* __restrict__ splits) {
+  constexpr int NV = D / 16, TPW = NV / 4;  // channel groups per thread
+  const int lane = threadIdx.x & 63, wave = uniform((int)threadIdx.x >> 6);
+  const int li = lane & 15, lq = lane >> 4;
+  const int units = header[11] * 8;
+  for (int u = blockIdx.x; u < units; u += gridDim.x) {
+    const int4 sp = splits[2 * (u >> 3)];
+    const int first = splits[2 * (u >> 3) + 1].x;
+    const int row0 = sp.x, rows = sp.y, h = sp.z, n = sp.w;
+    const int cg = u & 7;
+    const int col = 16 * cg + li, r = col / G, g = col % G;
+    if (n < 2 || r >= rows) continue;
+    const int64_t slot = (int64_t)first * p.Hkv + h;  // piece i: slot + i * Hkv
+    const float2* ml = p.ws_ml + (slot * 8 + cg) * 16 + li;
+    const float4* po = p.ws_o + (slot * 8 + cg) * NV * 64 + (wave * TPW) * 64 + lane;
+    const int64_t ml_s = (int64_t)p.Hkv * 8 * 16, po_s = (int64_t)p.Hkv * 8 * NV * 64;
+    float M = -INFINITY, L = 0.0f;
+    float4 acc[TPW];
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) acc[t] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int i0 = 0; i0 < n; i0 += kMergeBatch) {
+      float2 mlv[kMergeBatch];
+      float4 ov[kMergeBatch][TPW];
+#pragma unroll
+      for (int b = 0; b < kMergeBatch; ++b) {
+        const int i = min(i0 + b, n - 1);  // past the end: the last piece again, not used
+        mlv[b] = ml[i * ml_s];
+#pragma unroll
+        for (int t = 0; t < TPW; ++t) ov[b][t] = po[i * po_s + t * 64];
+      }
+      float mnew = M;
+#pragma unroll
+      for (int b = 0; b < kMergeBatch; ++b) mnew = fmaxf(mnew, mlv[b].x);
+      const float alpha = M == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(M - mnew);
+      L *= alpha;
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) {
+        acc[t].x *= alpha;
+        acc[t].y *= alpha;
+        acc[t].z *= alpha;
+        acc[t].w *= alpha;
+      }
+#pragma unroll
+      for (int b = 0; b < kMergeBatch; ++b) {
+        const bool use = i0 + b < n && mlv[b].x != -INFINITY;
+        const float w = use ? __builtin_amdgcn_exp2f(mlv[b].x - mnew) : 0.0f;
+        if (use) {
+          L += w * mlv[b].y;
+#pragma unroll
+          for (int t = 0; t < TPW; ++t) {
+            acc[t].x += w * ov[b][t].x;
+            acc[t].y += w * ov[b][t].y;
+            acc[t].z += w * ov[b][t].z;
+            acc[t].w += w * ov[b][t].w;
+          }
+        }
+      }
+      M = mnew;
+    }
+    const float vs = p.v_scale ? p.v_scale[h * p.vs_s] : 1.0f;
+    const float inv = L > 0.0f ? vs / L : 0.0f;
+    uint16_t* orow = (uint16_t*)p.out + (int64_t)(row0 + r) * p.o_sr + (int64_t)(h * G + g) * p.o_sh +
+                     16 * wave * TPW + 4 * lq;
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) {
+      uint2 packed;
+      packed.x = (uint32_t)out_bits<QT>(acc[t].x * inv) | ((uint32_t)out_bits<QT>(acc[t].y * inv) << 16);
+      packed.y = (uint32_t)out_bits<QT>(acc[t].z * inv) | ((uint32_t)out_bits<QT>(acc[t].w * inv) << 16);
+      *(uint2*)(orow + 16 * t) = packed;
+    }
   }
 }
 
@@ -805,18 +1073,50 @@ int prefill_cus() {
 }
 
 constexpr int kItemBlocksPerCU = 2;  // resident workgroups per CU (8 waves)
+constexpr int kMergeBlocks = 1024;
 
-template <int QT, int KT, int D, int G, bool VTOK>
-int32_t launch_t(PrefillParams& p, hipStream_t stream) {
+template <int QT, int KT, int D, int G, bool VTOK, bool DIRECT>
+int item_workers() {
   static int per_cu = 0;
   if (per_cu == 0) {
     int n = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, prefill_item_kernel<QT, KT, D, G, VTOK>, 256, 0) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, prefill_item_kernel<QT, KT, D, G, VTOK, DIRECT>, 256, 0) !=
             hipSuccess ||
         n < 1)
       n = 1;
     per_cu = n < kItemBlocksPerCU ? n : kItemBlocksPerCU;
   }
+  return prefill_cus() * per_cu;
+}
+
+// Calls of at most one item per resident workgroup: one piece per workgroup
+// (direct_piece), and the merge of the cut items.
+template <int QT, int KT, int D, int G, bool VTOK>
+int32_t launch_direct(PrefillParams& p, hipStream_t stream) {
+  // no item is longer than the tables' capacity, so short tables bound the
+  // pieces, and where one piece holds any item there is nothing to merge
+  const int64_t most = std::max<int64_t>(ceil_div((int64_t)p.Mb * 16, 32 * kMinPieceTiles), 1);
+  if (most == 1) p.splits = nullptr;
+  {
+    ProfileScope prof("cf_prefill_mfma", stream);
+    CF_LAUNCH((prefill_item_kernel<QT, KT, D, G, VTOK, true>),
+              dim3((unsigned)std::min<int64_t>(p.workers, p.max_items * most)), dim3(256), 0, stream, p, p.tables,
+              (const int4*)p.items, (const int4*)p.chunks, p.header, p.k_scale, p.v_scale);
+  }
+  CF_HIP_CHECK(hipGetLastError());
+  if (p.splits != nullptr) {
+    ProfileScope prof("cf_prefill_merge", stream);
+    CF_LAUNCH((prefill_merge_kernel<QT, D, G>), dim3(std::min(8 * p.max_items, kMergeBlocks)), dim3(256), 0, stream, p,
+              (const int*)p.header, (const int4*)p.splits);
+    CF_HIP_CHECK(hipGetLastError());
+  }
+  return CF_OK;
+}
+
+template <int QT, int KT, int D, int G, bool VTOK>
+int32_t launch_t(PrefillParams& p, hipStream_t stream) {
+  p.workers = item_workers<QT, KT, D, G, VTOK, true>();
+  if (p.max_items <= std::min(p.workers, p.split_slots)) return launch_direct<QT, KT, D, G, VTOK>(p, stream);
   {
     ProfileScope prof("cf_prefill_plan", stream);
     CF_LAUNCH(prefill_plan_kernel, dim3(1), dim3(kPlanThreads), 0, stream, p);
@@ -824,8 +1124,9 @@ int32_t launch_t(PrefillParams& p, hipStream_t stream) {
   CF_HIP_CHECK(hipGetLastError());
   {
     ProfileScope prof("cf_prefill_mfma", stream);
-    CF_LAUNCH((prefill_item_kernel<QT, KT, D, G, VTOK>), dim3(prefill_cus() * per_cu), dim3(256), 0, stream, p,
-                       p.tables, (const int4*)p.items, (const int4*)p.chunks, p.header, p.k_scale, p.v_scale);
+    CF_LAUNCH((prefill_item_kernel<QT, KT, D, G, VTOK, false>), dim3(item_workers<QT, KT, D, G, VTOK, false>()),
+              dim3(256), 0, stream, p, p.tables, (const int4*)p.items, (const int4*)p.chunks, p.header, p.k_scale,
+              p.v_scale);
   }
   CF_HIP_CHECK(hipGetLastError());
   return CF_OK;
@@ -893,22 +1194,41 @@ bool prefill_supported(const PrefillParams& p, int q_dt, int kv_dt) {
 
 int prefill_rows_per_item(int G) { return kCols / G; }
 
-// Workspace: [chunks int4 x N][items int4 x max_items][header 11 int]
+// Slots for the pieces of a direct launch, one per resident workgroup; none
+// when the call may hold more items than that (queued launches cut nothing).
+int64_t split_slots_of(int64_t max_items) {
+  const int64_t w = std::min<int64_t>((int64_t)prefill_cus() * kItemBlocksPerCU, kDirectItems);
+  return max_items <= w ? w : 0;
+}
+
+// Workspace: [chunks int4 x N][items int4 x max_items][header 12 int], and
+// for direct launches [merge records 2 int4 x max_items][(m, l) float2 x 128
+// per slot][o float x 128 x D per slot]
 uint64_t prefill_workspace_bytes(int64_t Tq, int64_t N, int64_t Hq, int64_t Hkv, int64_t D) {
-  (void)D;
   const int64_t G = Hkv > 0 ? Hq / Hkv : 1;
-  const int64_t RB = G > 0 ? kCols / G : 1;
-  const uint64_t max_items = (uint64_t)(Tq / RB + N) * (uint64_t)Hkv;
-  return pad256((uint64_t)N * 16) + pad256(max_items * 16) + 256;
+  const int64_t RB = std::max<int64_t>(G > 0 ? kCols / G : 1, 1);
+  const int64_t max_items = (Tq / RB + N) * Hkv;
+  const uint64_t slots = (uint64_t)split_slots_of(max_items);
+  const uint64_t base = pad256((uint64_t)N * 16) + pad256((uint64_t)max_items * 16) + 256;
+  if (slots == 0) return base;
+  return base + pad256((uint64_t)max_items * 32) + pad256(slots * kCols * 8) + slots * kCols * (uint64_t)D * 4;
 }
 
 void prefill_bind_workspace(PrefillParams& p, void* workspace) {
+  const uint64_t slots = (uint64_t)split_slots_of(p.max_items);
+  p.split_slots = (int)slots;
   char* w = (char*)workspace;
   p.chunks = (int4*)w;
   w += pad256((uint64_t)p.N * 16);
   p.items = (int4*)w;
   w += pad256((uint64_t)p.max_items * 16);
   p.header = (int*)w;
+  w += 256;
+  p.splits = (int4*)w;
+  w += pad256((uint64_t)p.max_items * 32);
+  p.ws_ml = (float2*)w;
+  w += pad256(slots * kCols * 8);
+  p.ws_o = (float4*)w;
 }
 
 int32_t launch_prefill(PrefillParams& p, int q_dt, int kv_dt, hipStream_t stream) {

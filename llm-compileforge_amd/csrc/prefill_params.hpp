@@ -31,7 +31,12 @@ struct PrefillParams {
   // workspace
   int4* chunks;  // [N] {first q row, rows, position of the first row, row blocks before it}
   int4* items;   // [max_items] {chunk, row block, KV head, tiles}, longest first
-  int* header;   // {items, shared queue counter, items in the per-XCD lists, 8 list counters}
+  int* header;   // {items, shared queue counter, items in the per-XCD lists, 8 list counters, direct launch's items}
+  int4* splits;  // direct launches, per item: {first q row, rows, KV head, pieces}, {first piece}; null: never cut
+  float2* ws_ml;  // [split_slots][128] a piece's (m in log2 units, l) per column
+  float4* ws_o;   // [split_slots][128 * D / 4] its un-normalized output
+  int split_slots;  // slots for pieces (0: the call may hold more items than workgroups)
+  int workers;      // direct launches: resident workgroups of the item kernel
 };
 
 // Query rows per work item for GQA group G.

@@ -361,3 +361,29 @@ def test_rejects_unsupported(gpu):
     t = workloads.materialize_mixed(case)
     with pytest.raises(NotImplementedError):
         _prefill(case, t)
+
+
+@pytest.mark.parametrize("chunks,cached", [
+    ([33], [3967]),            # one row past a row block, a table that ends inside a block
+    ([1], [191]),              # 6 tiles: the longest item that is never cut
+    ([1, 5], [192, 2000]),     # 7 tiles beside a longer item
+    ([100, 7, 16], [3001, 0, 700]),  # cut, whole and one-tile items in one call
+])
+@pytest.mark.parametrize("hq,hkv,d,kv_dtype,layout", [
+    (32, 8, 128, torch.float8_e4m3fn, "paired"),
+    (8, 8, 64, torch.bfloat16, "native"),
+    (16, 1, 128, torch.bfloat16, "token_major"),
+    (12, 12, 64, torch.float8_e4m3fn, "token_major"),
+])
+def test_items_cut_along_the_kv_range_match_oracle(gpu, chunks, cached, hq, hkv, d, kv_dtype, layout):
+    """Few items behind long prefixes: the plan cuts them into pieces whose
+    partial outputs the merge kernel combines."""
+    print(f"[case] cut prefill {chunks} behind {cached} hq={hq} hkv={hkv} d={d} kv={kv_dtype} {layout}", flush=True)
+    case = workloads.make_mixed_case(device=gpu, seed=5, chunks=chunks, cached=cached, decode_lens=[],
+                                     num_q_heads=hq, num_kv_heads=hkv, head_dim=d, kv_dtype=kv_dtype)
+    t = workloads.materialize_mixed(case, layout)
+    _write_new_rows(case, t)
+    out = _prefill(case, t)
+    ref, covered = oracle_prefill(case, t)
+    assert covered.all()
+    assert_close(out.float().cpu().numpy(), ref, torch.bfloat16, "cut prefill")
