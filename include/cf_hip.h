@@ -259,6 +259,27 @@ int32_t cf_fp8_quantize_kv(const CfTensor* k, const CfTensor* v,
                            const CfTensor* k_scales, const CfTensor* v_scales,
                            CfTensor* k_out, CfTensor* v_out, void* stream);
 
+/* Scales and codes of one tensor, or of two of one shape and dtype (K and V;
+ * y, y_scales and y_out NULL for one): x_scales[h] is cf_fp8_amax_scale's,
+ * x_out cf_fp8_quantize's with it, in at most two launches
+ * (FP8KVCacheQuantizer.quantize_block / quantize_kv,
+ * compiler/quantize/fp8_kv_cache.py:66-93, :107-122).
+ *   x, y [S0,S1,H,Dx] or [T,H,Dx] f32|f16|bf16; scales [H] f32; outs e4m3fn.
+ *   workspace: 4096 * H bytes, 256-byte aligned.
+ * CF_ERR_UNSUPPORTED (nothing launched) unless every tensor is contiguous and
+ * 16-byte aligned, Dx is a multiple of 16 and H is at most 64. */
+int32_t cf_fp8_scale_quantize(const CfTensor* x, const CfTensor* y,
+                              CfTensor* x_scales, CfTensor* y_scales,
+                              CfTensor* x_out, CfTensor* y_out,
+                              void* workspace, uint64_t workspace_bytes,
+                              void* stream);
+
+/* cf_fp8_dequantize of K and V (own scales) in one call; one launch when all
+ * four tensors are contiguous and the shapes agree. */
+int32_t cf_fp8_dequantize_kv(const CfTensor* k, const CfTensor* v,
+                             const CfTensor* k_scales, const CfTensor* v_scales,
+                             CfTensor* k_out, CfTensor* v_out, void* stream);
+
 /* out[t,h,d] = f32(q[t,h,d]) * scales[h].
  * Reference compiler/quantize/fp8_kv_cache.py:95-105.
  *   q [T,H,Dx] or [S0,S1,H,Dx] e4m3fn; scales [H] or [1] f32;

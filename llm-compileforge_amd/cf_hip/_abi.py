@@ -165,6 +165,9 @@ SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
     "cf_kv_amax_scale": (ctypes.c_int32, [_P, _P, ctypes.c_void_p]),
     "cf_fp8_quantize": (ctypes.c_int32, [_P, _P, _P, ctypes.c_void_p]),
     "cf_fp8_quantize_kv": (ctypes.c_int32, [_P, _P, _P, _P, _P, _P, ctypes.c_void_p]),
+    "cf_fp8_scale_quantize": (ctypes.c_int32, [_P, _P, _P, _P, _P, _P, ctypes.c_void_p, ctypes.c_uint64,
+                                               ctypes.c_void_p]),
+    "cf_fp8_dequantize_kv": (ctypes.c_int32, [_P, _P, _P, _P, _P, _P, ctypes.c_void_p]),
     "cf_fp8_dequantize": (ctypes.c_int32, [_P, _P, _P, ctypes.c_void_p]),
     "cf_kv_write_fp8": (ctypes.c_int32, [_P, _P, _P, _P, _P, _P, _P, ctypes.c_void_p]),
     "cf_paged_write": (ctypes.c_int32, [_P, _P, _P, _P, ctypes.c_void_p]),

@@ -384,6 +384,54 @@ def fp8_quantize_kv(k: torch.Tensor, v: torch.Tensor, k_scales: torch.Tensor, v_
     return k_out, v_out
 
 
+def fp8_scale_quantize(*xs: torch.Tensor, per_head: bool) -> list[tuple[torch.Tensor, torch.Tensor]] | None:
+    """(codes, scales) of one or two tensors in at most two launches: the
+    results of fp8_amax_scale and fp8_quantize with one scale per head (axis
+    -2, scales [H]) or one in total (scales [1]).  None where the tensors'
+    shapes, strides or alignment need the separate calls."""
+    x0 = xs[0]
+    n = x0.numel()
+    if n == 0 or n % 16 or not all(
+            x.is_cuda and x.is_contiguous() and x.shape == x0.shape and x.dtype == x0.dtype and x.device == x0.device
+            for x in xs):
+        return None
+    if per_head and (x0.dim() < 2 or x0.shape[-1] % 16):
+        return None
+    heads = x0.shape[-2] if per_head else 1
+    shape = (-1, heads, x0.shape[-1] if per_head else 16)
+    codes = [torch.empty(x.shape, dtype=torch.float8_e4m3fn, device=x.device) for x in xs]
+    scales = [torch.empty(heads, dtype=torch.float32, device=x.device) for x in xs]
+    ws = torch.empty(4096 * heads, dtype=torch.uint8, device=x0.device)
+    dx = [descriptor(x.view(shape)) for x in xs]
+    dc = [descriptor(c.view(shape)) for c in codes]
+    ds = [descriptor(s) for s in scales]
+    two = len(xs) == 2
+    with _on(x0.device):
+        rc = lib().cf_fp8_scale_quantize(
+            ref(dx[0]), ref(dx[1]) if two else None, ref(ds[0]), ref(ds[1]) if two else None, ref(dc[0]),
+            ref(dc[1]) if two else None, ws.data_ptr(), ws.numel(), stream_handle(x0.device))
+    if rc == _abi.CF_ERR_UNSUPPORTED:
+        return None
+    check(rc, "cf_fp8_scale_quantize")
+    return list(zip(codes, scales))
+
+
+def fp8_dequantize_kv(k: torch.Tensor, v: torch.Tensor, k_scales: torch.Tensor,
+                      v_scales: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+    """(f32(k) * k_scales[h], f32(v) * v_scales[h]); one launch for
+    contiguous tensors of one shape."""
+    for name, t in (("k", k), ("v", v), ("k_scales", k_scales), ("v_scales", v_scales)):
+        _require_device(name, t)
+    dev = _same_device(k, v, k_scales, v_scales)
+    outs = [torch.empty(x.shape, dtype=torch.float32, device=dev) for x in (k, v)]
+    d = [descriptor(x) for x in (_as3(k), _as3(v), k_scales.reshape(-1), v_scales.reshape(-1), _as3(outs[0]),
+                                 _as3(outs[1]))]
+    with _on(dev):
+        rc = lib().cf_fp8_dequantize_kv(*(ref(x) for x in d), stream_handle(dev))
+    check(rc, "cf_fp8_dequantize_kv")
+    return outs[0], outs[1]
+
+
 def fp8_dequantize(q: torch.Tensor, scales: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
     """f32(q) * scales[h]."""
     _require_device("q", q)
@@ -622,6 +670,8 @@ __all__ = [
     "run_concurrent",
     "fp8_amax_scale",
     "fp8_dequantize",
+    "fp8_dequantize_kv",
+    "fp8_scale_quantize",
     "fp8_quantize",
     "fp8_quantize_kv",
     "kv_write_fp8",

@@ -638,6 +638,78 @@ int32_t cf_fp8_quantize_kv(const CfTensor* k, const CfTensor* v, const CfTensor*
   return launch_quantize_kv(k4, v4, vk.dtype, ksp, kss, vsp, vss, ko4, vo4, as_stream(stream));
 }
 
+int32_t cf_fp8_scale_quantize(const CfTensor* x, const CfTensor* y, CfTensor* x_scales, CfTensor* y_scales,
+                              CfTensor* x_out, CfTensor* y_out, void* workspace, uint64_t workspace_bytes,
+                              void* stream) {
+  const CfTensor* in[2] = {x, y};
+  CfTensor* sc[2] = {x_scales, y_scales};
+  CfTensor* ou[2] = {x_out, y_out};
+  const int count = y != nullptr ? 2 : 1;
+  Rank4 xr[2], outr[2];
+  float* sp[2] = {nullptr, nullptr};
+  int dt = CF_F32;
+  int32_t rc;
+  for (int i = 0; i < count; ++i) {
+    View vx, vo, vs;
+    if ((rc = view_of_34(in[i], "x", &vx))) return rc;
+    if ((rc = view_of_34(ou[i], "out", &vo))) return rc;
+    if ((rc = view_of(sc[i], "scales", 1, &vs))) return rc;
+    CF_CHECK(is_float_dtype(vx.dtype), "x: dtype must be f32, f16 or bf16, got %s", dtype_name(vx.dtype));
+    CF_CHECK(vo.dtype == CF_F8E4M3FN, "out: expected f8e4m3fn, got %s", dtype_name(vo.dtype));
+    CF_CHECK(vs.dtype == CF_F32, "scales: expected f32, got %s", dtype_name(vs.dtype));
+    xr[i] = rank4_of(vx);
+    outr[i] = rank4_of(vo);
+    for (int d = 0; d < 4; ++d) CF_CHECK(outr[i].size[d] == xr[i].size[d], "out shape differs from x");
+    CF_CHECK(vs.size[0] == xr[i].size[2], "scales has %lld entries, x has %lld heads", (long long)vs.size[0],
+             (long long)xr[i].size[2]);
+    CF_CHECK(vs.stride[0] == 1 || vs.size[0] <= 1, "scales must be contiguous");
+    CF_CHECK(i == 0 || vx.dtype == dt, "both tensors must have one dtype");
+    dt = vx.dtype;
+    sp[i] = (float*)vs.base;
+  }
+  if (!scale_quantize_ok(xr, outr, count, dt)) {
+    set_error("scale_quantize: needs contiguous 16-byte aligned tensors of one shape, rows a multiple of 16, at most "
+              "64 heads");
+    return CF_ERR_UNSUPPORTED;
+  }
+  const uint64_t need = scale_quantize_workspace_bytes(xr[0].size[2]);
+  if (workspace == nullptr || workspace_bytes < need) {
+    set_error("workspace of %llu bytes needed, %llu given", (unsigned long long)need,
+              (unsigned long long)workspace_bytes);
+    return CF_ERR_WORKSPACE;
+  }
+  CF_CHECK(((uintptr_t)workspace & 255) == 0, "workspace must be 256-byte aligned");
+  return launch_scale_quantize(xr, outr, sp, count, dt, workspace, as_stream(stream));
+}
+
+int32_t cf_fp8_dequantize_kv(const CfTensor* k, const CfTensor* v, const CfTensor* k_scales, const CfTensor* v_scales,
+                             CfTensor* k_out, CfTensor* v_out, void* stream) {
+  const CfTensor* in[2] = {k, v};
+  const CfTensor* sc[2] = {k_scales, v_scales};
+  CfTensor* ou[2] = {k_out, v_out};
+  Rank4 q[2], o[2];
+  const float* sp[2];
+  int64_t ss[2];
+  int32_t rc;
+  for (int i = 0; i < 2; ++i) {
+    View vq, vo;
+    if ((rc = view_of_34(in[i], "q", &vq))) return rc;
+    if ((rc = view_of_34(ou[i], "out", &vo))) return rc;
+    CF_CHECK(vq.dtype == CF_F8E4M3FN, "q: expected f8e4m3fn, got %s", dtype_name(vq.dtype));
+    CF_CHECK(vo.dtype == CF_F32, "out: expected f32, got %s", dtype_name(vo.dtype));
+    q[i] = rank4_of(vq);
+    o[i] = rank4_of(vo);
+    for (int d = 0; d < 4; ++d) CF_CHECK(o[i].size[d] == q[i].size[d], "out shape differs from q");
+    if ((rc = scale_view(sc[i], "scales", q[i].size[2], &sp[i], &ss[i]))) return rc;
+  }
+  bool same = true;
+  for (int d = 0; d < 4; ++d) same = same && q[0].size[d] == q[1].size[d];
+  if (same && dequantize_dense_ok(q[0], o[0]) && dequantize_dense_ok(q[1], o[1]))
+    return launch_dequantize_dense(q, sp, ss, o, 2, as_stream(stream));
+  if ((rc = launch_dequantize(q[0], sp[0], ss[0], o[0], as_stream(stream)))) return rc;
+  return launch_dequantize(q[1], sp[1], ss[1], o[1], as_stream(stream));
+}
+
 int32_t cf_fp8_dequantize(const CfTensor* q, const CfTensor* scales, CfTensor* out, void* stream) {
   View vq, vo;
   int32_t rc;

@@ -52,20 +52,18 @@ __global__ __launch_bounds__(256) void amax_kernel(Rank4 x, uint32_t* amax_bits,
   if ((threadIdx.x & 63) == 0 && m != 0u) atomicMax(amax_bits + h, m);
 }
 
+__device__ __forceinline__ float scale_from_amax(float amax) {
+  if (amax == 0.0f) return 1.0f;
+  const float s = amax / 448.0f;
+  // torch.clamp(min=1e-12): NaN stays NaN, values below the bound are raised.
+  return s < 1e-12f ? 1e-12f : s;
+}
+
 __global__ void scale_from_amax_kernel(uint32_t* scale_bits, int64_t stride, int H) {
   const int h = blockIdx.x * blockDim.x + threadIdx.x;
   if (h >= H) return;
   uint32_t* slot = scale_bits + h * stride;
-  const float amax = u2f(*slot);
-  float s;
-  if (amax == 0.0f) {
-    s = 1.0f;
-  } else {
-    s = amax / 448.0f;
-    // torch.clamp(min=1e-12): NaN stays NaN, values below the bound are raised.
-    if (s < 1e-12f) s = 1e-12f;
-  }
-  *slot = f2u(s);
+  *slot = f2u(scale_from_amax(u2f(*slot)));
 }
 
 // ---- quantize / dequantize ----------------------------------------------
@@ -630,6 +628,266 @@ __global__ __launch_bounds__(256) void quantize_kv_tiles_kernel(Rank4 k, Rank4 v
   }
 }
 
+// ---- scale and quantize in one call (contiguous tensors) --------------------
+// Tensors of [.., H, D] values in one contiguous run, up to two (K and V) side
+// by side: piece k is 16 values of head (k / np) % H, np = D / 16.
+struct DenseQuant {
+  const char* x[2];
+  char* out[2];
+  float* scales[2];  // [H]
+  uint32_t* parts;   // [2][kPartWgs][H] amax bits of the first pass's workgroups
+  int n;             // pieces per tensor
+  int H, np, P;      // P = H * np
+};
+
+constexpr int kPartWgs = 512;      // first-pass workgroups per tensor, at most
+constexpr int kDenseHeads = 64;    // most heads of these kernels
+constexpr int kDenseBatch = 4;     // pieces a thread keeps in flight
+constexpr int kOneWgThreads = 1024;
+constexpr int kOneWgPieces = 2;    // pieces per thread of the one-workgroup kernel
+
+template <int XT>
+__device__ __forceinline__ uint32_t amax_bits16(const uint4* raw) {
+  float f[16];
+  unpack16<XT>(raw, f);
+  uint32_t m = 0u;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    const uint32_t u = f2u(f[e]) & 0x7FFFFFFFu;
+    m = m > u ? m : u;
+  }
+  return m;
+}
+
+// First pass: each workgroup's amax bits per head, stored (not accumulated:
+// nothing needs clearing, and no workgroup waits on an address the others
+// raise: with atomicMax on H addresses 2048 workgroups that end together
+// queued on them, 77 us for K and V of 33.5 MB of bf16 and one scale each;
+// 13.5 us here, 5.0 TB/s).
+template <int XT>
+__global__ __launch_bounds__(256) void amax_parts_kernel(DenseQuant p) {
+  constexpr int EB = sizeof(typename Elem<XT>::T);
+  __shared__ uint32_t hmax[kDenseHeads];
+  const int tid = threadIdx.x;
+  if (tid < p.H) hmax[tid] = 0u;
+  __syncthreads();
+  const char* x = p.x[blockIdx.y];
+  const int stride = gridDim.x * 256;
+  const int dr = stride % p.P;
+  int rem = (int)((blockIdx.x * 256u + tid) % (uint32_t)p.P);
+  int cur = rem / p.np;
+  uint32_t m = 0u;
+  for (int k0 = blockIdx.x * 256 + tid; k0 < p.n; k0 += kDenseBatch * stride) {
+    uint4 raw[kDenseBatch][EB];
+#pragma unroll
+    for (int b = 0; b < kDenseBatch; ++b) {
+      const int k = k0 + b * stride;
+      if (k < p.n) {
+#pragma unroll
+        for (int i = 0; i < EB; ++i) raw[b][i] = *(const uint4*)(x + (int64_t)k * 16 * EB + 16 * i);
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < kDenseBatch; ++b) {
+      if (k0 + b * stride < p.n) {
+        const int h = rem / p.np;
+        if (h != cur) {
+          if (m != 0u) atomicMax(&hmax[cur], m);
+          cur = h;
+          m = 0u;
+        }
+        const uint32_t u = amax_bits16<XT>(raw[b]);
+        m = m > u ? m : u;
+      }
+      rem += dr;
+      if (rem >= p.P) rem -= p.P;
+    }
+  }
+  if (p.H == 1) m = wave_umax(m);
+  if (p.H != 1 || (tid & 63) == 0) {
+    if (m != 0u) atomicMax(&hmax[cur], m);
+  }
+  __syncthreads();
+  if (tid < p.H) p.parts[((int64_t)blockIdx.y * kPartWgs + blockIdx.x) * p.H + tid] = hmax[tid];
+}
+
+// Second pass: every workgroup reduces the first pass's maxima to the scales
+// (a few KB from L2, while its first pieces are in flight), the first one
+// stores them, and all quantize.
+template <int XT>
+__global__ __launch_bounds__(256) void quantize_parts_kernel(DenseQuant p, int nparts) {
+  constexpr int EB = sizeof(typename Elem<XT>::T);
+  __shared__ uint32_t hmax[kDenseHeads];
+  __shared__ float sc[kDenseHeads], rc[kDenseHeads];
+  const int tid = threadIdx.x;
+  const char* x = p.x[blockIdx.y];
+  char* out = p.out[blockIdx.y];
+  const int stride = gridDim.x * 256;
+  int k0 = blockIdx.x * 256 + tid;
+  uint4 raw[kDenseBatch][EB];
+  auto load = [&](int k) {
+#pragma unroll
+    for (int b = 0; b < kDenseBatch; ++b) {
+      const int kk = k + b * stride;
+      if (kk < p.n) {
+#pragma unroll
+        for (int i = 0; i < EB; ++i) raw[b][i] = stream_load16(x + (int64_t)kk * 16 * EB + 16 * i);
+      }
+    }
+  };
+  load(k0);
+  if (tid < p.H) hmax[tid] = 0u;
+  __syncthreads();
+  const uint32_t* parts = p.parts + (int64_t)blockIdx.y * kPartWgs * p.H;
+  if (p.H == 1) {
+    uint32_t m = 0u;
+    for (int i = tid; i < nparts; i += 256) m = m > parts[i] ? m : parts[i];
+    m = wave_umax(m);
+    if ((tid & 63) == 0) atomicMax(&hmax[0], m);
+  } else {
+    for (int i = tid; i < nparts * p.H; i += 256) atomicMax(&hmax[i % p.H], parts[i]);
+  }
+  __syncthreads();
+  if (tid < p.H) {
+    const float s = scale_from_amax(u2f(hmax[tid]));
+    sc[tid] = s;
+    rc[tid] = 1.0f / s;
+    if (blockIdx.x == 0) p.scales[blockIdx.y][tid] = s;
+  }
+  __syncthreads();
+  while (k0 < p.n) {
+#pragma unroll
+    for (int b = 0; b < kDenseBatch; ++b) {
+      const int k = k0 + b * stride;
+      if (k < p.n) {
+        float f[16];
+        unpack16<XT>(raw[b], f);
+        const int h = p.H == 1 ? 0 : (k / p.np) % p.H;
+        const Fp8Quant qz(sc[h], rc[h]);
+        stream_store16(out + (int64_t)k * 16, qz.pack16(f));
+      }
+    }
+    k0 += kDenseBatch * stride;
+    load(k0);
+  }
+}
+
+// A KV block or two (at most kOneWgThreads * kOneWgPieces pieces): one
+// workgroup per tensor keeps the values in registers between the two passes,
+// so the call is one launch.
+template <int XT>
+__global__ __launch_bounds__(kOneWgThreads) void quantize_small_kernel(DenseQuant p) {
+  constexpr int EB = sizeof(typename Elem<XT>::T);
+  __shared__ uint32_t hmax[kDenseHeads];
+  __shared__ float sc[kDenseHeads], rc[kDenseHeads];
+  const int tid = threadIdx.x;
+  const char* x = p.x[blockIdx.x];
+  uint4 raw[kOneWgPieces][EB];
+#pragma unroll
+  for (int b = 0; b < kOneWgPieces; ++b) {
+    const int k = tid + b * kOneWgThreads;
+    if (k < p.n) {
+#pragma unroll
+      for (int i = 0; i < EB; ++i) raw[b][i] = *(const uint4*)(x + (int64_t)k * 16 * EB + 16 * i);
+    }
+  }
+  if (tid < p.H) hmax[tid] = 0u;
+  __syncthreads();
+  if (p.H == 1) {
+    uint32_t m = 0u;
+#pragma unroll
+    for (int b = 0; b < kOneWgPieces; ++b) {
+      if (tid + b * kOneWgThreads < p.n) {
+        const uint32_t u = amax_bits16<XT>(raw[b]);
+        m = m > u ? m : u;
+      }
+    }
+    m = wave_umax(m);
+    if ((tid & 63) == 0 && m != 0u) atomicMax(&hmax[0], m);
+  } else {
+#pragma unroll
+    for (int b = 0; b < kOneWgPieces; ++b) {
+      const int k = tid + b * kOneWgThreads;
+      if (k < p.n) {
+        const uint32_t u = amax_bits16<XT>(raw[b]);
+        if (u != 0u) atomicMax(&hmax[(k / p.np) % p.H], u);
+      }
+    }
+  }
+  __syncthreads();
+  if (tid < p.H) {
+    const float s = scale_from_amax(u2f(hmax[tid]));
+    sc[tid] = s;
+    rc[tid] = 1.0f / s;
+    p.scales[blockIdx.x][tid] = s;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int b = 0; b < kOneWgPieces; ++b) {
+    const int k = tid + b * kOneWgThreads;
+    if (k < p.n) {
+      float f[16];
+      unpack16<XT>(raw[b], f);
+      const int h = p.H == 1 ? 0 : (k / p.np) % p.H;
+      const Fp8Quant qz(sc[h], rc[h]);
+      *(uint4*)(p.out[blockIdx.x] + (int64_t)k * 16) = qz.pack16(f);
+    }
+  }
+}
+
+// f32(code) * scale over contiguous runs, up to two tensors: a thread takes
+// kDenseBatch words of 4 codes, 256 words apart, so that the wave's loads and
+// its 16-byte stores are both whole runs (a thread of 16 consecutive codes
+// stores 64 bytes apart: 63 us for 2 x 16.8 M codes; 28 us here, 6.0 TB/s).
+struct DenseDequant {
+  const uint32_t* q[2];
+  const float* scales[2];
+  int64_t s_stride[2];
+  float4* out[2];
+  int64_t n;   // words per tensor
+  int H, dw;   // heads, words per row of one head
+};
+
+__global__ __launch_bounds__(256) void dequantize_dense_kernel(DenseDequant p) {
+  const uint32_t* q = p.q[blockIdx.y];
+  float4* out = p.out[blockIdx.y];
+  const float* scales = p.scales[blockIdx.y];
+  const int64_t ss = p.s_stride[blockIdx.y];
+  const int64_t k0 = (int64_t)blockIdx.x * (256 * kDenseBatch) + threadIdx.x;
+  const bool small = p.n <= (int64_t)UINT32_MAX;  // 32-bit divisions
+  auto head = [&](int64_t k) {
+    if (small) return (int64_t)((uint32_t)k / (uint32_t)p.dw % (uint32_t)p.H);
+    return k / p.dw % p.H;
+  };
+  uint32_t w[kDenseBatch];
+  float s[kDenseBatch];
+#pragma unroll
+  for (int b = 0; b < kDenseBatch; ++b) {
+    const int64_t k = k0 + 256 * b;
+    if (k < p.n) {
+      w[b] = q[k];
+      s[b] = scales[p.H == 1 ? 0 : head(k) * ss];
+    }
+  }
+#pragma unroll
+  for (int b = 0; b < kDenseBatch; ++b) {
+    const int64_t k = k0 + 256 * b;
+    if (k < p.n)
+      out[k] = make_float4(f32_from_e4m3(w[b] & 0xFFu) * s[b], f32_from_e4m3((w[b] >> 8) & 0xFFu) * s[b],
+                           f32_from_e4m3((w[b] >> 16) & 0xFFu) * s[b], f32_from_e4m3(w[b] >> 24) * s[b]);
+  }
+}
+
+// Whether v is one contiguous run in index order.
+bool dense(const Rank4& v) {
+  int64_t want = 1;
+  for (int i = 3; i >= 0; --i) {
+    if (v.size[i] != 1 && v.stride[i] != want) return false;
+    want *= v.size[i];
+  }
+  return true;
+}
+
 // A SpanView of v (element size eb) when its rows fold into one uniformly
 // strided axis, its pieces are contiguous and 16-byte aligned and the launch
 // indexes fit in 31 bits.
@@ -789,6 +1047,69 @@ int32_t launch_quantize(const Rank4& x, int x_dt, const float* scales, int64_t s
   return CF_OK;
 }
 
+uint64_t scale_quantize_workspace_bytes(int64_t H) { return 2ull * kPartWgs * (uint64_t)H * 4; }
+
+// Scales and codes of one or two contiguous tensors; false: shapes, strides or
+// alignment that these kernels do not take (nothing is launched).
+bool scale_quantize_ok(const Rank4* x, const Rank4* out, int count, int x_dt) {
+  (void)x_dt;
+  for (int i = 0; i < count; ++i) {
+    if (!dense(x[i]) || !dense(out[i])) return false;
+    if ((((uintptr_t)x[i].base | (uintptr_t)out[i].base) & 15) != 0) return false;
+    for (int d = 0; d < 4; ++d)
+      if (x[i].size[d] != x[0].size[d]) return false;
+  }
+  const int64_t H = x[0].size[2], D = x[0].size[3];
+  const int64_t n = x[0].size[0] * x[0].size[1] * H * D;
+  return H >= 1 && H <= kDenseHeads && D >= 16 && D % 16 == 0 && n > 0 && n / 16 < ((int64_t)1 << 30);
+}
+
+int32_t launch_scale_quantize(const Rank4* x, const Rank4* out, float* const* scales, int count, int x_dt,
+                              void* workspace, hipStream_t stream) {
+  DenseQuant p{};
+  const int64_t D = x[0].size[3];
+  p.n = (int)(x[0].size[0] * x[0].size[1] * x[0].size[2] * D / 16);
+  p.H = (int)x[0].size[2];
+  p.np = (int)(D / 16);
+  p.P = p.H * p.np;
+  p.parts = (uint32_t*)workspace;
+  for (int i = 0; i < count; ++i) {
+    p.x[i] = (const char*)x[i].base;
+    p.out[i] = (char*)out[i].base;
+    p.scales[i] = scales[i];
+  }
+#define CF_SQ(KERNEL, ...)                                                \
+  switch (x_dt) {                                                         \
+    case kF32: CF_LAUNCH((KERNEL<kF32>), __VA_ARGS__); break;             \
+    case kF16: CF_LAUNCH((KERNEL<kF16>), __VA_ARGS__); break;             \
+    case kBF16: CF_LAUNCH((KERNEL<kBF16>), __VA_ARGS__); break;           \
+    default: set_error("scale_quantize: unsupported dtype %d", x_dt); return CF_ERR_UNSUPPORTED; \
+  }
+  if (p.n <= kOneWgThreads * kOneWgPieces) {
+    ProfileScope prof("cf_fp8_quantize", stream);
+    CF_SQ(quantize_small_kernel, dim3(count), dim3(kOneWgThreads), 0, stream, p)
+    CF_HIP_CHECK(hipGetLastError());
+    return CF_OK;
+  }
+  const int wgs = (int)std::min<int64_t>(kPartWgs, ceil_div(p.n, 256 * kDenseBatch));
+  {
+    ProfileScope prof("cf_fp8_amax", stream);
+    CF_SQ(amax_parts_kernel, dim3(wgs, count), dim3(256), 0, stream, p)
+  }
+  CF_HIP_CHECK(hipGetLastError());
+  {
+    // 16 workgroups per CU at most, as each reduces the maxima (2 x 33.5 MB of
+    // bf16: 19-23 us, 4.4-5.3 TB/s; 4 to 32 per CU lie within the spread that
+    // the buffers' placement gives)
+    const int blocks = (int)std::min<int64_t>(16 * (int64_t)device_cu_count() / count, ceil_div(p.n, 256 * kDenseBatch));
+    ProfileScope prof("cf_fp8_quantize", stream);
+    CF_SQ(quantize_parts_kernel, dim3(blocks, count), dim3(256), 0, stream, p, wgs)
+  }
+  CF_HIP_CHECK(hipGetLastError());
+#undef CF_SQ
+  return CF_OK;
+}
+
 static bool quantize_kv_tiles_ok(const Rank4& k, const Rank4& v, int x_dt, const Rank4& ko, const Rank4& vo) {
   const int eb = x_dt == kF32 ? 4 : 2;
   for (int i = 0; i < 4; ++i)
@@ -829,10 +1150,38 @@ int32_t launch_quantize_kv(const Rank4& k, const Rank4& v, int x_dt, const float
   return launch_quantize(v, x_dt, vs, vs_s, vo, stream);
 }
 
+bool dequantize_dense_ok(const Rank4& q, const Rank4& out) {
+  return q.size[3] % 4 == 0 && dense(q) && dense(out) && (((uintptr_t)q.base) & 3) == 0 &&
+         (((uintptr_t)out.base) & 15) == 0 &&
+         q.size[0] * q.size[1] * q.size[2] * q.size[3] < (int64_t)INT32_MAX * kDenseBatch * 256;
+}
+
+int32_t launch_dequantize_dense(const Rank4* q, const float* const* scales, const int64_t* s_stride, const Rank4* out,
+                                int count, hipStream_t stream) {
+  DenseDequant p{};
+  p.n = q[0].size[0] * q[0].size[1] * q[0].size[2] * q[0].size[3] / 4;
+  if (p.n == 0) return CF_OK;
+  bool one = true;  // one scale for the whole tensor
+  for (int i = 0; i < count; ++i) {
+    p.q[i] = (const uint32_t*)q[i].base;
+    p.out[i] = (float4*)out[i].base;
+    p.scales[i] = scales[i];
+    p.s_stride[i] = s_stride[i];
+    one = one && s_stride[i] == 0;
+  }
+  p.H = one ? 1 : (int)q[0].size[2];
+  p.dw = (int)(q[0].size[3] / 4);
+  ProfileScope prof("cf_fp8_dequantize", stream);
+  CF_LAUNCH(dequantize_dense_kernel, dim3((unsigned)ceil_div(p.n, 256 * kDenseBatch), count), dim3(256), 0, stream, p);
+  CF_HIP_CHECK(hipGetLastError());
+  return CF_OK;
+}
+
 int32_t launch_dequantize(const Rank4& q, const float* scales, int64_t s_stride, const Rank4& out,
                           hipStream_t stream) {
   const int64_t n = q.size[0] * q.size[1] * q.size[2] * q.size[3];
   if (n == 0) return CF_OK;
+  if (dequantize_dense_ok(q, out)) return launch_dequantize_dense(&q, &scales, &s_stride, &out, 1, stream);
   ProfileScope prof("cf_fp8_dequantize", stream);
   if (q.size[3] % 16 == 0) {
     CF_LAUNCH(dequantize_rows_kernel, dim3(grid_for(n / 16)), dim3(256), 0, stream, q, scales, s_stride, out,

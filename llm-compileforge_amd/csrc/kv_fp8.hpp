@@ -36,6 +36,15 @@ int32_t launch_quantize(const Rank4& x, int x_dt, const float* scales, int64_t s
 // native-tile (e.g. paired) K and V views of [S0, 16, H, D] pools.
 int32_t launch_quantize_kv(const Rank4& k, const Rank4& v, int x_dt, const float* ks, int64_t ks_s, const float* vs,
                            int64_t vs_s, const Rank4& ko, const Rank4& vo, hipStream_t stream);
+// Scales (amax / 448 per head) and codes of `count` (1 or 2) contiguous tensors
+// of one shape; workspace of scale_quantize_workspace_bytes(heads).
+uint64_t scale_quantize_workspace_bytes(int64_t H);
+bool scale_quantize_ok(const Rank4* x, const Rank4* out, int count, int x_dt);
+int32_t launch_scale_quantize(const Rank4* x, const Rank4* out, float* const* scales, int count, int x_dt,
+                              void* workspace, hipStream_t stream);
+bool dequantize_dense_ok(const Rank4& q, const Rank4& out);
+int32_t launch_dequantize_dense(const Rank4* q, const float* const* scales, const int64_t* s_stride, const Rank4* out,
+                                int count, hipStream_t stream);
 int32_t launch_dequantize(const Rank4& q, const float* scales, int64_t s_stride, const Rank4& out,
                           hipStream_t stream);
 int32_t launch_kv_write_fp8(const KvWriteParams& p, int x_dt, int slot_dt, hipStream_t stream);

@@ -66,6 +66,13 @@ class FP8KVCacheQuantizer:
             where = t.device if isinstance(t, torch.Tensor) else type(t).__name__
             raise ValueError(f"{name} must be a ROCm device tensor (got {where})")
 
+    def _check_block(self, kv_block: torch.Tensor) -> None:
+        self._check_device("kv_block", kv_block)
+        if not self._has_fp8_dtype():
+            raise RuntimeError("torch.float8_e4m3fn is required")
+        if kv_block.numel() == 0:
+            raise RuntimeError("max(): Expected reduction dim to be specified for input.numel() == 0.")
+
     def quantize_block(self, kv_block: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         """Quantizes a KV block with one scale for the whole tensor.
 
@@ -73,11 +80,11 @@ class FP8KVCacheQuantizer:
             (quant_block, scale): float8_e4m3fn codes of kv_block's shape and
             a 0-d float32 scale on the same device.
         """
-        self._check_device("kv_block", kv_block)
-        if not self._has_fp8_dtype():
-            raise RuntimeError("torch.float8_e4m3fn is required")
-        if kv_block.numel() == 0:
-            raise RuntimeError("max(): Expected reduction dim to be specified for input.numel() == 0.")
+        self._check_block(kv_block)
+        fused = _ops.fp8_scale_quantize(kv_block, per_head=False)
+        if fused is not None:
+            (quant, scale), = fused
+            return quant, scale.reshape(())
         rows = kv_block.reshape(-1, 1, kv_block.shape[-1]) if kv_block.dim() > 0 else kv_block.reshape(1, 1, 1)
         scale = _ops.fp8_amax_scale(rows)
         quant = _ops.fp8_quantize(kv_block, scale)
@@ -85,17 +92,27 @@ class FP8KVCacheQuantizer:
 
     def dequantize_block(self, quant_block: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
         """float32(quant_block) * scale."""
+        return _ops.fp8_dequantize(quant_block, self._scale_for(quant_block, scale))
+
+    def _scale_for(self, quant_block: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
+        """`scale` as a float32 tensor beside quant_block."""
         self._check_device("quant_block", quant_block)
         if quant_block.dtype != torch.float8_e4m3fn:
             raise ValueError(f"quant_block must be float8_e4m3fn, got {quant_block.dtype}")
         if not isinstance(scale, torch.Tensor):
-            scale = torch.tensor(float(scale), dtype=torch.float32, device=quant_block.device)
-        return _ops.fp8_dequantize(quant_block, scale.to(device=quant_block.device, dtype=torch.float32))
+            return torch.tensor(float(scale), dtype=torch.float32, device=quant_block.device)
+        return scale.to(device=quant_block.device, dtype=torch.float32)
 
     def quantize_kv(
         self, k: torch.Tensor, v: torch.Tensor
     ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
         """Quantizes K and V, each with its own scale."""
+        self._check_block(k)
+        self._check_block(v)
+        fused = _ops.fp8_scale_quantize(k, v, per_head=False)
+        if fused is not None:
+            (k_quant, k_scale), (v_quant, v_scale) = fused
+            return k_quant, k_scale.reshape(()), v_quant, v_scale.reshape(())
         k_quant, k_scale = self.quantize_block(k)
         v_quant, v_scale = self.quantize_block(v)
         return k_quant, k_scale, v_quant, v_scale
@@ -108,7 +125,10 @@ class FP8KVCacheQuantizer:
         v_scale: torch.Tensor,
     ) -> tuple[torch.Tensor, torch.Tensor]:
         """Dequantizes K and V to float32."""
-        return self.dequantize_block(k_quant, k_scale), self.dequantize_block(v_quant, v_scale)
+        k_scale, v_scale = self._scale_for(k_quant, k_scale), self._scale_for(v_quant, v_scale)
+        if k_quant.device != v_quant.device:
+            return _ops.fp8_dequantize(k_quant, k_scale), _ops.fp8_dequantize(v_quant, v_scale)
+        return _ops.fp8_dequantize_kv(k_quant, v_quant, k_scale, v_scale)
 
     # ---- additions ------------------------------------------------------
 
@@ -121,6 +141,9 @@ class FP8KVCacheQuantizer:
         self._check_device("x", x)
         if x.dim() < 2:
             raise ValueError("x must have a head axis: [..., num_kv_heads, head_dim]")
+        fused = _ops.fp8_scale_quantize(x, per_head=True)
+        if fused is not None:
+            return fused[0]
         scales = _ops.fp8_amax_scale(x)
         return _ops.fp8_quantize(x, scales), scales
 

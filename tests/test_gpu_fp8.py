@@ -296,3 +296,55 @@ def test_kv_write_runs_bit_exact(gpu, slot_dtype, h, d, x_dtype):
         assert np.array_equal(kcodes[s // bs, s % bs], wk[i]), (i, s)
         assert np.array_equal(vcodes[s // bs, s % bs], wv[i]), (i, s)
     assert np.all(kcodes[~written] == 0xAA) and np.all(vcodes[~written] == 0xAA)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shape", [
+    (1, 1, 16),            # one piece
+    (16, 8, 128),          # one KV block: one workgroup
+    (32768 // 48, 3, 16),  # the most a workgroup holds, less a row
+    (2049, 1, 16),         # one piece more: two passes
+    (700, 12, 64),         # heads that do not divide a workgroup's pieces
+    (4099, 64, 32),        # the most heads, a ragged last batch
+    (130, 65, 16),         # more heads: the separate kernels
+    (40, 3, 24),           # rows that are not pieces: the separate kernels
+])
+def test_scale_and_quantize_in_one_call_bit_exact(gpu, shape, dtype):
+    """quantize_block / quantize_kv / quantize_per_head and back, at the sizes
+    where the kernels change, against the oracle."""
+    torch.manual_seed(shape[0])
+    k = (torch.randn(shape) * 3).to(dtype)
+    v = torch.randn(shape).to(dtype)
+    v[..., 0, :] = 0.0  # an all-zero head (scale 1.0)
+    quant = FP8KVCacheQuantizer()
+    kq, ks, vq, vs = quant.quantize_kv(k.to(gpu), v.to(gpu))
+    for x, q, s in ((k, kq, ks), (v, vq, vs)):
+        wc, ws = ofp8.quantize_block(x.float().numpy())
+        assert s.dim() == 0 and s.item() == ws and np.array_equal(codes(q), wc)
+    kf, vf = quant.dequantize_kv(kq, ks, vq, vs)
+    assert np.array_equal(kf.cpu().numpy(), ofp8.decode(codes(kq)) * ks.cpu().numpy())
+    assert np.array_equal(vf.cpu().numpy(), ofp8.decode(codes(vq)) * vs.cpu().numpy())
+    hq, hs = quant.quantize_per_head(v.to(gpu))
+    wc, ws = ofp8.quantize_per_head(v.float().numpy()[None])
+    assert np.array_equal(hs.cpu().numpy(), ws) and np.array_equal(codes(hq), wc[0])
+    deq = ops.fp8_dequantize(hq, hs)
+    assert np.array_equal(deq.cpu().numpy(), ofp8.decode(codes(hq)) * hs.cpu().numpy()[:, None])
+
+
+def test_one_call_quantize_keeps_nan_and_infinity_rules(gpu):
+    """NaN and infinite values: the scale and codes of the separate calls
+    (torch's max propagates NaN); an unaligned or strided block takes them."""
+    quant = FP8KVCacheQuantizer()
+    for bad in (float("nan"), float("inf")):
+        for n in (1024, 1 << 16):
+            x = torch.randn(n // 64, 4, 16, device=gpu)
+            x[3, 1, 5] = bad
+            want_s = ops.fp8_amax_scale(x)
+            q, s = quant.quantize_per_head(x)
+            assert torch.equal(s.view(torch.int32), want_s.view(torch.int32))
+            assert np.array_equal(codes(q), codes(ops.fp8_quantize(x, want_s)))
+    base = torch.randn(4097, device=gpu)
+    for x in (base[1:], torch.randn(64, 4, 32, device=gpu).transpose(0, 1)):
+        q, s = quant.quantize_block(x)
+        wc, ws = ofp8.quantize_block(x.cpu().numpy())
+        assert s.item() == ws and np.array_equal(codes(q), wc)
