@@ -251,6 +251,8 @@ int32_t cf_last_error(char* buf, uint64_t len) {
   return (int32_t)e.size();
 }
 
+constexpr int32_t kDefaultPartitionTokens = 512;  // the binding's default
+
 static int64_t decode_max_parts(int64_t max_blocks, int32_t bs, int32_t pt) {
   return std::max<int64_t>(1, ceil_div(max_blocks * (int64_t)bs, pt));
 }
@@ -409,7 +411,15 @@ int32_t cf_paged_decode_shared(const CfTensor* q, const CfTensor* k_cache, const
   }
   if (B == 0) return CF_OK;
 
-  const bool mfma = decode_mfma_supported(p, vq.dtype, vk.dtype);
+  bool mfma = decode_mfma_supported(p, vq.dtype, vk.dtype);
+  // fp32 caches also run on the generic kernel.  It takes the calls that ask
+  // for a partition length of their own (the MFMA kernel has no partitions),
+  // and those whose workspace, or the fixed scratch, holds its partials
+  // (none for short tables) but not the MFMA kernel's rows.
+  if (mfma && vk.dtype == CF_F32 &&
+      (partition_tokens != kDefaultPartitionTokens ||
+       workspace_bytes < decode_mfma_workspace_bytes(B, Hq, Hkv, D)))
+    mfma = false;
   const uint64_t need = mfma ? decode_mfma_workspace_bytes(B, Hq, Hkv, D)
                              : generic_workspace_bytes(B, Hq, D, p.max_parts);
   if (need > 0) {

@@ -1,4 +1,4 @@
-// MFMA paged-decode kernel for bf16 and OCP e4m3fn KV caches (gfx950).
+// MFMA paged-decode kernel for bf16, fp16, fp32 and OCP e4m3fn KV caches (gfx950).
 //
 // Same semantics as the generic kernel (reference kernels/paged_attention.py
 // :21-73): softmax(q.k * scale) . v over a sequence's first
@@ -420,7 +420,19 @@ __device__ __forceinline__ void store_out4(void* out, int64_t off, float a, floa
 // Writes out a finished run (normalized output, record or wave-slot
 // partial) and, from the wave holding the run's first tile, the merge
 // descriptors of the sequences it covers.
-template <int QT, bool PL, int D>
+// The four consecutive channels of store t that a lane holds of its column:
+// channels 16 t + 4 lq .. + 3 of O tile t, or (QUAD: fp32 token-major V) the
+// t-th four of its 16 channels 64 u + 16 lq, spread over O tiles 4 u .. 4 u + 3.
+template <bool QUAD>
+__device__ __forceinline__ int o_chan(int t, int lq) {
+  return QUAD ? 64 * (t >> 2) + 16 * lq + 4 * (t & 3) : 16 * t + 4 * lq;
+}
+template <bool QUAD>
+__device__ __forceinline__ float o_elem(const f32x4_t* o, int t, int e) {
+  return QUAD ? o[4 * (t >> 2) + e][t & 3] : o[t][e];
+}
+
+template <int QT, bool PL, int D, bool QUAD = false>
 __device__ __forceinline__ void flush_run(const DecodeParams& p, const Index& ix, const Plan* pl, const Coord& c,
                                           const f32x4_t* o, float m, float l, int run_j0, bool first_run,
                                           int64_t chunk, int w, int lane) {
@@ -462,12 +474,23 @@ __device__ __forceinline__ void flush_run(const DecodeParams& p, const Index& ix
     }
   }
   if (li >= c.ncols) return;
-  if (direct) {
-    const float inv = lt > 0.0f ? vs / lt : 0.0f;
-    const int64_t orow = (int64_t)c.b * p.o_sb + (int64_t)(c.h * G + li) * p.o_sh + 4 * lq;
+  if (direct && QT == kF32) {
+    // one rounding per output: divide, rather than multiply by 1 / l
+    const int64_t orow = (int64_t)c.b * p.o_sb + (int64_t)(c.h * G + li) * p.o_sh;
+    auto nrm = [&](float a) { return lt > 0.0f ? a * vs / lt : 0.0f; };
 #pragma unroll
     for (int t = 0; t < NV; ++t)
-      store_out4<QT>(p.out, orow + 16 * t, o[t][0] * inv, o[t][1] * inv, o[t][2] * inv, o[t][3] * inv);
+      store_out4<QT>(p.out, orow + o_chan<QUAD>(t, lq), nrm(o_elem<QUAD>(o, t, 0)), nrm(o_elem<QUAD>(o, t, 1)),
+                     nrm(o_elem<QUAD>(o, t, 2)), nrm(o_elem<QUAD>(o, t, 3)));
+    return;
+  }
+  if (direct) {
+    const float inv = lt > 0.0f ? vs / lt : 0.0f;
+    const int64_t orow = (int64_t)c.b * p.o_sb + (int64_t)(c.h * G + li) * p.o_sh;
+#pragma unroll
+    for (int t = 0; t < NV; ++t)
+      store_out4<QT>(p.out, orow + o_chan<QUAD>(t, lq), o_elem<QUAD>(o, t, 0) * inv, o_elem<QUAD>(o, t, 1) * inv,
+                     o_elem<QUAD>(o, t, 2) * inv, o_elem<QUAD>(o, t, 3) * inv);
     return;
   }
   int64_t row;
@@ -479,12 +502,13 @@ __device__ __forceinline__ void flush_run(const DecodeParams& p, const Index& ix
     const int mm = li / G;
     row = p.rec_pre + ((int64_t)(c.b + mm) * p.Hkv + c.h) * G + (li - mm * G);
   }
-  float* os = p.ws_o + row * D + 4 * lq;
+  float* os = p.ws_o + row * D;
 #pragma unroll
   for (int t = 0; t < NV; ++t)
-    *(float4*)(os + 16 * t) = make_float4(o[t][0] * vs, o[t][1] * vs, o[t][2] * vs, o[t][3] * vs);
+    *(float4*)(os + o_chan<QUAD>(t, lq)) = make_float4(o_elem<QUAD>(o, t, 0) * vs, o_elem<QUAD>(o, t, 1) * vs,
+                                                       o_elem<QUAD>(o, t, 2) * vs, o_elem<QUAD>(o, t, 3) * vs);
   if (lq == 0) {
-    p.ws_ml[row * 2] = m == -INFINITY ? -INFINITY : m * (1.0f / kLog2e);
+    p.ws_ml[row * 2] = m;  // log2 units
     p.ws_ml[row * 2 + 1] = lt;
   }
 }
@@ -507,6 +531,172 @@ __device__ __forceinline__ int stream_wave(int w, int Wtot, int Hkv) {
   const int x = g % kXcds, lw = (g / kXcds) * 4 + i;  // XCD, wave index within it
   const int k = x * (Wtot / kXcds / Hkv) + lw / Hkv;     // range among the Wtot / Hkv per head
   return (lw % Hkv) * (Wtot / Hkv) + k;
+}
+
+// A wave's tiles of an fp32 cache under fp32 queries: as the loop of
+// decode_stream_kernel, on v_mfma_f32_16x16x4_f32.  A tile is 2 x 16 KiB at
+// head_dim 128 (128 VGPRs), so it is not double-buffered: the next tile's K
+// loads go out into the K registers once the scores have read them, its V
+// loads once P.V has, and one half or the other is always in flight.  The
+// 128 MFMAs of a tile take 1.7 us against the 5.6 us that its bytes take at
+// 6 TB/s over 1024 waves: bound by HBM.  16 sequences of 256-2,048 tokens
+// (147 MB, 32 query / 8 KV heads of 128): 102 us on the generic kernel (VALU,
+// 4 bytes a load), 39 us here.
+template <int D, bool PL, bool VTOK>
+__device__ __forceinline__ void stream_f32(const DecodeParams& p, const Index& ix, const Seqs<PL>& seqs,
+                                           const Plan* pl, const KvCacheView& kv, Coord c0, Coord c1, bool has1,
+                                           int64_t v_end, int64_t chunk, int w, int lane) {
+  constexpr int NC = D / 16, NV = D / 16;
+  const int li = lane & 15, lq = lane >> 4;
+  TileF32<D> r;
+  load_k_f32<D, VTOK>(r, kv, c0.blkA, c0.blkB, li, lq, c0.h);
+  load_v_f32<D, VTOK>(r, kv, c0.blkA, c0.blkB, li, lq, c0.h);
+  float4 q[NC];
+  // column i < ncols: query head i % G of sequence b + i / G; the rest zero
+  auto load_cols = [&](const Coord& c) {
+    const bool used = li < c.ncols;
+    const int m = used ? li / p.G : 0, g = used ? li - m * p.G : 0;
+    const float* qrow =
+        (const float*)p.q + (int64_t)(c.b + m) * p.q_sb + (int64_t)(c.h * p.G + g) * p.q_sh + 4 * lq;
+#pragma unroll
+    for (int cc = 0; cc < NC; ++cc) {
+      const float4 x = *(const float4*)(qrow + 16 * cc);
+      q[cc] = used ? x : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+  };
+  load_cols(c0);
+  float m = -INFINITY, l = 0.0f;
+  f32x4_t o[NV];
+#pragma unroll
+  for (int t = 0; t < NV; ++t) o[t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  int run_j0 = c0.j;
+  bool first_run = true;
+  // Scores in log2 units, scale * log2(e) = qk_scale + qk_lo to twice the
+  // precision: p = 2^(s * scale * log2(e) - m) is formed in one rounding of
+  // the exponent.
+  const float qk_scale = p.scale * kLog2e;
+  const float qk_lo = __builtin_fmaf(p.scale, kLog2e, -qk_scale) + p.scale * kLog2eLo;
+  for (;;) {
+    const bool run_ends = !has1 || c1.b != c0.b || c1.h != c0.h || c1.kind != c0.kind;
+    // four partial sums per score: a short chain rounds less (and the MFMAs
+    // of a chain wait on each other)
+    f32x4_t se[2][4];
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) se[x][e] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+          se[x][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(elem4(r.k[x][c], e), elem4(q[c], e), se[x][e], 0, 0, 0);
+    f32x4_t s[2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x) s[x] = (se[x][0] + se[x][1]) + (se[x][2] + se[x][3]);
+    // (the last iteration reloads its own tile, so every path has the same
+    // number of loads in flight)
+    load_k_f32<D, VTOK>(r, kv, c1.blkA, c1.blkB, li, lq, c1.h);
+    const bool has2 = has1 && next_slot<PL>(c1) < v_end;
+    Coord c2 = c1;
+    if (has2) c2 = advance(p, ix, seqs, c1);
+
+    // lane (li, lq): s[x][v] -> token 16 x + 4 lq + v, column li
+    float sc[8];
+#pragma unroll
+    for (int v = 0; v < 8; ++v) sc[v] = s[v >> 2][v & 3] * qk_scale;
+    if (c0.len - 32 * c0.j < 32 || c0.blkA < 0 || c0.blkB < 0) {
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        const int nvalid = (x == 0 ? c0.blkA : c0.blkB) < 0 ? 0 : c0.len - 32 * c0.j - 16 * x - 4 * lq;
+        // cache slots past the end may hold any bits: p = 0 there, and V too
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          if (v >= nvalid) sc[4 * x + v] = -INFINITY;
+#pragma unroll
+        for (int t = 0; t < NV; ++t) {
+          float4& f = r.v[x][t];
+          if constexpr (VTOK) {
+            if ((t & 3) >= nvalid) f = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+          } else {
+            if (0 >= nvalid) f.x = 0.0f;
+            if (1 >= nvalid) f.y = 0.0f;
+            if (2 >= nvalid) f.z = 0.0f;
+            if (3 >= nvalid) f.w = 0.0f;
+          }
+        }
+      }
+    }
+    float mt = sc[0];
+#pragma unroll
+    for (int v = 1; v < 8; ++v) mt = fmaxf(mt, sc[v]);
+    // lazy rescaling, as in decode_stream_kernel
+    if (__any(mt > m + 8.0f)) {
+      mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
+      mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+      const float mnew = mt > m + 8.0f ? mt : m;
+      const float alpha = mnew == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mnew);
+      l *= alpha;
+#pragma unroll
+      for (int t = 0; t < NV; ++t) o[t] = o[t] * alpha;
+      m = mnew;
+    }
+    const bool live = m != -INFINITY;
+    float pr[8];
+    float psum = 0.0f;
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+      const float raw = s[v >> 2][v & 3];
+      const float ex = __builtin_fmaf(raw, qk_scale, __builtin_fmaf(raw, qk_lo, -m));
+      pr[v] = live && sc[v] != -INFINITY ? __builtin_amdgcn_exp2f(ex) : 0.0f;
+    }
+    psum = ((pr[0] + pr[1]) + (pr[2] + pr[3])) + ((pr[4] + pr[5]) + (pr[6] + pr[7]));
+    l += psum;
+    // Step s of block x: tokens 4 lq + s, this lane's own p.  Each block's sum
+    // is formed apart and the tile's added to O once, so a sum over n tokens
+    // is a chain of n / 32 additions instead of n / 4 (the error against 64
+    // bits over contexts of 16 to 10,000 tokens: 1.5e-7 to 2.2e-7, where one
+    // running sum gave up to 4.7e-7 and the generic kernel up to 3.2e-7).
+    constexpr int kOT = 2;  // O tiles at a time
+#pragma unroll
+    for (int t0 = 0; t0 < NV; t0 += kOT) {
+      f32x4_t ot[2][kOT];
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int t = 0; t < kOT; ++t) ot[x][t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int st = 0; st < 4; ++st)
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+          for (int t = 0; t < kOT; ++t) {
+            const int ti = t0 + t;
+            const float a = VTOK ? elem4(r.v[x][(ti & ~3) + st], ti & 3) : elem4(r.v[x][ti], st);
+            ot[x][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, pr[4 * x + st], ot[x][t], 0, 0, 0);
+          }
+#pragma unroll
+      for (int t = 0; t < kOT; ++t) o[t0 + t] = o[t0 + t] + (ot[0][t] + ot[1][t]);
+    }
+    load_v_f32<D, VTOK>(r, kv, c1.blkA, c1.blkB, li, lq, c1.h);
+    if (run_ends) {
+      flush_run<kF32, PL, D, VTOK>(p, ix, pl, c0, o, m, l, run_j0, first_run, chunk, w, lane);
+      first_run = false;
+    }
+    if (!has1) break;
+    c0 = c1;
+    c1 = c2;
+    has1 = has2;
+    if (run_ends) {
+      load_cols(c0);
+      m = -INFINITY;
+      l = 0.0f;
+#pragma unroll
+      for (int t = 0; t < NV; ++t) o[t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      run_j0 = c0.j;
+    }
+  }
 }
 
 template <int QT, int KT, int D, bool PL, bool VTOK>
@@ -591,6 +781,9 @@ __global__ __launch_bounds__(256) void decode_stream_kernel(DecodeParams p, cons
 
   const KvCacheView kv{(const uint8_t*)p.k, (const uint8_t*)p.v, p.k_s[0], p.k_s[2], p.v_s[0], p.v_s[2],
                        p.k_s[1], p.v_s[1]};
+  if constexpr (KT == kF32) {
+    stream_f32<D, PL, VTOK>(p, ix, seqs, pl, kv, c0, c1, has1, v_end, chunk, w, lane);
+  } else {
   // token-major V: this wave's LDS staging rows, after the plan
   uint8_t* vstage = (uint8_t*)dyn_lds + (PL ? kPlanLdsBytes : 0) + wave * vtok_stage_bytes<D, KvTraits<KT>::kBytes>();
   (void)vstage;
@@ -800,6 +993,7 @@ __global__ __launch_bounds__(256) void decode_stream_kernel(DecodeParams p, cons
       run_j0 = c0.j;
     }
   }
+  }
 }
 
 // Row of the k-th partial a merge descriptor names: {row, -1} is one
@@ -865,7 +1059,7 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeParams p) {
 #pragma unroll
       for (int k = 0; k < KMAX; ++k) {
         if (k < nsrc) {
-          const float w = mk[k][g] == -INFINITY ? 0.0f : __expf(mk[k][g] - Mg[g]);
+          const float w = mk[k][g] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mk[k][g] - Mg[g]);
           mk[k][g] = w;  // now the weight
           Lg[g] += w * lk[k][g];
         }
@@ -951,13 +1145,13 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeParams p) {
       float ls = 0.0f;
       for (int k = lane; k < n; k += 64) {
         const float mk = sm[g][k];
-        const float w = mk == -INFINITY ? 0.0f : __expf(mk - mnew);
+        const float w = mk == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mk - mnew);
         sm[g][k] = w;
         ls += w * sl[g][k];
       }
       ls = wave_sum(ls);
       if (lane == 0) {
-        const float sc = mold == -INFINITY ? 0.0f : __expf(mold - mnew);
+        const float sc = mold == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mold - mnew);
         run_sc[g] = sc;
         run_l[g] = run_l[g] * sc + ls;
         run_m[g] = mnew;
@@ -1048,7 +1242,7 @@ constexpr int kMergeSplitBelow = 256;
 
 template <int KT, int D, bool PL, bool VTOK>
 constexpr size_t stream_lds_bytes() {
-  return (PL ? kPlanLdsBytes : 0) + (VTOK ? 4 * (size_t)vtok_stage_bytes<D, KvTraits<KT>::kBytes>() : 0);
+  return (PL ? kPlanLdsBytes : 0) + (VTOK && KT != kF32 ? 4 * (size_t)vtok_stage_bytes<D, KvTraits<KT>::kBytes>() : 0);
 }
 
 template <int QT, int KT, int D, bool PL, bool VTOK>
@@ -1147,9 +1341,9 @@ void decode_mfma_bind_workspace(DecodeParams& p, void* workspace) {
 
 bool decode_mfma_supported(const DecodeParams& p, int q_dt, int kv_dt) {
   // bf16 or fp32 queries over bf16 or e4m3 caches; fp16 queries over fp16
-  // or e4m3
+  // or e4m3; fp32 queries over fp32
   if (q_dt == kBF16 || q_dt == kF32) {
-    if (kv_dt != kBF16 && kv_dt != kE4M3) return false;
+    if (kv_dt != kBF16 && kv_dt != kE4M3 && (kv_dt != kF32 || q_dt != kF32)) return false;
   } else if (q_dt == kF16) {
     if (kv_dt != kF16 && kv_dt != kE4M3) return false;
   } else {
@@ -1160,7 +1354,7 @@ bool decode_mfma_supported(const DecodeParams& p, int q_dt, int kv_dt) {
   if (p.NB < 1) return false;  // invalid block ids are redirected to block 0 (then masked)
   // partial-row indices and descriptors are int32
   if ((uint64_t)total_rows(p.B, p.Hq) >= (uint64_t)INT32_MAX / 2) return false;
-  const int kb = kv_dt == kE4M3 ? 1 : 2;
+  const int kb = kv_dt == kE4M3 ? 1 : (kv_dt == kF32 ? 4 : 2);
   // K: token rows with unit channel stride, 16-byte aligned (token stride D
   // in the native / paired layouts, any multiple of 16 bytes token-major).
   // V: the native tile [D][bs] (token stride 1, channel stride bs), or
@@ -1194,6 +1388,7 @@ int32_t launch_d(const DecodeParams& p, hipStream_t stream) {
 
 int32_t launch_decode_mfma(const DecodeParams& p, int q_dt, int kv_dt, hipStream_t stream) {
   if (q_dt == kF16) return kv_dt == kE4M3 ? launch_d<kF16, kE4M3>(p, stream) : launch_d<kF16, kF16>(p, stream);
+  if (q_dt == kF32 && kv_dt == kF32) return launch_d<kF32, kF32>(p, stream);
   if (q_dt == kF32) return kv_dt == kE4M3 ? launch_d<kF32, kE4M3>(p, stream) : launch_d<kF32, kBF16>(p, stream);
   return kv_dt == kE4M3 ? launch_d<kBF16, kE4M3>(p, stream) : launch_d<kBF16, kBF16>(p, stream);
 }

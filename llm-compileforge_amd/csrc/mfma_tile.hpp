@@ -25,6 +25,7 @@ typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr float kLog2e = 1.4426950408889634f;
+constexpr float kLog2eLo = 1.9259629911e-8f;  // log2(e) - kLog2e
 
 // KV data is read once per call: non-temporal (streaming) loads.
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
@@ -64,6 +65,10 @@ struct KvTraits<kBF16> {
 template <>
 struct KvTraits<kF16> {
   static constexpr int kBytes = 2;
+};
+template <>
+struct KvTraits<kF32> {
+  static constexpr int kBytes = 4;
 };
 
 // Raw per-lane registers of one 32-token tile.  VTOK: V stored token-major
@@ -131,6 +136,67 @@ __device__ __forceinline__ void load_tile(TileRegs<KT, D, VTOK>& r, const KvCach
 #pragma unroll
     for (int t = 0; t < R::NV; ++t) r.v[t] = stream_load<typename R::VT>(vp + t * 256 * KB);
   }
+}
+
+// fp32 tiles (v_mfma_f32_16x16x4_f32, products and sums in fp32).  A operand:
+// row l % 16, k = l / 16; B: column l % 16, k = l / 16; the output holds rows
+// 4 (l / 16) + v of column l % 16.  Per 16-token block X (0, 1) of the tile:
+//   S^T = K Q^T, D/4 steps: step 4 c + e multiplies channels 16 c + 4 k + e,
+//   so lane (li, lq) feeds K row li, channels 16 c + 4 lq .. + 3 (one 16-byte
+//   load per c, 64-byte runs per row) and its output is the scores of tokens
+//   4 lq + v;
+//   O^T += V^T P^T: step s multiplies tokens 4 k + s, so the lane feeds its
+//   own scores' p_s, and V of token 4 lq + s.  Channel-major V: channel
+//   16 t + li, tokens 4 lq .. + 3 in one 16-byte load, O tile t = channels
+//   16 t + row.  Token-major V: channels 64 u + 4 li .. + 3 of token 4 lq + s
+//   in one load, element e of it feeding O tile 4 u + e = channels
+//   64 u + 4 row + e: no transpose is needed, only another order of O.
+template <int D>
+struct TileF32 {
+  static constexpr int NC = D / 16;  // 16-byte K loads per row of a lane
+  static constexpr int NV = D / 16;  // 16-byte V loads per block of a lane
+  float4 k[2][NC];
+  float4 v[2][NV];
+};
+
+__device__ __forceinline__ float4 stream_load_f4(const void* p) {
+  return __builtin_bit_cast(float4, stream_load<uint4>(p));
+}
+
+template <int D, bool VTOK>
+__device__ __forceinline__ void load_k_f32(TileF32<D>& r, const KvCacheView& kv, int blkA, int blkB, int li, int lq,
+                                           int h) {
+#pragma unroll
+  for (int x = 0; x < 2; ++x) {
+    const int64_t b = x == 0 ? (blkA < 0 ? 0 : blkA) : (blkB < 0 ? 0 : blkB);
+    const float* row = (const float*)kv.k + b * kv.k_blk + (int64_t)h * kv.k_head + li * (VTOK ? kv.k_tok : D) + 4 * lq;
+#pragma unroll
+    for (int c = 0; c < TileF32<D>::NC; ++c) r.k[x][c] = stream_load_f4(row + 16 * c);
+  }
+}
+
+template <int D, bool VTOK>
+__device__ __forceinline__ void load_v_f32(TileF32<D>& r, const KvCacheView& kv, int blkA, int blkB, int li, int lq,
+                                           int h) {
+#pragma unroll
+  for (int x = 0; x < 2; ++x) {
+    const int64_t b = x == 0 ? (blkA < 0 ? 0 : blkA) : (blkB < 0 ? 0 : blkB);
+    const float* base = (const float*)kv.v + b * kv.v_blk + (int64_t)h * kv.v_head;
+    if constexpr (VTOK) {
+      // load 4 u + s: token 4 lq + s, channels 64 u + 4 li .. + 3
+#pragma unroll
+      for (int t = 0; t < TileF32<D>::NV; ++t)
+        r.v[x][t] = stream_load_f4(base + (4 * lq + (t & 3)) * kv.v_tok + 64 * (t >> 2) + 4 * li);
+    } else {
+      // load t: channel 16 t + li, tokens 4 lq .. + 3
+#pragma unroll
+      for (int t = 0; t < TileF32<D>::NV; ++t) r.v[x][t] = stream_load_f4(base + (16 * t + li) * 16 + 4 * lq);
+    }
+  }
+}
+
+__device__ __forceinline__ float elem4(const float4& f, int e) {
+  return e == 0 ? f.x : (e == 1 ? f.y : (e == 2 ? f.z : f.w));
 }
 
 // Token-major V: the wave's LDS staging area holds the tile's 32 token rows

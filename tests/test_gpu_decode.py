@@ -17,7 +17,7 @@ import pytest
 import torch
 
 from cf_hip import layout as L
-from cf_hip import ops, workloads
+from cf_hip import _abi, ops, workloads
 from kernels.paged_attention import paged_attention, paged_attention_tensors
 from tests.gpu_util import assert_close, oracle_decode
 
@@ -181,6 +181,71 @@ def test_fp32_queries_c3_batch(gpu):
                                   k_scale=ks, v_scale=vs, shared_prefix_lens=sh)
     torch.cuda.synchronize()
     assert_close(out.cpu().numpy(), oracle_decode(case, kc, vc, ks, vs), torch.float32, "c3 fp32 q")
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(32, 8, 128), (16, 2, 64), (12, 12, 64), (16, 1, 128)])
+@pytest.mark.parametrize("layout", ["paired", "native", "token_major"])
+def test_fp32_caches_take_the_mfma_path(gpu, hq, hkv, d, layout):
+    """fp32 queries over fp32 caches (v_mfma_f32_16x16x4_f32): ends inside a
+    block, at a block and at a tile, NaN past them, an invalid table entry, a
+    shared prefix and a sequence split over many waves."""
+    print(f"[case] fp32 cache hq={hq} hkv={hkv} d={d} layout={layout}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(11 * hq + d)
+    lens = [1, 15, 16, 17, 32, 33, 0, 1024 + 70, 1024 + 5, 5000]
+    nb = 600
+    perm = torch.randperm(nb, generator=torch.Generator().manual_seed(4)).tolist()
+    shared, pos, tables = perm[:64], 64, []
+    for i, n in enumerate(lens):
+        k = max(1, (n + 15) // 16) - (64 if i in (7, 8) else 0)
+        tables.append((shared if i in (7, 8) else []) + perm[pos:pos + k])
+        pos += k
+    q = torch.randn(len(lens), hq, d, generator=g, device=gpu) * 2.0
+    k, v = (torch.randn(nb, 16, hkv, d, generator=g, device=gpu) for _ in range(2))
+    case = workloads.DecodeCase("fp32kv", q, k, v, tables, lens, 16, 1 / math.sqrt(d), torch.float32)
+    kc, vc, _, _ = workloads.materialize(case, layout)
+    ref = oracle_decode(case, kc, vc, None, None)
+    for t, n in zip(tables, lens):  # what lies past the end is never used
+        if n % 16:
+            kc[t[n // 16], n % 16:] = float("nan")
+            vc[t[n // 16], n % 16:] = float("nan")
+    sh = torch.tensor(ops.shared_prefix_lens(tables, lens, 16), dtype=torch.int32, device=gpu)
+    with ops.KernelTimer() as timer:
+        out = paged_attention_tensors(q, kc, vc, case.tables_tensor(gpu), case.seq_lens_tensor(gpu), 16, case.scale,
+                                      shared_prefix_lens=sh)
+        torch.cuda.synchronize()
+        assert timer.query("cf_decode_mfma")[1] == 1 and timer.query("cf_decode_generic")[1] == 0
+    assert_close(out.cpu().numpy(), ref, torch.float32, f"fp32 cache / {layout}")
+    bad = case.tables_tensor(gpu)
+    bad[9, 100] = nb  # its 16 tokens drop out
+    out = paged_attention_tensors(q, kc, vc, bad, case.seq_lens_tensor(gpu), 16, case.scale)
+    cut = [t[:100] + t[101:] for t in tables[9:]]
+    one = workloads.DecodeCase("cut", q[9:], k, v, cut, [lens[9] - 16], 16, case.scale, torch.float32)
+    assert_close(out[9:].cpu().numpy(), oracle_decode(one, kc, vc, None, None), torch.float32, "invalid entry")
+
+
+def test_fp32_cache_routes(gpu):
+    """A batch beyond the kernel's per-sequence plan; a workspace that holds
+    only the partitioned kernel's partials still runs, on that kernel."""
+    g = torch.Generator(device=gpu).manual_seed(3)
+    b, hq, hkv, d = 2100, 2, 1, 64
+    lens = [1 + (7 * i) % 50 for i in range(b)]
+    tables = [[(4 * i + j) % 512 for j in range((n + 15) // 16)] for i, n in enumerate(lens)]
+    q = torch.randn(b, hq, d, generator=g, device=gpu)
+    k, v = (torch.randn(512, 16, hkv, d, generator=g, device=gpu) for _ in range(2))
+    case = workloads.DecodeCase("many", q, k, v, tables, lens, 16, 1 / math.sqrt(d), torch.float32)
+    kc, vc, _, _ = workloads.materialize(case, "native")
+    ref = oracle_decode(case, kc, vc, None, None)
+    tab, ln = case.tables_tensor(gpu), case.seq_lens_tensor(gpu)
+    assert_close(paged_attention_tensors(q, kc, vc, tab, ln, 16).cpu().numpy(), ref, torch.float32, "2100 sequences")
+    out = torch.empty_like(q)
+    d_ = [_abi.descriptor(t) for t in (q, kc, vc, tab, ln, out)]
+    with ops.KernelTimer() as timer:
+        rc = _abi.lib().cf_paged_decode(*(_abi.ref(x) for x in d_[:5]), None, None, 1 / math.sqrt(d), 16, 512,
+                                        _abi.ref(d_[5]), None, 0, _abi.stream_handle(q.device))
+        torch.cuda.synchronize()
+        assert rc == 0, _abi.last_error()
+        assert timer.query("cf_decode_generic")[1] == 1 and timer.query("cf_decode_mfma")[1] == 0
+    assert_close(out.cpu().numpy(), ref, torch.float32, "no workspace")
 
 
 def test_edge_lengths(gpu):
