@@ -264,6 +264,11 @@ def ref(d: CfTensor | None) -> Any:
 _RAW_STREAM = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
+def raw_stream(index: int) -> int:
+    """The current stream of device `index` as a hipStream_t value."""
+    return _RAW_STREAM(index) if _RAW_STREAM is not None else torch.cuda.current_stream(index).cuda_stream
+
+
 def stream_handle(device: torch.device) -> int:
     """The current stream of `device` as a hipStream_t value."""
     if _RAW_STREAM is not None:

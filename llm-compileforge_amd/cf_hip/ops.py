@@ -75,6 +75,40 @@ def _cached_workspace(nbytes: int, device: torch.device) -> torch.Tensor:
     return ws
 
 
+# The native call path (_fastcall.cpp): each wrapper below tries it first and
+# goes on by itself where it returns None (arguments that are not plain
+# tensors on the current device), which raises or handles the case.
+_FAST = None
+
+
+def _fast():
+    global _FAST
+    if _FAST is None:
+        handle = lib()
+        try:
+            from . import _fastcall
+        except ImportError as e:
+            raise RuntimeError(f"cf_hip._fastcall is not built ({e}): build it with "
+                               "`python llm-compileforge_amd/csrc/build.py`") from e
+        _fastcall.bind(
+            {name: ctypes.cast(getattr(handle, name), ctypes.c_void_p).value for name in _abi.SIGNATURES},
+            _abi._RAW_STREAM or _abi.raw_stream, getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device), _WORKSPACES,
+            _cached_workspace)
+        _FAST = _fastcall
+    return _FAST
+
+
+def _on_gpu(t) -> bool:
+    return isinstance(t, torch.Tensor) and t.is_cuda
+
+
+def _result(r, what: str):
+    """A native call's result, or the error its status stands for."""
+    if type(r) is int:
+        check(r, what)
+    return r
+
+
 def shared_prefix_lens(block_tables: list[list[int]], seq_lens: list[int], block_size: int) -> list[int]:
     """Tokens each sequence shares with the previous one (host-side).
 
@@ -126,6 +160,11 @@ def paged_decode(
     with any strides (f32/f16/bf16/e4m3fn); e4m3fn caches need per-KV-head
     fp32 k_scale/v_scale of shape [Hkv] or [1].
     """
+    if _on_gpu(q):
+        r = _fast().paged_decode(q, k_cache, v_cache, block_tables, seq_lens, float(scale), int(block_size), k_scale,
+                                 v_scale, int(partition_tokens), out, workspace, shared_prefix_lens)
+        if r is not None:
+            return _result(r, "cf_paged_decode_shared")
     for name, t in (("q", q), ("k_cache", k_cache), ("v_cache", v_cache), ("block_tables", block_tables),
                     ("seq_lens", seq_lens)):
         _require_device(name, t)
@@ -242,6 +281,11 @@ def prefill_chunk(
     paired tile layout or the reference's token-major rows ([NB, 16, Hkv,
     D] contiguous).
     """
+    if _on_gpu(q):
+        r = _fast().prefill_chunk(q, k_cache, v_cache, block_tables, seq_lens, q_start, float(scale), int(block_size),
+                                  k_scale, v_scale, out, workspace)
+        if r is not None:
+            return _result(r, "cf_prefill_chunk_fp8")
     for name, t in (("q", q), ("k_cache", k_cache), ("v_cache", v_cache), ("block_tables", block_tables),
                     ("seq_lens", seq_lens), ("q_start", q_start)):
         _require_device(name, t)
@@ -390,6 +434,9 @@ def fp8_scale_quantize(*xs: torch.Tensor, per_head: bool) -> list[tuple[torch.Te
     -2, scales [H]) or one in total (scales [1]).  None where the tensors'
     shapes, strides or alignment need the separate calls."""
     x0 = xs[0]
+    r = _fast().scale_quantize(x0, xs[1] if len(xs) == 2 else None, per_head)
+    if r is not None:
+        return list(_result(r, "cf_fp8_scale_quantize"))
     n = x0.numel()
     if n == 0 or n % 16 or not all(
             x.is_cuda and x.is_contiguous() and x.shape == x0.shape and x.dtype == x0.dtype and x.device == x0.device
@@ -420,6 +467,10 @@ def fp8_dequantize_kv(k: torch.Tensor, v: torch.Tensor, k_scales: torch.Tensor,
                       v_scales: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """(f32(k) * k_scales[h], f32(v) * v_scales[h]); one launch for
     contiguous tensors of one shape."""
+    if _on_gpu(k):
+        r = _fast().dequantize_kv(k, v, k_scales, v_scales)
+        if r is not None:
+            return _result(r, "cf_fp8_dequantize_kv")
     for name, t in (("k", k), ("v", v), ("k_scales", k_scales), ("v_scales", v_scales)):
         _require_device(name, t)
     dev = _same_device(k, v, k_scales, v_scales)
@@ -459,6 +510,11 @@ def kv_write_fp8(
     """Quantizes new K/V rows [T, Hkv, D] into paged e4m3fn caches at
     slot_mapping[T].  Slots must be distinct (rows repeating a slot race);
     slots outside the cache are skipped."""
+    if _on_gpu(k_new):
+        r = _fast().kv_write_fp8(k_new, v_new, slot_mapping, k_cache, v_cache, k_scale, v_scale)
+        if r is not None:
+            _result(r, "cf_kv_write_fp8")
+            return
     for name, t in (("k_new", k_new), ("v_new", v_new), ("slot_mapping", slot_mapping), ("k_cache", k_cache),
                     ("v_cache", v_cache), ("k_scale", k_scale), ("v_scale", v_scale)):
         _require_device(name, t)
@@ -477,6 +533,11 @@ def paged_write(
     layout) at slots block * bs + offset; e4m3fn caches quantize with the
     per-head `scale` [H] (or one scale).  Slots outside the cache are
     skipped; slots must be distinct (rows repeating a slot race)."""
+    if _on_gpu(x_new):
+        r = _fast().paged_write(x_new, slot_mapping, cache, scale)
+        if r is not None:
+            _result(r, "cf_paged_write")
+            return
     for name, t in (("x_new", x_new), ("slot_mapping", slot_mapping), ("cache", cache)):
         _require_device(name, t)
     dev = _same_device(x_new, slot_mapping, cache)
@@ -501,6 +562,10 @@ def paged_gather(
     """Dense [R, seq_len, H, D] rows of the tables' first seq_len tokens
     (e4m3fn caches dequantized with `scale`, returned as float32 unless
     out_dtype says otherwise); table entries < 0 give zero rows."""
+    if _on_gpu(cache):
+        r = _fast().paged_gather(cache, block_tables, seq_len, out_dtype, scale, out)
+        if r is not None:
+            return _result(r, "cf_paged_gather")
     _require_device("cache", cache)
     _require_device("block_tables", block_tables)
     dev = _same_device(cache, block_tables)
@@ -529,6 +594,25 @@ def stage_from_host(host_ptr: int, dev_ptr: int, nbytes: int, device: torch.devi
         return False
     check(rc, "cf_stage_from_host")
     return True
+
+
+def stage_tables(host: torch.Tensor, dbuf: torch.Tensor, n_req: int, mb: int
+                 ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """Uploads packed int32 tables [n_req, mb] | lengths | shared-prefix
+    lengths from `host` to `dbuf` (both at least n_req * (mb + 2) + 4 long) on
+    the current stream and returns the three views of `dbuf`.
+
+    The library's upload kernel reads the pinned buffer on the compute queue,
+    ordered with the decode kernels without a copy-engine hand-off; a torch
+    copy where the buffer is not mapped pinned memory."""
+    r = _fast().stage_tables(host, dbuf, n_req, mb)
+    if r is not None:
+        return _result(r, "cf_stage_from_host")
+    used = n_req * (mb + 2)
+    if not stage_from_host(host.data_ptr(), dbuf.data_ptr(), ((used + 3) // 4) * 16, dbuf.device):
+        dbuf[:used].copy_(host[:used], non_blocking=True)
+    return (dbuf[: n_req * mb].view(n_req, mb), dbuf[n_req * mb: n_req * (mb + 1)],
+            dbuf[n_req * (mb + 1): used])
 
 
 def block_tables_apply(table: torch.Tensor, lens: torch.Tensor, deltas: torch.Tensor) -> None:
@@ -681,5 +765,6 @@ __all__ = [
     "paged_write",
     "shared_prefix_lens",
     "stage_from_host",
+    "stage_tables",
     "_abi",
 ]

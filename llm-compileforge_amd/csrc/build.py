@@ -80,6 +80,7 @@ def build(jobs: int = 8, verbose: bool = False) -> Path:
     _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)])
     os.replace(tmp, LIB)
     build_tablepack()
+    build_fastcall()
     return LIB
 
 
@@ -91,6 +92,25 @@ def build_tablepack() -> Path:
     tmp = out.with_name(out.name + ".tmp")
     _run(["gcc", "-O2", "-shared", "-fPIC", "-Wall", f"-I{sysconfig.get_paths()['include']}", str(src), "-o",
           str(tmp)])
+    os.replace(tmp, out)
+    return out
+
+
+def build_fastcall() -> Path:
+    """The CPython extension behind ops.py's calls (host code over torch's C++
+    tensors, g++, in-tree next to the ctypes binding)."""
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    src = PKG / "cf_hip" / "_fastcall.cpp"
+    out = PKG / "cf_hip" / ("_fastcall" + sysconfig.get_config_var("EXT_SUFFIX"))
+    tmp = out.with_name(out.name + ".tmp")
+    libs = library_paths()
+    _run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall", "-Wno-unused-function", "-fvisibility=hidden",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+          *(f"-isystem{p}" for p in include_paths()), f"-I{sysconfig.get_paths()['include']}", f"-I{ROOT / 'include'}",
+          str(src), *(f"-L{p}" for p in libs), *(f"-Wl,-rpath,{p}" for p in libs),
+          "-ltorch_python", "-ltorch_cpu", "-lc10", "-o", str(tmp)])
     os.replace(tmp, out)
     return out
 

@@ -115,39 +115,29 @@ def _as_ids(blocks) -> np.ndarray:
     return np.asarray(blocks, dtype=np.int64)
 
 
-def _staging(device: torch.device, n: int) -> tuple[torch.Tensor, torch.Tensor]:
-    """(pinned host buffer, device buffer) of the next slot, each >= n int32."""
+def _staging(device: torch.device, n: int) -> tuple[torch.Tensor, torch.Tensor, list]:
+    """(pinned host buffer, device buffer) of the next slot, each >= n int32,
+    and the slots' state for _staged."""
     key = (device, _ops.stream_handle(device))
     st = _STAGE.get(key)
     if st is None:
-        st = _STAGE[key] = [[None] * _SLOTS, [None] * _SLOTS, [None] * _SLOTS, 0]
-    hosts, devs, events, k = st
+        st = _STAGE[key] = [[None] * _SLOTS, [None] * _SLOTS, [None] * _SLOTS, 0, torch.cuda.current_stream(device)]
+    hosts, devs, events, k, _ = st
     if events[k] is not None:
         events[k].synchronize()
     if hosts[k] is None or hosts[k].numel() < n + 4:
         size = max(n + 4, 1 << 16)  # + 4: the upload moves whole 16-byte words
         hosts[k] = torch.empty(size, dtype=torch.int32, pin_memory=True)
         devs[k] = torch.empty(size, dtype=torch.int32, device=device)
-    return hosts[k], devs[k]
+    return hosts[k], devs[k], st
 
 
-def _staged(device: torch.device) -> None:
-    st = _STAGE[(device, _ops.stream_handle(device))]
+def _staged(st: list) -> None:
     ev = st[2][st[3]]
     if ev is None:
         ev = st[2][st[3]] = torch.cuda.Event()
-    ev.record(torch.cuda.current_stream(device))
+    ev.record(st[4])
     st[3] = (st[3] + 1) % _SLOTS
-
-def _upload(host: torch.Tensor, dbuf: torch.Tensor, n: int, device: torch.device) -> None:
-    """host[:n] -> dbuf[:n] on the current stream: with the library's
-    compute-queue upload (a kernel reading the pinned buffer, ordered with
-    the decode kernels without a copy-engine hand-off), or a torch copy where
-    the buffer is not mapped pinned memory."""
-    nbytes = ((n + 3) // 4) * 16
-    if _ops.stage_from_host(host.data_ptr(), dbuf.data_ptr(), nbytes, device):
-        return
-    dbuf[:n].copy_(host[:n], non_blocking=True)
 
 
 DEFAULT_PARTITION_TOKENS = _ops.DEFAULT_PARTITION_TOKENS
@@ -254,18 +244,15 @@ def paged_attention(
     nb = k_cache.shape[0]
     n_req = len(rids)
     width = table_width(block_tables)
-    host, dbuf = _staging(q.device, n_req * (width + 2))
+    host, dbuf, slots = _staging(q.device, n_req * (width + 2))
     mb = pack_tables(block_tables, seq_lens, block_size, nb, host.numpy(), width)
-    used = n_req * (mb + 2)
-    dev = dbuf[:used]
-    _upload(host, dbuf, used, q.device)
-    _staged(q.device)
-    dev_tables = dev[: n_req * mb].view(n_req, mb)
-    dev_lens = dev[n_req * mb: n_req * (mb + 1)]
-    dev_shared = dev[n_req * (mb + 1):]
-    out = paged_attention_tensors(
-        q[:n_req], k_cache, v_cache, dev_tables, dev_lens, block_size, scale,
-        k_scale=k_scale, v_scale=v_scale, partition_tokens=partition_tokens, shared_prefix_lens=dev_shared,
+    tables, lens, shared = _ops.stage_tables(host, dbuf, n_req, mb)
+    _staged(slots)
+    if scale is None:
+        scale = 1.0 / math.sqrt(q.shape[-1])
+    out = _ops.paged_decode(
+        q if n_req == q.shape[0] else q[:n_req], k_cache, v_cache, tables, lens, float(scale), int(block_size),
+        k_scale=k_scale, v_scale=v_scale, partition_tokens=partition_tokens, shared_prefix_lens=shared,
     )
     return dict(zip(rids, out.unbind(0)))
 

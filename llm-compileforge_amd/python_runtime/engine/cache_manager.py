@@ -375,7 +375,7 @@ class CacheManager:
 
     def layer_view(self, slab_id: str, layer_idx: int) -> torch.Tensor:
         """Layer `layer_idx` of a paged slab as [num_blocks, block_size, heads, dim]."""
-        return self._slabs[slab_id][:, layer_idx]
+        return self._slabs[slab_id].select(1, layer_idx)
 
     def write_paged(self, slab_id: str, layer_idx: int, data: torch.Tensor, positions: torch.Tensor) -> None:
         """Writes token rows `data` at `positions` of this step's requests.
@@ -496,7 +496,8 @@ class CacheManager:
         rows = normalize_kv(data, spec.num_heads, spec.head_dim)
         if rows.dim() != 3:
             raise ValueError(f"write_slots: cannot read {tuple(data.shape)} as [seq, {spec.num_heads}, {spec.head_dim}]")
-        slots = torch.as_tensor(slots).reshape(-1).to(self._device)
+        if not (isinstance(slots, torch.Tensor) and slots.dim() == 1 and slots.device == self._device):
+            slots = torch.as_tensor(slots).reshape(-1).to(self._device)
         if slots.numel() != rows.shape[0]:
             raise ValueError(f"write_slots: {slots.numel()} slots for {rows.shape[0]} rows")
         if rows.device != self._device:
