@@ -259,13 +259,15 @@ __global__ __launch_bounds__(256) void kv_write_native_kernel(KvWriteParams p, u
   // Lane 1 + e <-> row e of the group.  Runs start at valid rows that do not
   // continue the previous one; the group owns the valid rows 0..15 from its
   // first run start on, and rows 16..30 that continue its last run.
+  // each row's destination (block row base + token offset), per lane: computed
+  // before any lane leaves, as rows are read from lanes whose channel is past
+  // the last one too
+  const int64_t dst = valid ? (sl >> 4) * p.vc_s[0] + (sl & 15) : 0;
   const uint32_t starts = vm & ~cm & 0x1FFFEu;
   if (!mine || starts == 0u) return;
   const int e0 = __builtin_ctz(starts) - 1;     // first owned row, 0..15
   const int ext = __builtin_ctz(~(cm >> 17));  // <= 15: runs stop at a block end
   const uint32_t own = ((vm & 0x1FFFEu & ~((2u << e0) - 1u)) >> 1) | (((1u << ext) - 1u) << 16);
-  // each row's destination (block row base + token offset), per lane
-  const int64_t dst = valid ? (sl >> 4) * p.vc_s[0] + (sl & 15) : 0;
   const uint32_t chan = (uint32_t)((int64_t)h * p.vc_s[2] + d * 16);
   uint8_t* vcache = (uint8_t*)p.v_cache;
   auto dst_of = [&](int e) {  // row e's destination (uniform)

@@ -348,3 +348,23 @@ def test_one_call_quantize_keeps_nan_and_infinity_rules(gpu):
         q, s = quant.quantize_block(x)
         wc, ws = ofp8.quantize_block(x.cpu().numpy())
         assert s.item() == ws and np.array_equal(codes(q), wc)
+
+
+@pytest.mark.parametrize("h,d", [(1, 16), (3, 16), (1, 80), (5, 48)])
+def test_paged_write_of_channels_that_do_not_fill_a_wave(gpu, h, d):
+    """K/V rows of fewer (or more) channels than whole 64-lane waves: every
+    row lands, whichever lanes have a channel."""
+    g = torch.Generator(device=gpu).manual_seed(h * d)
+    n, nb = 75, 9
+    k, v = (torch.randn(n, h, d, generator=g, device=gpu).to(torch.bfloat16) for _ in range(2))
+    ks, vs = ops.fp8_amax_scale(k), ops.fp8_amax_scale(v)
+    kc, vc = L.alloc_kv_cache(nb, 16, h, d, torch.float8_e4m3fn, gpu, "native")
+    kc.view(torch.uint8).zero_()
+    vc.view(torch.uint8).zero_()
+    slots = torch.arange(n, device=gpu) + 37
+    ops.kv_write_fp8(k, v, slots, kc, vc, ks, vs)
+    for x, sc, c in ((k, ks, kc), (v, vs, vc)):
+        want = np.zeros((nb * 16, h, d), np.uint8)
+        for i in range(h):
+            want[37:37 + n, i] = ofp8.quantize(x[:, i].float().cpu().numpy(), float(sc[i]))
+        assert np.array_equal(codes(c).reshape(nb * 16, h, d), want)
