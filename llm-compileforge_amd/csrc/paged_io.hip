@@ -14,11 +14,14 @@
 // request's blocks in table order and leaves positions past its table zero,
 // cache_manager.py:173-197).
 //
-// Both kernels give one thread a piece of 16 channels of one (token, head)
-// row when the head dim is a multiple of 16 (a lone channel otherwise),
-// and move a piece with 16-byte loads / stores where the row is contiguous
-// and aligned, element by element otherwise (e.g. the channel-major V
-// layout, token stride 1).
+// A thread of the row kernels takes a piece of one (token, head) row: as many
+// channels as make 16 bytes of the wider side where rows are contiguous and
+// aligned (so a wave's accesses on that side are whole 1 KiB runs), one
+// channel otherwise.  Channel-major caches of 16-token blocks (the native V
+// tile: the 16 tokens of a channel are contiguous) have kernels of their own,
+// a thread taking one channel's tokens of a block: every access is then a run
+// along the channels or along the tokens.  All are bound by latency for a
+// decode step's rows and by bytes for a prompt's.
 #include "cf_device.hpp"
 #include "cf_host.hpp"
 #include "paged_io.hpp"
@@ -39,192 +42,401 @@ __device__ __forceinline__ void store_from_f32(void* base, int64_t i, float v) {
   E::store((typename E::T*)base + i, v);
 }
 
-// Loads n (<= 16) elements of one row as f32: 16-byte vectors when `vec`
-// (then n == 16 and the address is 16-byte aligned), strided otherwise.
+// Bytes of an element, and channels per piece of a pair of dtypes.
 template <int DT>
-__device__ __forceinline__ void load_row(const void* base, int64_t off, int64_t stride, int n, bool vec, float* f) {
-  if (vec) {
-    constexpr int EB = sizeof(typename Elem<DT>::T);
-    const uint4* s = (const uint4*)((const char*)base + off * EB);
+constexpr int esize() {
+  return (int)sizeof(typename Elem<DT>::T);
+}
+template <int A, int B>
+constexpr int piece_channels() {
+  return 16 / (esize<A>() > esize<B>() ? esize<A>() : esize<B>());
+}
+
+template <int BYTES>
+struct Raw;
+template <>
+struct Raw<4> {
+  using T = uint32_t;
+};
+template <>
+struct Raw<8> {
+  using T = uint2;
+};
+template <>
+struct Raw<16> {
+  using T = uint4;
+};
+
+// N consecutive elements (one aligned access of 4, 8 or 16 bytes) as f32.
+template <int DT, int N>
+__device__ __forceinline__ void load_piece(const void* base, int64_t off, float* f) {
+  using T = typename Elem<DT>::T;
+  using R = typename Raw<N * esize<DT>()>::T;
+  union {
+    R raw;
+    T e[N];
+  } u;
+  u.raw = *(const R*)((const T*)base + off);
 #pragma unroll
-    for (int q = 0; q < 16 * EB / 16; ++q) {
-      const uint4 u = s[q];
-      const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+  for (int k = 0; k < N; ++k) f[k] = Elem<DT>::load(&u.e[k]);
+}
+
+// One value as DT's bits (e4m3fn: the code of f / scale).
+template <int DT>
+__device__ __forceinline__ typename Elem<DT>::T encode(float f, const Fp8Quant& qz) {
+  typename Elem<DT>::T v;
+  if constexpr (DT == kE4M3) v = qz(f);
+  else Elem<DT>::store(&v, f);
+  return v;
+}
+
+template <int DT, int N>
+__device__ __forceinline__ void store_piece(void* base, int64_t off, const float* f, const Fp8Quant& qz) {
+  using T = typename Elem<DT>::T;
+  using R = typename Raw<N * esize<DT>()>::T;
+  union {
+    R raw;
+    T e[N];
+  } u;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if constexpr (EB == 4) {
-          f[4 * q + j] = u2f(w[j]);
-        } else if constexpr (EB == 2) {
-          f[8 * q + 2 * j] = Elem<DT>::load((const typename Elem<DT>::T*)&w[j]);
-          f[8 * q + 2 * j + 1] = Elem<DT>::load((const typename Elem<DT>::T*)&w[j] + 1);
-        } else {
+  for (int k = 0; k < N; ++k) u.e[k] = encode<DT>(f[k], qz);
+  *(R*)((T*)base + off) = u.raw;
+}
+
+template <int ST>
+__device__ __forceinline__ int64_t slot_of(const PagedWriteParams& p, int64_t i) {
+  return ST == kI64 ? ((const int64_t*)p.slots)[i * p.slot_s] : (int64_t)((const int32_t*)p.slots)[i * p.slot_s];
+}
+
+// One thread per piece of N channels (N == 1: any strides).
+template <int XT, int ST, int CT, int N>
+__global__ __launch_bounds__(256) void paged_write_kernel(PagedWriteParams p) {
+  const int np = p.D / N;
+  const int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t total = p.T * p.H * np;
+  if (u >= total) return;
+  int64_t i;
+  int h, c;
+  if (total <= (int64_t)UINT32_MAX) {  // 32-bit divisions
+    const uint32_t v = (uint32_t)u, r = v / (uint32_t)np;
+    c = (int)(v - r * (uint32_t)np);
+    i = r / (uint32_t)p.H;
+    h = (int)(r - (uint32_t)i * (uint32_t)p.H);
+  } else {
+    c = (int)(u % np), h = (int)((u / np) % p.H);
+    i = u / ((int64_t)np * p.H);
+  }
+  float f[N];
+  const int64_t xo = i * p.x_s[0] + h * p.x_s[1] + (int64_t)c * N * p.x_s[2];
+  if constexpr (N == 1) f[0] = load_as_f32<XT>(p.x, xo);
+  else load_piece<XT, N>(p.x, xo, f);
+  const int64_t sl = slot_of<ST>(p, i);
+  if (sl < 0 || sl >= p.NB * p.bs) return;
+  const int64_t blk = sl / p.bs, off = sl - blk * p.bs;
+  const Fp8Quant qz(CT == kE4M3 ? p.scale[h * p.sc_s] : 1.0f);
+  const int64_t co = blk * p.c_s[0] + off * p.c_s[1] + h * p.c_s[2] + (int64_t)c * N * p.c_s[3];
+  if constexpr (N == 1) ((typename Elem<CT>::T*)p.cache)[co] = encode<CT>(f[0], qz);
+  else store_piece<CT, N>(p.cache, co, f, qz);
+}
+
+// Channel-major 16-token blocks (token stride 1, channel stride 16): a
+// workgroup takes 16 new rows of 256 (head, channel)s, a thread one channel.
+// Rows are split into runs of consecutive slots inside one block; the group
+// writes the runs that start in it (the last may reach up to 15 rows past
+// it), a run of 16 as the block's whole channel row.  Run boundaries depend
+// only on the slots, so every thread of the group writes the same runs.
+template <int XT, int ST, int CT>
+__global__ __launch_bounds__(256) void paged_write_tile_kernel(PagedWriteParams p, uint32_t chunks) {
+  using X = typename Elem<XT>::T;
+  using C = typename Elem<CT>::T;
+  const uint32_t g = blockIdx.x / chunks;
+  const int hd = (int)(blockIdx.x - g * chunks) * 256 + (int)threadIdx.x;
+  const bool mine = hd < p.H * p.D;
+  const int h = mine ? hd / p.D : 0, d = mine ? hd % p.D : 0;
+  // lane l: the slot of row g * 16 - 1 + l (-1 outside [0, T))
+  const int lane = (int)(threadIdx.x & 63);
+  const int64_t r = (int64_t)g * 16 - 1 + lane;
+  const int64_t sl = r >= 0 && r < p.T ? slot_of<ST>(p, r) : -1;
+  // rows g*16 .. g*16+30 of this channel (clamped to the last row), loaded
+  // while the slots are in flight
+  const int64_t row0 = (int64_t)g * 16;
+  const int last = (int)(p.T - 1 - row0 < 30 ? p.T - 1 - row0 : 30);
+  const X* src = (const X*)p.x + row0 * p.x_s[0] + h * p.x_s[1] + (int64_t)d * p.x_s[2];
+  X raw[31];
 #pragma unroll
-          for (int b = 0; b < 4; ++b) f[16 * q + 4 * j + b] = Elem<DT>::load((const typename Elem<DT>::T*)&w[j] + b);
-        }
+  for (int e = 0; e < 31; ++e) raw[e] = src[(int64_t)(e < last ? e : last) * p.x_s[0]];
+  const bool valid = sl >= 0 && sl < p.NB * 16;
+  const int64_t up = __shfl_up(sl, 1, 64);
+  const bool cont = valid && lane > 0 && sl == up + 1 && (sl & 15) != 0;
+  const uint32_t vm = (uint32_t)__ballot(valid), cm = (uint32_t)__ballot(cont);
+  // lane 1 + e <-> row e of the group
+  // (computed before any lane leaves: rows are read from lanes whose channel
+  // is past the last one too)
+  const int64_t dst = valid ? (sl >> 4) * p.c_s[0] + (sl & 15) : 0;
+  const uint32_t starts = vm & ~cm & 0x1FFFEu;
+  if (!mine || starts == 0u) return;
+  const int e0 = __builtin_ctz(starts) - 1;    // first owned row, 0..15
+  const int ext = __builtin_ctz(~(cm >> 17));  // rows past the group that continue its last run, <= 15
+  const uint32_t own = ((vm & 0x1FFFEu & ~((2u << e0) - 1u)) >> 1) | (((1u << ext) - 1u) << 16);
+  C* chan = (C*)p.cache + (int64_t)h * p.c_s[2] + (int64_t)d * 16;
+  auto dst_of = [&](int e) {  // row e's block and token offset (uniform)
+    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)(uint64_t)dst, e + 1);
+    const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)((uint64_t)dst >> 32), e + 1);
+    return (int64_t)(((uint64_t)hi << 32) | lo);
+  };
+  const Fp8Quant qz(CT == kE4M3 ? p.scale[h * p.sc_s] : 1.0f);
+  if ((own >> e0) == 0xFFFFu && ((cm >> (e0 + 2)) & 0x7FFFu) == 0x7FFFu) {
+    // 16 rows that fill a block's channel row
+    union {
+      uint4 q[esize<CT>()];
+      C c[16];
+    } out;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      if (e0 == k) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) out.c[j] = encode<CT>(Elem<XT>::load(&raw[k + j]), qz);
       }
     }
-  } else {
-    for (int e = 0; e < n; ++e) f[e] = load_as_f32<DT>(base, off + e * stride);
-  }
-}
-
-// Stores n (<= 16) values of one row converted to DT (e4m3fn: divided by
-// `div` first); vector stores when `vec`.
-template <int DT>
-__device__ __forceinline__ void store_row(void* base, int64_t off, int64_t stride, int n, bool vec, const float* f,
-                                          float div) {
-  using E = Elem<DT>;
-  using T = typename E::T;
-  if (vec) {
-    constexpr int EB = sizeof(T);
-    T tmp[16];
+    uint4* to = (uint4*)(chan + dst_of(e0));
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      if constexpr (DT == kE4M3) tmp[e] = e4m3_from_f32(f[e] / div);
-      else E::store(&tmp[e], f[e]);
-    }
-    uint4* d = (uint4*)((char*)base + off * EB);
-#pragma unroll
-    for (int q = 0; q < 16 * EB / 16; ++q) d[q] = ((const uint4*)tmp)[q];
-  } else {
-    for (int e = 0; e < n; ++e) {
-      T* dst = (T*)base + off + e * stride;
-      if constexpr (DT == kE4M3) *dst = e4m3_from_f32(f[e] / div);
-      else E::store(dst, f[e]);
-    }
+    for (int q = 0; q < esize<CT>(); ++q) to[q] = out.q[q];
+    return;
   }
+#pragma unroll
+  for (int e = 0; e < 31; ++e)
+    if ((own >> e) & 1u) chan[dst_of(e)] = encode<CT>(Elem<XT>::load(&raw[e]), qz);
 }
 
-template <int XT, int ST, int CT>
-__global__ __launch_bounds__(256) void paged_write_kernel(PagedWriteParams p, int pw, bool xvec, bool cvec) {
-  const int np = p.D / pw;
+template <int CT, int OT, int N>
+__global__ __launch_bounds__(256) void paged_gather_kernel(PagedGatherParams p) {
+  const int np = p.D / N;
   const int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (u >= p.T * p.H * np) return;
-  const int c = (int)(u % np), h = (int)((u / np) % p.H);
-  const int64_t i = u / ((int64_t)np * p.H);
-  const int64_t sl = ST == kI64 ? ((const int64_t*)p.slots)[i * p.slot_s]
-                                : (int64_t)((const int32_t*)p.slots)[i * p.slot_s];
-  if (sl < 0 || sl >= p.NB * p.bs) return;
-  const int64_t blk = sl / p.bs, off = sl % p.bs;
-  float f[16];
-  load_row<XT>(p.x, i * p.x_s[0] + h * p.x_s[1] + (int64_t)c * pw * p.x_s[2], p.x_s[2], pw, xvec, f);
-  const float div = CT == kE4M3 ? p.scale[h * p.sc_s] : 1.0f;
-  store_row<CT>(p.cache, blk * p.c_s[0] + off * p.c_s[1] + h * p.c_s[2] + (int64_t)c * pw * p.c_s[3], p.c_s[3], pw,
-                cvec, f, div);
-}
-
-template <int CT, int OT>
-__global__ __launch_bounds__(256) void paged_gather_kernel(PagedGatherParams p, int pw, bool cvec, bool ovec) {
-  const int np = p.D / pw;
-  const int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (u >= (int64_t)p.R * p.S * p.H * np) return;
-  const int c = (int)(u % np), h = (int)((u / np) % p.H);
-  const int64_t rs = u / ((int64_t)np * p.H);
-  const int s = (int)(rs % p.S), r = (int)(rs / p.S);
+  const int64_t total = (int64_t)p.R * p.S * p.H * np;
+  if (u >= total) return;
+  int c, h, s, r;
+  if (total <= (int64_t)UINT32_MAX) {
+    const uint32_t v = (uint32_t)u, a = v / (uint32_t)np, b = a / (uint32_t)p.H;
+    c = (int)(v - a * (uint32_t)np);
+    h = (int)(a - b * (uint32_t)p.H);
+    r = (int)(b / (uint32_t)p.S);
+    s = (int)(b - (uint32_t)r * (uint32_t)p.S);
+  } else {
+    c = (int)(u % np), h = (int)((u / np) % p.H);
+    const int64_t rs = u / ((int64_t)np * p.H);
+    s = (int)(rs % p.S), r = (int)(rs / p.S);
+  }
   const int jb = s / p.bs;
   int64_t blk = -1;
   if (jb < p.Mb) {
     const int id = p.tables[(int64_t)r * p.t_sr + (int64_t)jb * p.t_sm];
     if (id >= 0 && id < p.NB) blk = id;
   }
-  float f[16];
+  float f[N];
   if (blk >= 0) {
-    load_row<CT>(p.cache, blk * p.c_s[0] + (int64_t)(s % p.bs) * p.c_s[1] + h * p.c_s[2] + (int64_t)c * pw * p.c_s[3],
-                 p.c_s[3], pw, cvec, f);
+    const int64_t co =
+        blk * p.c_s[0] + (int64_t)(s - jb * p.bs) * p.c_s[1] + h * p.c_s[2] + (int64_t)c * N * p.c_s[3];
+    if constexpr (N == 1) f[0] = load_as_f32<CT>(p.cache, co);
+    else load_piece<CT, N>(p.cache, co, f);
     if constexpr (CT == kE4M3) {
       const float sc = p.scale[h * p.sc_s];
-      for (int e = 0; e < pw; ++e) f[e] *= sc;
+#pragma unroll
+      for (int e = 0; e < N; ++e) f[e] *= sc;
     }
   } else {
-    for (int e = 0; e < pw; ++e) f[e] = 0.0f;
+#pragma unroll
+    for (int e = 0; e < N; ++e) f[e] = 0.0f;
   }
-  store_row<OT>(p.out, (int64_t)r * p.o_s[0] + (int64_t)s * p.o_s[1] + h * p.o_s[2] + (int64_t)c * pw * p.o_s[3],
-                p.o_s[3], pw, ovec, f, 1.0f);
+  const int64_t oo = (int64_t)r * p.o_s[0] + (int64_t)s * p.o_s[1] + h * p.o_s[2] + (int64_t)c * N * p.o_s[3];
+  if constexpr (N == 1) store_from_f32<OT>(p.out, oo, f[0]);
+  else store_piece<OT, N>(p.out, oo, f, Fp8Quant(1.0f));
 }
 
-int dt_bytes(int dt) { return dt == kF32 ? 4 : (dt == kE4M3 ? 1 : 2); }
+// Channel-major 16-token blocks into token rows: a thread reads the 16 tokens
+// of P adjacent channels of one block (whole runs along the channels) and
+// writes them to the 16 rows, P channels a store (4 bytes: 256-byte runs).
+template <int CT, int OT, int P>
+__global__ __launch_bounds__(256) void paged_gather_tile_kernel(PagedGatherParams p, int blocks_per_row) {
+  using C = typename Elem<CT>::T;
+  using O = typename Elem<OT>::T;
+  const uint32_t per = (uint32_t)(p.H * p.D / P);
+  const int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t total = (int64_t)p.R * blocks_per_row * per;
+  if (u >= total) return;
+  int64_t rb;
+  int r;
+  if (total <= (int64_t)UINT32_MAX) {
+    rb = (uint32_t)u / per;
+    r = (int)((uint32_t)rb / (uint32_t)blocks_per_row);
+  } else {
+    rb = u / per;
+    r = (int)(rb / blocks_per_row);
+  }
+  const int hd = (int)(u - rb * per) * P;
+  const int jb = (int)(rb - (int64_t)r * blocks_per_row);
+  const int h = hd / p.D, d = hd - h * p.D;
+  int64_t blk = -1;
+  if (jb < p.Mb) {
+    const int id = p.tables[(int64_t)r * p.t_sr + (int64_t)jb * p.t_sm];
+    if (id >= 0 && id < p.NB) blk = id;
+  }
+  union {
+    uint4 q[P][esize<CT>()];
+    C c[P][16];
+  } in;
+  if (blk >= 0) {
+    const uint4* src = (const uint4*)((const C*)p.cache + blk * p.c_s[0] + (int64_t)h * p.c_s[2] + (int64_t)d * 16);
+#pragma unroll
+    for (int k = 0; k < P; ++k)
+#pragma unroll
+      for (int q = 0; q < esize<CT>(); ++q) in.q[k][q] = src[k * esize<CT>() + q];
+  }
+  const float sc = CT == kE4M3 ? p.scale[h * p.sc_s] : 1.0f;
+  const int s0 = jb * 16, ns = min(16, p.S - s0);
+  O* out = (O*)p.out + (int64_t)r * p.o_s[0] + (int64_t)s0 * p.o_s[1] + (int64_t)h * p.o_s[2] + d;
+#pragma unroll
+  for (int t = 0; t < 16; ++t) {
+    if (t < ns) {
+      O v[P];
+#pragma unroll
+      for (int k = 0; k < P; ++k) {
+        float f = blk >= 0 ? Elem<CT>::load(&in.c[k][t]) : 0.0f;
+        if constexpr (CT == kE4M3) f = blk >= 0 ? f * sc : 0.0f;
+        Elem<OT>::store(&v[k], f);
+      }
+      if constexpr (P * sizeof(O) == 4) *(uint32_t*)(out + (int64_t)t * p.o_s[1]) = __builtin_bit_cast(uint32_t, v);
+      else out[(int64_t)t * p.o_s[1]] = v[0];
+    }
+  }
+}
 
-// A row piece of 16 elements at element offsets base + k * (row strides)
-// moves as 16-byte vectors when the innermost stride is 1 and every row
-// start is 16-byte aligned.
-bool rows_aligned(const void* base, const int64_t* strides, int n_outer, int64_t inner, int eb) {
-  if (inner != 1 || ((uintptr_t)base & 15)) return false;
+// Whether rows at element strides `strides` (and base) start on multiples of
+// `bytes` and are contiguous along the channels.
+bool rows_aligned(const void* base, const int64_t* strides, int n_outer, int64_t inner, int eb, int bytes) {
+  if (inner != 1 || ((uintptr_t)base & (uintptr_t)(bytes - 1))) return false;
   for (int i = 0; i < n_outer; ++i)
-    if ((strides[i] * eb) % 16 != 0) return false;
+    if ((strides[i] * eb) % bytes != 0) return false;
   return true;
 }
 
+// The native V tile: 16-token blocks, token stride 1, channel stride 16,
+// 16-byte aligned channel rows.
+bool channel_tiles(const void* base, const int64_t* c_s, int bs, int eb) {
+  return bs == 16 && c_s[1] == 1 && c_s[3] == 16 && ((uintptr_t)base & 15) == 0 && (c_s[0] * eb) % 16 == 0 &&
+         (c_s[2] * eb) % 16 == 0;
+}
+
 int64_t grid_of(int64_t threads) { return (threads + 255) / 256; }
+
+// Values (rows x channels) from which the channel-major write goes by whole
+// blocks.  A thread there walks 16 rows, which takes 5.4 us however few they
+// are; a thread per element is done in 2.3 us for a decode step, but writes 2
+// bytes of every 32.  Both sides, fp16 rows of 8 heads of 128 (4 of 64): 512
+// rows 4.1 / 5.6 us by element / by block (2.9 / 5.4), 1,024 rows 6.0 / 5.7
+// (3.6 / 5.4), 3,577 rows 15.4 / 8.2 (7.4 / 5.4); fp32 and e4m3 cross there too.
+constexpr int64_t kTileWriteValues = 3 << 18;
+
+template <int XT, int ST, int CT>
+int32_t launch_write_t(const PagedWriteParams& p, hipStream_t stream) {
+  ProfileScope prof("cf_paged_write", stream);
+  if (p.T * p.H * p.D >= kTileWriteValues && channel_tiles(p.cache, p.c_s, p.bs, esize<CT>())) {
+    const int64_t chunks = grid_of((int64_t)p.H * p.D), blocks = ceil_div(p.T, 16) * chunks;
+    CF_CHECK(blocks < (int64_t)INT32_MAX, "paged write too large");
+    CF_LAUNCH((paged_write_tile_kernel<XT, ST, CT>), dim3((unsigned)blocks), dim3(256), 0, stream, p, (uint32_t)chunks);
+    CF_HIP_CHECK(hipGetLastError());
+    return CF_OK;
+  }
+  constexpr int N = piece_channels<XT, CT>();
+  const bool vec = p.D % N == 0 && rows_aligned(p.x, p.x_s, 2, p.x_s[2], esize<XT>(), N * esize<XT>()) &&
+                   rows_aligned(p.cache, p.c_s, 3, p.c_s[3], esize<CT>(), N * esize<CT>());
+  const int64_t threads = p.T * p.H * (vec ? p.D / N : p.D);
+  CF_CHECK(grid_of(threads) < (int64_t)INT32_MAX, "paged write too large");
+  const dim3 grid((unsigned)grid_of(threads));
+  if (vec) CF_LAUNCH((paged_write_kernel<XT, ST, CT, N>), grid, dim3(256), 0, stream, p);
+  else CF_LAUNCH((paged_write_kernel<XT, ST, CT, 1>), grid, dim3(256), 0, stream, p);
+  CF_HIP_CHECK(hipGetLastError());
+  return CF_OK;
+}
+
+template <int XT, int ST>
+int32_t launch_write_c(const PagedWriteParams& p, int cache_dt, hipStream_t stream) {
+  switch (cache_dt) {
+    case kF32: return launch_write_t<XT, ST, kF32>(p, stream);
+    case kF16: return launch_write_t<XT, ST, kF16>(p, stream);
+    case kBF16: return launch_write_t<XT, ST, kBF16>(p, stream);
+    case kE4M3: return launch_write_t<XT, ST, kE4M3>(p, stream);
+  }
+  set_error("paged write: unsupported cache dtype %d", cache_dt);
+  return CF_ERR_UNSUPPORTED;
+}
+
+template <int ST>
+int32_t launch_write_x(const PagedWriteParams& p, int x_dt, int cache_dt, hipStream_t stream) {
+  switch (x_dt) {
+    case kF32: return launch_write_c<kF32, ST>(p, cache_dt, stream);
+    case kF16: return launch_write_c<kF16, ST>(p, cache_dt, stream);
+    case kBF16: return launch_write_c<kBF16, ST>(p, cache_dt, stream);
+  }
+  set_error("paged write: unsupported row dtype %d", x_dt);
+  return CF_ERR_UNSUPPORTED;
+}
+
+template <int CT, int OT>
+int32_t launch_gather_t(const PagedGatherParams& p, hipStream_t stream) {
+  ProfileScope prof("cf_paged_gather", stream);
+  // channels per thread of the tile kernel: 4 bytes of output
+  constexpr int P = esize<OT>() == 4 ? 1 : 2;
+  if (channel_tiles(p.cache, p.c_s, p.bs, esize<CT>()) && p.D % P == 0 && (int64_t)p.H * p.D < INT32_MAX &&
+      rows_aligned(p.out, p.o_s, 3, p.o_s[3], esize<OT>(), P * esize<OT>())) {
+    const int64_t bpr = ceil_div(p.S, 16);
+    const int64_t threads = (int64_t)p.R * bpr * (p.H * p.D / P);
+    CF_CHECK(grid_of(threads) < (int64_t)INT32_MAX, "paged gather too large");
+    CF_LAUNCH((paged_gather_tile_kernel<CT, OT, P>), dim3((unsigned)grid_of(threads)), dim3(256), 0, stream, p,
+              (int)bpr);
+    CF_HIP_CHECK(hipGetLastError());
+    return CF_OK;
+  }
+  constexpr int N = piece_channels<CT, OT>();
+  const bool vec = p.D % N == 0 && rows_aligned(p.cache, p.c_s, 3, p.c_s[3], esize<CT>(), N * esize<CT>()) &&
+                   rows_aligned(p.out, p.o_s, 3, p.o_s[3], esize<OT>(), N * esize<OT>());
+  const int64_t threads = (int64_t)p.R * p.S * p.H * (vec ? p.D / N : p.D);
+  CF_CHECK(grid_of(threads) < (int64_t)INT32_MAX, "paged gather too large");
+  const dim3 grid((unsigned)grid_of(threads));
+  if (vec) CF_LAUNCH((paged_gather_kernel<CT, OT, N>), grid, dim3(256), 0, stream, p);
+  else CF_LAUNCH((paged_gather_kernel<CT, OT, 1>), grid, dim3(256), 0, stream, p);
+  CF_HIP_CHECK(hipGetLastError());
+  return CF_OK;
+}
+
+template <int CT>
+int32_t launch_gather_o(const PagedGatherParams& p, int out_dt, hipStream_t stream) {
+  switch (out_dt) {
+    case kF32: return launch_gather_t<CT, kF32>(p, stream);
+    case kF16: return launch_gather_t<CT, kF16>(p, stream);
+    case kBF16: return launch_gather_t<CT, kBF16>(p, stream);
+  }
+  set_error("paged gather: unsupported output dtype %d", out_dt);
+  return CF_ERR_UNSUPPORTED;
+}
 
 }  // namespace
 
 int32_t launch_paged_write(const PagedWriteParams& p, int x_dt, int slot_dt, int cache_dt, hipStream_t stream) {
   if (p.T == 0 || p.H == 0 || p.D == 0) return CF_OK;
-  const int pw = p.D % 16 == 0 ? 16 : 1;
-  const bool xvec = pw == 16 && rows_aligned(p.x, p.x_s, 2, p.x_s[2], dt_bytes(x_dt));
-  const bool cvec = pw == 16 && rows_aligned(p.cache, p.c_s, 3, p.c_s[3], dt_bytes(cache_dt));
-  const int64_t threads = p.T * p.H * (p.D / pw);
-  CF_CHECK(grid_of(threads) < (int64_t)INT32_MAX, "paged write too large");
-  const dim3 grid((unsigned)grid_of(threads));
-  ProfileScope prof("cf_paged_write", stream);
-#define CF_PW(XT, ST, CT) \
-  CF_LAUNCH((paged_write_kernel<XT, ST, CT>), grid, dim3(256), 0, stream, p, pw, xvec, cvec)
-#define CF_PW_C(XT, ST)                                                              \
-  switch (cache_dt) {                                                                \
-    case kF32: CF_PW(XT, ST, kF32); break;                                           \
-    case kF16: CF_PW(XT, ST, kF16); break;                                           \
-    case kBF16: CF_PW(XT, ST, kBF16); break;                                         \
-    case kE4M3: CF_PW(XT, ST, kE4M3); break;                                         \
-    default: set_error("paged write: unsupported cache dtype %d", cache_dt); return CF_ERR_UNSUPPORTED; \
-  }
-#define CF_PW_X(ST)                                                                  \
-  switch (x_dt) {                                                                    \
-    case kF32: CF_PW_C(kF32, ST); break;                                             \
-    case kF16: CF_PW_C(kF16, ST); break;                                             \
-    case kBF16: CF_PW_C(kBF16, ST); break;                                           \
-    default: set_error("paged write: unsupported row dtype %d", x_dt); return CF_ERR_UNSUPPORTED; \
-  }
-  if (slot_dt == kI64) {
-    CF_PW_X(kI64);
-  } else {
-    CF_PW_X(kI32);
-  }
-#undef CF_PW_X
-#undef CF_PW_C
-#undef CF_PW
-  CF_HIP_CHECK(hipGetLastError());
-  return CF_OK;
+  return slot_dt == kI64 ? launch_write_x<kI64>(p, x_dt, cache_dt, stream)
+                         : launch_write_x<kI32>(p, x_dt, cache_dt, stream);
 }
 
 int32_t launch_paged_gather(const PagedGatherParams& p, int cache_dt, int out_dt, hipStream_t stream) {
   if (p.R == 0 || p.S == 0 || p.H == 0 || p.D == 0) return CF_OK;
-  const int pw = p.D % 16 == 0 ? 16 : 1;
-  const bool cvec = pw == 16 && rows_aligned(p.cache, p.c_s, 3, p.c_s[3], dt_bytes(cache_dt));
-  const bool ovec = pw == 16 && rows_aligned(p.out, p.o_s, 3, p.o_s[3], dt_bytes(out_dt));
-  const int64_t threads = (int64_t)p.R * p.S * p.H * (p.D / pw);
-  CF_CHECK(grid_of(threads) < (int64_t)INT32_MAX, "paged gather too large");
-  const dim3 grid((unsigned)grid_of(threads));
-  ProfileScope prof("cf_paged_gather", stream);
-#define CF_PG(CT, OT) \
-  CF_LAUNCH((paged_gather_kernel<CT, OT>), grid, dim3(256), 0, stream, p, pw, cvec, ovec)
-#define CF_PG_O(CT)                                                                  \
-  switch (out_dt) {                                                                  \
-    case kF32: CF_PG(CT, kF32); break;                                               \
-    case kF16: CF_PG(CT, kF16); break;                                               \
-    case kBF16: CF_PG(CT, kBF16); break;                                             \
-    default: set_error("paged gather: unsupported output dtype %d", out_dt); return CF_ERR_UNSUPPORTED; \
-  }
   switch (cache_dt) {
-    case kF32: CF_PG_O(kF32); break;
-    case kF16: CF_PG_O(kF16); break;
-    case kBF16: CF_PG_O(kBF16); break;
-    case kE4M3: CF_PG_O(kE4M3); break;
-    default: set_error("paged gather: unsupported cache dtype %d", cache_dt); return CF_ERR_UNSUPPORTED;
+    case kF32: return launch_gather_o<kF32>(p, out_dt, stream);
+    case kF16: return launch_gather_o<kF16>(p, out_dt, stream);
+    case kBF16: return launch_gather_o<kBF16>(p, out_dt, stream);
+    case kE4M3: return launch_gather_o<kE4M3>(p, out_dt, stream);
   }
-#undef CF_PG_O
-#undef CF_PG
-  CF_HIP_CHECK(hipGetLastError());
-  return CF_OK;
+  set_error("paged gather: unsupported cache dtype %d", cache_dt);
+  return CF_ERR_UNSUPPORTED;
 }
 
 // ---- upload of host-packed tables --------------------------------------------

@@ -371,3 +371,58 @@ def test_hal_cache_ops(gpu):
     assert out.shape == (2, 2, 20, 2, 64) and out.dtype == torch.float32
     assert torch.equal(out[0], ops.paged_gather(kc, table, 20, scale=ks))
     assert torch.equal(out[1], ops.paged_gather(vc, table, 20, scale=vs))
+
+
+@pytest.mark.parametrize("rows_dtype,cache_dtype", [
+    (torch.float32, torch.float32), (torch.float16, torch.float16), (torch.bfloat16, torch.float8_e4m3fn),
+    (torch.float32, torch.bfloat16)])
+@pytest.mark.parametrize("cut", [[1], [0], [-16], [5, 31, 16, -40, 1, 32]])
+@pytest.mark.parametrize("h,d", [(8, 128), (3, 40), (1, 16)])
+def test_channel_major_rows_bit_exact(gpu, rows_dtype, cache_dtype, cut, h, d):
+    """Rows of several sequences (some skipped, some out of order) into a
+    channel-major cache and back, against torch's indexing and casts; one row
+    below and at the size from which the write goes by blocks, and above it
+    with ragged runs."""
+    at_size = (3 << 18) // (h * d) + 1
+    lens = [n for n in cut if n > 0] if len(cut) > 1 else []
+    lens = lens[:3] + [at_size - min(cut)] + lens[3:]
+    g = torch.Generator(device=gpu).manual_seed(sum(lens) + d)
+    nb = sum(-(-n // 16) for n in lens) + 3
+    perm = torch.randperm(nb, generator=torch.Generator().manual_seed(d)).tolist()
+    slots, tables, at = [], [], 0
+    for n in lens:
+        t = perm[at: at + -(-n // 16)]
+        at += len(t)
+        tables.append(t)
+        slots += [t[p // 16] * 16 + p % 16 for p in range(n)]
+    for i in (1, 20, 200):  # a skipped row, one outside the cache, two rows swapped
+        if i + 1 < len(slots):
+            if i == 1:
+                slots[i] = -1
+            elif i == 20:
+                slots[i] = nb * 16
+            else:
+                slots[i], slots[i + 1] = slots[i + 1], slots[i]
+    x = torch.randn(len(slots), h, d, generator=g, device=gpu).to(rows_dtype)
+    st = torch.tensor(slots, dtype=torch.int64, device=gpu)
+    fp8 = cache_dtype == torch.float8_e4m3fn
+    scale = torch.rand(h, generator=g, device=gpu) + 0.01 if fp8 else None
+    cache = torch.zeros(nb, h, d, 16, dtype=torch.uint8, device=gpu).view(cache_dtype) if fp8 else torch.zeros(
+        nb, h, d, 16, dtype=cache_dtype, device=gpu)
+    cache = cache.permute(0, 3, 1, 2)
+    ops.paged_write(x, st, cache, scale)
+    want = torch.zeros(nb * 16, h, d, dtype=torch.float32)
+    val = (x.float().cpu() / scale.cpu()[:, None] if fp8 else x.cpu()).to(cache_dtype).float()
+    st = st.cpu()
+    want[st[(st >= 0) & (st < nb * 16)]] = val[(st >= 0) & (st < nb * 16)]
+    raw = cache.float().cpu().reshape(nb * 16, h, d)
+    assert torch.equal(raw, want)
+    width = max(len(t) for t in tables)
+    tab = torch.tensor([t + [-1] * (width - len(t)) for t in tables], dtype=torch.int32, device=gpu)
+    for seq in (1, 17, min(width * 16 + 5, 3000)):
+        got = ops.paged_gather(cache, tab, seq, scale=scale).float().cpu()
+        for r, t in enumerate(tables):
+            full = torch.zeros(seq, h, d)
+            have = want.view(nb, 16, h, d)[torch.tensor(t)].reshape(-1, h, d)[:seq]
+            full[: have.shape[0]] = have * scale.cpu()[:, None] if fp8 else have
+            assert torch.equal(got[r], full), (seq, r)
