@@ -125,8 +125,7 @@ __device__ void plan_pass1(const DecodeParams& p, const Index& ix, const int32_t
     const int b = base + lane;
     const int len = b < p.B ? eff_len(p, ix, b) : 0;
     const int full = len >> 5;
-    int fprev = __shfl_up(full, 1, 64);
-    if (lane == 0) fprev = carry_full;
+    const int fprev = wave_prev(full, carry_full);
     int lcpt = 0;
     if (shared != nullptr && SG > 1 && b > 0 && b < p.B) {
       const int sh = shared[(int64_t)b * p.sh_s];
@@ -139,8 +138,8 @@ __device__ void plan_pass1(const DecodeParams& p, const Index& ix, const int32_t
       pl->j0[b] = lcpt;
       pl->psum[b] = hs + SG * ((b - hs) / SG);
     }
-    carry_full = __shfl(full, 63, 64);
-    carry_hs = __shfl(hs, 63, 64);
+    carry_full = wave_last(full);
+    carry_hs = wave_last(hs);
   }
 }
 
@@ -184,9 +183,43 @@ __device__ void plan_pass3(const DecodeParams& p, Plan* pl, int lane) {
       pl->j0[b] = j0;
       pl->psum[b] = incl - rt;
     }
-    carry = __shfl(incl, 63, 64);
+    carry = wave_last(incl);
   }
   if (lane == 0) pl->psum[p.B] = carry;
+}
+
+// The plan of a call without groups (no statement, or one sequence fills the
+// columns): lengths and the scan of the runs, one pass.
+__device__ void plan_plain(const DecodeParams& p, const Index& ix, Plan* pl, int lane) {
+  int carry = 0;
+  for (int base = 0; base < p.B; base += 64) {
+    const int b = base + lane;
+    const int len = b < p.B ? eff_len(p, ix, b) : 0;
+    const int rt = len > 0 ? kRunPad + ((len + 31) >> 5) : 0;
+    const int incl = wave_incl_scan(rt, lane) + carry;
+    if (b < p.B) {
+      pl->len[b] = len;
+      pl->j0[b] = 0;
+      pl->pre[b] = 0;
+      pl->psum[b] = incl - rt;
+    }
+    carry = wave_last(incl);
+  }
+  if (lane == 0) pl->psum[p.B] = carry;
+}
+
+// Orders a wave's LDS writes before its own later reads.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// a / b of non-negative stream slots (b > 0): 32-bit wherever they fit, which
+// is always but for streams of 2^32 tiles (the 64-bit division is 4x as long).
+__device__ __forceinline__ int64_t div_slots(int64_t a, int64_t b) {
+  if ((((uint64_t)a | (uint64_t)b) >> 32) == 0) return (int64_t)((uint32_t)a / (uint32_t)b);
+  return a / b;
 }
 
 // Largest b with psum[b] <= r (64-ary search; psum[0] = 0 <= r): the
@@ -454,8 +487,8 @@ __device__ __forceinline__ void flush_run(const DecodeParams& p, const Index& ix
       // w1..w2; w1 holds it in slot 1 when its range also holds the
       // previous run's last tile (slot s_tile - pad - 1), else in slot 0
       const int64_t s_tile = c.v - (c.j - c.first);
-      const int64_t w1 = s_tile / chunk;
-      const int64_t w2 = (s_tile + (c.last - c.first) - 1) / chunk;
+      const int64_t w1 = div_slots(s_tile, chunk);
+      const int64_t w2 = div_slots(s_tile + (c.last - c.first) - 1, chunk);
       d = make_int2((int)((w1 * 2 + (s_tile - pad - 1 >= w1 * chunk ? 1 : 0)) * kSlotCols), (int)(w2 - w1 + 1));
     }
     if (c.kind == kOwn) {
@@ -717,19 +750,28 @@ __global__ __launch_bounds__(256) void decode_stream_kernel(DecodeParams p, cons
   const int Wtot = gridDim.x * 4;
   const int w = uniform(stream_wave(blockIdx.x * 4 + wave, Wtot, p.Hkv));
 
+  // The plan, by wave 0; every cycle up to the first tile's loads is idle
+  // time of the whole launch (7,000 cycles with shuffle scans, block barriers
+  // between the passes, lengths read twice and 64-bit divisions).
   if constexpr (PL) {
-    if (wave == 0) plan_pass1(p, ix, shared, pl, lane);
-    __syncthreads();
-    if (wave == 0) plan_pass2(p, pl, lane);
-    __syncthreads();
-    if (wave == 0) plan_pass3(p, pl, lane);
+    if (wave == 0) {
+      if (shared == nullptr || p.G == kSlotCols) {
+        plan_plain(p, ix, pl, lane);
+      } else {
+        plan_pass1(p, ix, shared, pl, lane);
+        wave_lds_fence();
+        plan_pass2(p, pl, lane);
+        wave_lds_fence();
+        plan_pass3(p, pl, lane);
+      }
+    }
     __syncthreads();
   }
 
   // Sequences with no tokens get zero rows (no tile of theirs is ever
   // visited); wave w takes sequences w, w + Wtot, ...
   for (int bz = w; bz < p.B; bz += Wtot) {
-    if (eff_len(p, ix, bz) == 0) {
+    if (seqs.len(bz) == 0) {
       const int64_t orow = (int64_t)bz * p.o_sb;
       for (int e = lane; e < p.Hq * D; e += 64) store_out1<QT>(p.out, orow + (int64_t)(e / D) * p.o_sh + e % D, 0.0f);
       for (int hh = lane; hh < p.Hkv; hh += 64) {
@@ -743,15 +785,15 @@ __global__ __launch_bounds__(256) void decode_stream_kernel(DecodeParams p, cons
   else Tb = tiles_per_head(p, ix, lane);
   const int64_t T = (int64_t)p.Hkv * Tb;
   if (T == 0) return;
-  const int64_t chunk = (T + Wtot - 1) / Wtot;
+  const int64_t chunk = div_slots(T + Wtot - 1, Wtot);
   const int64_t v0 = (int64_t)w * chunk;  // this wave's stream slots [v0, v_end)
   if (v0 >= T) return;
   const int64_t v_end = v0 + chunk < T ? v0 + chunk : T;
 
   Coord c0;
-  c0.h = uniform((int)(v0 / Tb));
+  c0.h = uniform((int)div_slots(v0, Tb));
   {
-    const int r = uniform((int)(v0 % Tb));
+    const int r = uniform((int)(v0 - (int64_t)c0.h * Tb));
     if constexpr (PL) {
       // slot r: a run's padding (start at that run's first tile) or a tile
       const int b = plan_find(pl, p.B, r, lane);

@@ -352,23 +352,40 @@ __device__ __forceinline__ int wave_sum_i(int v) {
   return v;
 }
 
-__device__ __forceinline__ int wave_incl_scan(int v, int lane) {
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int u = __shfl_up(v, o, 64);
-    if (lane >= o) v += u;
-  }
+// Inclusive scans over the 64 lanes by DPP moves within and between the rows
+// of 16 (a shuffle goes through LDS and costs ten times as much): after the
+// row_shr steps each row holds its own scan, row_bcast:15 adds row 0's (2's)
+// last lane to row 1 (3), row_bcast:31 row 1's to rows 2 and 3.  Lanes without
+// a source take the identity.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_or(int identity, int v) {
+  return __builtin_amdgcn_update_dpp(identity, v, CTRL, ROWS, 0xF, false);
+}
+
+__device__ __forceinline__ int wave_incl_scan(int v, int) {
+  v += dpp_or<0x111, 0xF>(0, v);
+  v += dpp_or<0x112, 0xF>(0, v);
+  v += dpp_or<0x114, 0xF>(0, v);
+  v += dpp_or<0x118, 0xF>(0, v);
+  v += dpp_or<0x142, 0xA>(0, v);
+  v += dpp_or<0x143, 0xC>(0, v);
   return v;
 }
 
-__device__ __forceinline__ int wave_incl_max(int v, int lane) {
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int u = __shfl_up(v, o, 64);
-    if (lane >= o) v = max(v, u);
-  }
+__device__ __forceinline__ int wave_incl_max(int v, int) {
+  constexpr int kMin = -0x7FFFFFFF - 1;
+  v = max(v, dpp_or<0x111, 0xF>(kMin, v));
+  v = max(v, dpp_or<0x112, 0xF>(kMin, v));
+  v = max(v, dpp_or<0x114, 0xF>(kMin, v));
+  v = max(v, dpp_or<0x118, 0xF>(kMin, v));
+  v = max(v, dpp_or<0x142, 0xA>(kMin, v));
+  v = max(v, dpp_or<0x143, 0xC>(kMin, v));
   return v;
 }
+
+// Lane l's value from lane l - 1 (`first` on lane 0), and lane 63's.
+__device__ __forceinline__ int wave_prev(int v, int first) { return dpp_or<0x138, 0xF>(first, v); }
+__device__ __forceinline__ int wave_last(int v) { return __builtin_amdgcn_readlane(v, 63); }
 
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
