@@ -78,7 +78,7 @@ constexpr int kCostBins = 2048;   // tile counts at or above share the last bin
 constexpr int kXcds = 8;          // workgroup g runs on XCD g % 8, each with its own L2
 constexpr int kAffinePct = 75;    // share of the tiles taken from per-XCD lists
 constexpr int kPlanChunks = 1024; // chunk records the plan kernel keeps in LDS
-constexpr int kDirectItems = 512; // most items of a direct launch (one piece per workgroup)
+constexpr int kDirectItems = 768; // most items of a direct launch (one piece per workgroup)
 constexpr int kDirectCandidates = 16;
 constexpr int kMinPieceTiles = 6; // shortest piece an item is cut into: a piece costs its (m, l, o) record and the merge
 
@@ -156,7 +156,7 @@ __device__ __forceinline__ int block_tiles(const PrefillParams& p, const int4& c
 //
 // Measured, whole calls (e4m3, 32 query / 8 KV heads of 128): 100 rows behind
 // 12,001 cached tokens 354 us (32 workgroups walking 380 tiles each) -> 46 us;
-// a 1,237-row prompt (bf16, 32 / 4 heads of 64) 50.6 -> 36.2 us.  Above W items
+// a 1,237-row prompt (bf16, 32 / 4 heads of 64) 50.8 -> 34.3 us.  Above W items
 // the longest-first queue is within a few percent of even shares, and cutting
 // them only adds records and a merge launch (eight 512-row chunks behind
 // 0-4,096 tokens, cut in the queue's plan: 123 us against 114 us uncut).
@@ -1072,7 +1072,10 @@ int prefill_cus() {
   return n;
 }
 
-constexpr int kItemBlocksPerCU = 2;  // resident workgroups per CU (8 waves)
+// Resident workgroups per CU: 2 (8 waves).  A direct launch at head_dim 64 (141
+// VGPRs) fits 3: a 1,237-row prompt of 32 / 4 heads 34.9 us against 36.2 us
+// with 2.
+constexpr int item_blocks_per_cu(int64_t D, bool direct) { return direct && D == 64 ? 3 : 2; }
 constexpr int kMergeBlocks = 1024;
 
 template <int QT, int KT, int D, int G, bool VTOK, bool DIRECT>
@@ -1084,7 +1087,7 @@ int item_workers() {
             hipSuccess ||
         n < 1)
       n = 1;
-    per_cu = n < kItemBlocksPerCU ? n : kItemBlocksPerCU;
+    per_cu = std::min(n, item_blocks_per_cu(D, DIRECT));
   }
   return prefill_cus() * per_cu;
 }
@@ -1196,8 +1199,8 @@ int prefill_rows_per_item(int G) { return kCols / G; }
 
 // Slots for the pieces of a direct launch, one per resident workgroup; none
 // when the call may hold more items than that (queued launches cut nothing).
-int64_t split_slots_of(int64_t max_items) {
-  const int64_t w = std::min<int64_t>((int64_t)prefill_cus() * kItemBlocksPerCU, kDirectItems);
+int64_t split_slots_of(int64_t max_items, int64_t D) {
+  const int64_t w = std::min<int64_t>((int64_t)prefill_cus() * item_blocks_per_cu(D, true), kDirectItems);
   return max_items <= w ? w : 0;
 }
 
@@ -1208,14 +1211,14 @@ uint64_t prefill_workspace_bytes(int64_t Tq, int64_t N, int64_t Hq, int64_t Hkv,
   const int64_t G = Hkv > 0 ? Hq / Hkv : 1;
   const int64_t RB = std::max<int64_t>(G > 0 ? kCols / G : 1, 1);
   const int64_t max_items = (Tq / RB + N) * Hkv;
-  const uint64_t slots = (uint64_t)split_slots_of(max_items);
+  const uint64_t slots = (uint64_t)split_slots_of(max_items, D);
   const uint64_t base = pad256((uint64_t)N * 16) + pad256((uint64_t)max_items * 16) + 256;
   if (slots == 0) return base;
   return base + pad256((uint64_t)max_items * 32) + pad256(slots * kCols * 8) + slots * kCols * (uint64_t)D * 4;
 }
 
 void prefill_bind_workspace(PrefillParams& p, void* workspace) {
-  const uint64_t slots = (uint64_t)split_slots_of(p.max_items);
+  const uint64_t slots = (uint64_t)split_slots_of(p.max_items, p.D);
   p.split_slots = (int)slots;
   char* w = (char*)workspace;
   p.chunks = (int4*)w;

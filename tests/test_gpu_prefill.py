@@ -387,3 +387,31 @@ def test_items_cut_along_the_kv_range_match_oracle(gpu, chunks, cached, hq, hkv,
     ref, covered = oracle_prefill(case, t)
     assert covered.all()
     assert_close(out.float().cpu().numpy(), ref, torch.bfloat16, "cut prefill")
+
+
+@pytest.mark.parametrize("chunks,cached,hq,hkv,d,kv_dtype,layout", [
+    ([512] * 5, [0, 0, 16, 0, 3000], 32, 8, 128, torch.float8_e4m3fn, "paired"),   # 640 items: queued
+    ([700, 33, 1], [5000, 1, 900], 12, 12, 64, torch.bfloat16, "token_major"),     # 84 items: one piece per workgroup
+    ([1300, 33, 1300], [0, 6000, 2000], 32, 4, 64, torch.bfloat16, "native"),      # ragged row blocks beside cut ones
+])
+def test_chunks_of_a_call_equal_the_chunks_alone(gpu, chunks, cached, hq, hkv, d, kv_dtype, layout):
+    """Calls of more items than workgroups (queued, nothing is cut) and of
+    fewer: every chunk as in a call of its own (whose long items are cut), and
+    a sample of rows against the oracle."""
+    print(f"[case] queued and cut prefill {chunks} behind {cached} {hq}/{hkv}/{d} {kv_dtype} {layout}", flush=True)
+    case = workloads.make_mixed_case(device=gpu, seed=8, chunks=chunks, cached=cached, decode_lens=[],
+                                     num_q_heads=hq, num_kv_heads=hkv, head_dim=d, kv_dtype=kv_dtype)
+    t = workloads.materialize_mixed(case, layout)
+    _write_new_rows(case, t)
+    out = _prefill(case, t)
+    at = 0
+    for i, n in enumerate(chunks):
+        alone = _prefill(case, t, q=t["q_prefill"][at:at + n], tables=t["prefill_tables"][i:i + 1],
+                         lens=t["prefill_lens"][i:i + 1],
+                         q_start=torch.tensor([0, n], dtype=torch.int32, device=gpu))
+        assert_close(out[at:at + n].float().cpu().numpy(), alone.float().cpu().numpy(), torch.bfloat16, f"chunk {i}")
+        first = chunks[i] - min(chunks[i], 3)  # the last rows: the longest items
+        ref, _ = oracle_prefill(case, t, q=t["q_prefill"][at + first:at + n], tables=[case.prefill_tables[i]],
+                                lens=[case.prefill_lens[i]], q_start=[0, n - first])
+        assert_close(out[at + first:at + n].float().cpu().numpy(), ref, torch.bfloat16, f"chunk {i}, last rows")
+        at += n
