@@ -82,12 +82,17 @@ constexpr int kDirectItems = 768; // most items of a direct launch (one piece pe
 constexpr int kDirectCandidates = 16;
 constexpr int kMinPieceTiles = 6; // shortest piece an item is cut into: a piece costs its (m, l, o) record and the merge
 
-__device__ __forceinline__ float wave_incl_scanf(float v, int lane) {
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const float u = __shfl_up(v, o, 64);
-    if (lane >= o) v += u;
-  }
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_or_zero(float v) {
+  return __builtin_bit_cast(float, dpp_or<CTRL, ROWS>(0, __builtin_bit_cast(int, v)));
+}
+__device__ __forceinline__ float wave_incl_scanf(float v) {  // as wave_incl_scan
+  v += dpp_or_zero<0x111, 0xF>(v);
+  v += dpp_or_zero<0x112, 0xF>(v);
+  v += dpp_or_zero<0x114, 0xF>(v);
+  v += dpp_or_zero<0x118, 0xF>(v);
+  v += dpp_or_zero<0x142, 0xA>(v);
+  v += dpp_or_zero<0x143, 0xC>(v);
   return v;
 }
 
@@ -155,17 +160,19 @@ __device__ __forceinline__ int block_tiles(const PrefillParams& p, const int4& c
 // read its K/V through one XCD's L2), and so is its workspace slot.
 //
 // Measured, whole calls (e4m3, 32 query / 8 KV heads of 128): 100 rows behind
-// 12,001 cached tokens 354 us (32 workgroups walking 380 tiles each) -> 46 us;
-// a 1,237-row prompt (bf16, 32 / 4 heads of 64) 50.8 -> 34.3 us.  Above W items
+// 12,001 cached tokens 354 us (32 workgroups walking 380 tiles each) -> 44 us;
+// a 1,237-row prompt (bf16, 32 / 4 heads of 64) 50.6 -> 33.1 us.  Above W items
 // the longest-first queue is within a few percent of even shares, and cutting
 // them only adds records and a merge launch (eight 512-row chunks behind
 // 0-4,096 tokens, cut in the queue's plan: 123 us against 114 us uncut).
 struct DirectPlan {
   int4 chunks[kDirectItems];
   int tiles[kDirectItems];
-  int red[3][4];
+  int nblocks;
   float sum[4];
+  int most[4];
   int pieces[kDirectCandidates];
+  int scan[4];
 };
 struct DirectPiece {
   int4 chunk;
@@ -178,17 +185,21 @@ __device__ __forceinline__ int piece_count(int t, int P) {
   return max(1, (int)ceilf((float)t / (float)P));
 }
 
+// Every cycle here is idle time of the launch: DPP scans, one LDS read for all
+// candidates and three block barriers take 6,300 cycles (half of them the
+// chunk table's loads), where shuffles and a loop over the candidates took
+// 10,100.
 __device__ bool direct_piece(const PrefillParams& p, DirectPlan* s, DirectPiece* out, int tid) {
   const int lane = tid & 63, wave = uniform(tid >> 6);
   if (wave == 0) {
     const int nrb = chunk_rows(p, lane, [&](int n, const int4& c) { s->chunks[n] = c; });
-    if (lane == 0) s->red[0][0] = nrb;
+    if (lane == 0) {
+      s->nblocks = nrb;
+      out->n = -1;
+    }
   }
-  if (tid < kDirectCandidates) s->pieces[tid] = 0;
-  if (tid == 0) out->n = -1;
   __syncthreads();
-  const int nblocks = s->red[0][0];
-  __syncthreads();
+  const int nblocks = uniform(s->nblocks);
   auto chunk_at = [&](int n) { return s->chunks[n]; };
   float sum = 0.0f;
   int most = 0;
@@ -198,31 +209,42 @@ __device__ bool direct_piece(const PrefillParams& p, DirectPlan* s, DirectPiece*
     sum += (float)t;
     most = max(most, t);
   }
-  sum = wave_sum(sum);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o, 64));
-  if (lane == 0) {
+  sum = wave_incl_scanf(sum);
+  most = wave_incl_max(most, lane);
+  if (lane == 63) {
     s->sum[wave] = sum;
-    s->red[1][wave] = most;
+    s->most[wave] = most;
   }
   __syncthreads();
-  most = max(max(s->red[1][0], s->red[1][1]), max(s->red[1][2], s->red[1][3]));
+  most = max(max(s->most[0], s->most[1]), max(s->most[2], s->most[3]));
   const float share = (s->sum[0] + s->sum[1] + s->sum[2] + s->sum[3]) * (float)p.Hkv / (float)p.workers;
   auto candidate = [&](int k) {
     return max(kMinPieceTiles, (int)fminf(ceilf(share * (1.0f + 0.125f * k)), 16777216.0f));
   };
   int P = 1 << 24;
   if (most > candidate(0)) {  // uniform
-    for (int k = wave; k < kDirectCandidates; k += 4) {
-      const int Pk = candidate(k);
-      int n = 0;
-      for (int f = lane; f < nblocks; f += 64) n += piece_count(s->tiles[f], Pk);
-      n = wave_sum_i(n);
-      if (lane == 0) s->pieces[k] = n;
+    // wave w counts the pieces of candidates w, w + 4, ...
+    constexpr int kPer = kDirectCandidates / 4;
+    int Pk[kPer], n[kPer];
+#pragma unroll
+    for (int c = 0; c < kPer; ++c) {
+      Pk[c] = candidate(wave + 4 * c);
+      n[c] = 0;
+    }
+    for (int f = lane; f < nblocks; f += 64) {
+      const int t = s->tiles[f];
+#pragma unroll
+      for (int c = 0; c < kPer; ++c) n[c] += piece_count(t, Pk[c]);
+    }
+#pragma unroll
+    for (int c = 0; c < kPer; ++c) {
+      n[c] = wave_incl_scan(n[c], lane);
+      if (lane == 63) s->pieces[wave + 4 * c] = n[c];
     }
     __syncthreads();
-    for (int k = kDirectCandidates - 1; k >= 0; --k)
-      if (s->pieces[k] * p.Hkv <= p.workers) P = candidate(k);
+    const bool fits = lane < kDirectCandidates && s->pieces[lane & (kDirectCandidates - 1)] * p.Hkv <= p.workers;
+    const unsigned long long ok = __ballot(fits);
+    if (ok != 0) P = candidate(__builtin_ctzll(ok));
   }
   // this workgroup's piece: an exclusive scan of the row blocks' piece counts
   const int want = (int)blockIdx.x / p.Hkv;
@@ -231,12 +253,14 @@ __device__ bool direct_piece(const PrefillParams& p, DirectPlan* s, DirectPiece*
     const int f = f0 + tid;
     const int n = f < nblocks ? piece_count(s->tiles[f], P) : 0;
     const int incl = wave_incl_scan(n, lane);
-    if (lane == 63) s->red[2][wave] = incl;
+    if (lane == 63) s->scan[wave] = incl;
     __syncthreads();
     int before = carry;
+#pragma unroll
     for (int w = 0; w < 4; ++w) {
-      if (w < wave) before += s->red[2][w];
-      carry += s->red[2][w];
+      const int c = s->scan[w];
+      if (w < wave) before += c;
+      carry += c;
     }
     const int at = before + incl - n;  // first piece of f
     if (want >= at && want < at + n) {
@@ -304,7 +328,7 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PrefillParam
   const int h0 = hist[2 * tid], h1 = hist[2 * tid + 1];
   const float t0 = (float)h0 * (float)(kCostBins - 1 - 2 * tid), t1 = (float)h1 * (float)(kCostBins - 2 - 2 * tid);
   const int incl = wave_incl_scan(h0 + h1, lane);
-  const float tincl = wave_incl_scanf(t0 + t1, lane);
+  const float tincl = wave_incl_scanf(t0 + t1);
   if (lane == 63) {
     wave_tot[wave] = incl;
     wave_tiles[wave] = tincl;
