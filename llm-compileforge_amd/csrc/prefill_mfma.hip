@@ -80,7 +80,9 @@ constexpr int kAffinePct = 75;    // share of the tiles taken from per-XCD lists
 constexpr int kPlanChunks = 1024; // chunk records the plan kernel keeps in LDS
 constexpr int kDirectItems = 768; // most items of a direct launch (one piece per workgroup)
 constexpr int kDirectCandidates = 16;
-constexpr int kMinPieceTiles = 6; // shortest piece an item is cut into: a piece costs its (m, l, o) record and the merge
+constexpr int kMinPieceTiles = 6; // shortest piece an item is cut into
+constexpr int kCutTiles = 6;      // the merge launch, in tiles of about 1 us
+constexpr float kPieceTiles = 0.025f;  // a piece's record at head_dim 128 (64 KiB written and read), in tiles
 
 template <int CTRL, int ROWS>
 __device__ __forceinline__ float dpp_or_zero(float v) {
@@ -153,8 +155,17 @@ __device__ __forceinline__ int block_tiles(const PrefillParams& p, const int4& c
 // single prompts) need no queue: each workgroup works out its own piece from
 // the chunk table, and there is no plan launch.  With T tiles in all, a
 // workgroup's share is T / W; items longer than P tiles are cut along the KV
-// range into equal pieces, P the shortest of share * (1 + k / 8), at least
-// kMinPieceTiles, for which all pieces fit the W workgroups at once.  Piece
+// range into equal pieces, all of which fit the W workgroups at once.  P is
+// the cheapest of max(share, kMinPieceTiles) * (1 + k / 8) by the launch's
+// length in tiles: P, plus kCutTiles for the merge launch, plus kPieceTiles a
+// piece for its record written and read (at head_dim 128); nothing is cut
+// where the longest item is shorter than that.  Measured against always
+// cutting at max(share, 6) * (1 + k / 8), the first that fits: 256 rows of
+// 32 / 8 heads 16.8 -> 13.3 us, 400 rows of 64 / 8 heads 23.4 -> 20.8 us, two
+// chunks of 128 behind 256 22.8 -> 17.2 us, 100 rows behind 3,000 29.0 -> 28.1 us;
+// no shorter than 10 or 24 tiles would cost 40 rows behind 500 (12 heads of
+// 64) 13.3 -> 15.2 and 16.9 us.  512 rows of 32 / 8 heads lose 0.7 us.
+// Piece
 // number i of row block f for head h is workgroup (first piece of f + i) *
 // Hkv + h (heads fastest, so with Hkv a multiple of 8 the pieces of a head
 // read its K/V through one XCD's L2), and so is its workspace slot.
@@ -171,7 +182,7 @@ struct DirectPlan {
   int nblocks;
   float sum[4];
   int most[4];
-  int pieces[kDirectCandidates];
+  int2 pieces[kDirectCandidates];  // {all pieces, pieces of cut items}
   int scan[4];
 };
 struct DirectPiece {
@@ -185,10 +196,9 @@ __device__ __forceinline__ int piece_count(int t, int P) {
   return max(1, (int)ceilf((float)t / (float)P));
 }
 
-// Every cycle here is idle time of the launch: DPP scans, one LDS read for all
-// candidates and three block barriers take 6,300 cycles (half of them the
-// chunk table's loads), where shuffles and a loop over the candidates took
-// 10,100.
+// Every cycle here is idle time of the launch: with DPP scans and one LDS read
+// for all candidates it takes 6,300 cycles, where shuffles, a loop over the
+// candidates and more block barriers took 10,100.
 __device__ bool direct_piece(const PrefillParams& p, DirectPlan* s, DirectPiece* out, int tid) {
   const int lane = tid & 63, wave = uniform(tid >> 6);
   if (wave == 0) {
@@ -219,32 +229,45 @@ __device__ bool direct_piece(const PrefillParams& p, DirectPlan* s, DirectPiece*
   most = max(max(s->most[0], s->most[1]), max(s->most[2], s->most[3]));
   const float share = (s->sum[0] + s->sum[1] + s->sum[2] + s->sum[3]) * (float)p.Hkv / (float)p.workers;
   auto candidate = [&](int k) {
-    return max(kMinPieceTiles, (int)fminf(ceilf(share * (1.0f + 0.125f * k)), 16777216.0f));
+    return (int)fminf(ceilf(fmaxf(share, (float)kMinPieceTiles) * (1.0f + 0.125f * k)), 16777216.0f);
   };
   int P = 1 << 24;
-  if (most > candidate(0)) {  // uniform
-    // wave w counts the pieces of candidates w, w + 4, ...
+  if (most > candidate(0) + kCutTiles) {  // uniform
+    // wave w counts the pieces, and those of cut items, of candidates w, w + 4, ...
     constexpr int kPer = kDirectCandidates / 4;
-    int Pk[kPer], n[kPer];
+    int Pk[kPer], n[kPer], cut[kPer];
 #pragma unroll
     for (int c = 0; c < kPer; ++c) {
       Pk[c] = candidate(wave + 4 * c);
-      n[c] = 0;
+      n[c] = cut[c] = 0;
     }
     for (int f = lane; f < nblocks; f += 64) {
       const int t = s->tiles[f];
 #pragma unroll
-      for (int c = 0; c < kPer; ++c) n[c] += piece_count(t, Pk[c]);
+      for (int c = 0; c < kPer; ++c) {
+        const int k = piece_count(t, Pk[c]);
+        n[c] += k;
+        cut[c] += k > 1 ? k : 0;
+      }
     }
 #pragma unroll
     for (int c = 0; c < kPer; ++c) {
       n[c] = wave_incl_scan(n[c], lane);
-      if (lane == 63) s->pieces[wave + 4 * c] = n[c];
+      cut[c] = wave_incl_scan(cut[c], lane);
+      if (lane == 63) s->pieces[wave + 4 * c] = make_int2(n[c], cut[c]);
     }
     __syncthreads();
-    const bool fits = lane < kDirectCandidates && s->pieces[lane & (kDirectCandidates - 1)] * p.Hkv <= p.workers;
-    const unsigned long long ok = __ballot(fits);
-    if (ok != 0) P = candidate(__builtin_ctzll(ok));
+    // lane k: candidate k's cost in tiles (as bits: positive floats order as ints)
+    const int2 pc = s->pieces[lane & (kDirectCandidates - 1)];
+    const float cost = (float)(candidate(lane & (kDirectCandidates - 1)) + kCutTiles) +
+                       kPieceTiles * ((float)p.D / 128.0f) * (float)pc.y * (float)p.Hkv;
+    const int key = pc.x * p.Hkv <= p.workers ? __builtin_bit_cast(int, cost) : 0x7F800000;
+    int best = min(key, dpp_or<0x111, 0xF>(0x7F800000, key));
+    best = min(best, dpp_or<0x112, 0xF>(0x7F800000, best));
+    best = min(best, dpp_or<0x114, 0xF>(0x7F800000, best));
+    best = min(best, dpp_or<0x118, 0xF>(0x7F800000, best));
+    best = __builtin_amdgcn_readlane(best, kDirectCandidates - 1);  // of the first row of 16 lanes
+    if (__builtin_bit_cast(float, best) < (float)most) P = candidate(__builtin_ctzll(__ballot(key == best)));
   }
   // this workgroup's piece: an exclusive scan of the row blocks' piece counts
   const int want = (int)blockIdx.x / p.Hkv;
@@ -1121,8 +1144,10 @@ int item_workers() {
 template <int QT, int KT, int D, int G, bool VTOK>
 int32_t launch_direct(PrefillParams& p, hipStream_t stream) {
   // no item is longer than the tables' capacity, so short tables bound the
-  // pieces, and where one piece holds any item there is nothing to merge
-  const int64_t most = std::max<int64_t>(ceil_div((int64_t)p.Mb * 16, 32 * kMinPieceTiles), 1);
+  // pieces, and where no item is long enough for a cut there is nothing to merge
+  // (an empty merge launch is 2 us: 256 rows, 8 heads of 128, 15.2 -> 13.3 us)
+  const int64_t tiles = ceil_div((int64_t)p.Mb * 16, 32);
+  const int64_t most = tiles > kMinPieceTiles + kCutTiles ? ceil_div(tiles, kMinPieceTiles) : 1;
   if (most == 1) p.splits = nullptr;
   {
     ProfileScope prof("cf_prefill_mfma", stream);

@@ -365,8 +365,11 @@ def test_rejects_unsupported(gpu):
 
 @pytest.mark.parametrize("chunks,cached", [
     ([33], [3967]),            # one row past a row block, a table that ends inside a block
-    ([1], [191]),              # 6 tiles: the longest item that is never cut
+    ([1], [191]),              # 6 tiles: the shortest piece
     ([1, 5], [192, 2000]),     # 7 tiles beside a longer item
+    ([1], [383]),              # 12 tiles: the longest item that is never cut
+    ([1], [384]),              # 13 tiles: the shortest that may be cut
+    ([65, 3], [319, 511]),     # cut and whole items in one launch
     ([100, 7, 16], [3001, 0, 700]),  # cut, whole and one-tile items in one call
 ])
 @pytest.mark.parametrize("hq,hkv,d,kv_dtype,layout", [
