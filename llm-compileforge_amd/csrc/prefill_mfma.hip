@@ -165,14 +165,14 @@ __device__ __forceinline__ int block_tiles(const PrefillParams& p, const int4& c
 // chunks of 128 behind 256 22.8 -> 17.2 us, 100 rows behind 3,000 29.0 -> 28.1 us;
 // no shorter than 10 or 24 tiles would cost 40 rows behind 500 (12 heads of
 // 64) 13.3 -> 15.2 and 16.9 us.  512 rows of 32 / 8 heads lose 0.7 us.
-// Piece
-// number i of row block f for head h is workgroup (first piece of f + i) *
+//
+// Piece number i of row block f for head h is workgroup (first piece of f + i) *
 // Hkv + h (heads fastest, so with Hkv a multiple of 8 the pieces of a head
 // read its K/V through one XCD's L2), and so is its workspace slot.
 //
 // Measured, whole calls (e4m3, 32 query / 8 KV heads of 128): 100 rows behind
 // 12,001 cached tokens 354 us (32 workgroups walking 380 tiles each) -> 44 us;
-// a 1,237-row prompt (bf16, 32 / 4 heads of 64) 50.6 -> 33.1 us.  Above W items
+// a 1,237-row prompt (bf16, 32 / 4 heads of 64) 50.6 -> 32.9 us.  Above W items
 // the longest-first queue is within a few percent of even shares, and cutting
 // them only adds records and a merge launch (eight 512-row chunks behind
 // 0-4,096 tokens, cut in the queue's plan: 123 us against 114 us uncut).
