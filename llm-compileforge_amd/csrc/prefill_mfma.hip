@@ -1035,6 +1035,10 @@ __global__ __launch_bounds__(256, 2) void prefill_item_kernel(PrefillParams p, c
 // the pieces were written in (1 KiB runs).  It is bound by one round trip and
 // the 64 * D bytes a piece's group holds: (m, l) and o are read side by side,
 // kMergeBatch pieces at a time.
+//
+// A piece whose column saw no finite score has m = -inf and weight 1: its l
+// and o are exact zeros where everything was masked, and NaN where a score or
+// a V value was, which the output then is too, as that of an uncut item.
 constexpr int kMergeBatch = 4;
 
 template <int QT, int D, int G>
@@ -1083,9 +1087,8 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p, con
       }
 #pragma unroll
       for (int b = 0; b < kMergeBatch; ++b) {
-        const bool use = i0 + b < n && mlv[b].x != -INFINITY;
-        const float w = use ? __builtin_amdgcn_exp2f(mlv[b].x - mnew) : 0.0f;
-        if (use) {
+        const float w = mlv[b].x == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(mlv[b].x - mnew);
+        if (i0 + b < n) {
           L += w * mlv[b].y;
 #pragma unroll
           for (int t = 0; t < TPW; ++t) {

@@ -15,6 +15,7 @@ import numpy as np
 import pytest
 import torch
 
+from cf_hip import layout as L
 from cf_hip import ops, workloads
 from kernels.paged_attention import chunked_prefill_attention, paged_attention_tensors
 from oracle import fp8 as ofp8
@@ -418,3 +419,78 @@ def test_chunks_of_a_call_equal_the_chunks_alone(gpu, chunks, cached, hq, hkv, d
                                 lens=[case.prefill_lens[i]], q_start=[0, n - first])
         assert_close(out[at + first:at + n].float().cpu().numpy(), ref, torch.bfloat16, f"chunk {i}, last rows")
         at += n
+
+
+def _cut_call(gpu, q_dtype, kv_dtype, hq, hkv, d, cached, rows, seed=1):
+    """One chunk of a few rows behind a long prefix, in a native cache: its
+    items are cut into pieces.  (q, k, v, ks, vs, tables, lens, q_start)."""
+    g = torch.Generator(device=gpu).manual_seed(seed)
+    n = cached + rows
+    nb = (n + 15) // 16
+    k, v = (torch.randn(nb, 16, hkv, d, generator=g, device=gpu).to(torch.bfloat16) for _ in range(2))
+    kc, vc = L.alloc_kv_cache(nb, 16, hkv, d, kv_dtype, gpu, "native")
+    ks = vs = None
+    if kv_dtype == torch.float8_e4m3fn:
+        ks, vs = ops.fp8_amax_scale(k), ops.fp8_amax_scale(v)
+        ops.fp8_quantize_kv(k, v, ks, vs, kc, vc)
+    else:
+        kc.copy_(k)
+        vc.copy_(v)
+    q = torch.randn(rows, hq, d, generator=g, device=gpu).to(q_dtype)
+    return (q, kc, vc, ks, vs, torch.arange(nb, dtype=torch.int32, device=gpu).view(1, nb),
+            torch.tensor([n], dtype=torch.int32, device=gpu), torch.tensor([0, rows], dtype=torch.int32, device=gpu))
+
+
+@pytest.mark.parametrize("q_dtype,kv_dtype", [
+    (torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float8_e4m3fn), (torch.float16, torch.float16),
+    (torch.float16, torch.float8_e4m3fn)])
+@pytest.mark.parametrize("where", ["query row", "keys of whole pieces", "every key", "one key", "one value", "scale"])
+def test_nan_reaches_the_output_of_a_cut_item(gpu, q_dtype, kv_dtype, where):
+    """A NaN among what a (row, head) sees makes its output NaN although the
+    item was cut, also where a piece saw nothing else; the other rows and heads
+    are those of the call without it, bit for bit."""
+    hq, hkv, d, cached, rows = 32, 8, 128, 4000, 40
+    if where == "scale" and kv_dtype != torch.float8_e4m3fn:
+        pytest.skip("no scale")
+    q, kc, vc, ks, vs, tables, lens, q_start = _cut_call(gpu, q_dtype, kv_dtype, hq, hkv, d, cached, rows)
+
+    def run():
+        with ops.KernelTimer() as timer:
+            out = chunked_prefill_attention(q, kc, vc, tables, lens, q_start, k_scale=ks, v_scale=vs)
+            torch.cuda.synchronize()
+            assert timer.query("cf_prefill_merge")[1] == 1  # cut
+        return out
+
+    clean = run()
+    assert torch.isfinite(clean).all()
+    want = torch.zeros(rows, hq, dtype=torch.bool, device=gpu)
+    nan = float("nan")
+
+    def put(cache, blocks, head):
+        if cache.dtype == torch.float8_e4m3fn:
+            cache.view(torch.uint8)[blocks, :, head] = 0x7F
+        else:
+            cache[blocks, :, head] = nan
+
+    if where == "query row":
+        q[3] = nan
+        want[3] = True
+    elif where == "keys of whole pieces":
+        put(kc, slice(0, 150), 2)  # 2,400 of 4,040 tokens: the rest is finite
+        want[:, 8:12] = True
+    elif where == "every key":
+        put(kc, slice(None), 2)
+        want[:, 8:12] = True
+    elif where == "one key":
+        put(kc[:, 5:6], slice(7, 8), 2)
+        want[:, 8:12] = True
+    elif where == "one value":
+        put(vc[:, 5:6], slice(7, 8), 2)
+        want[:, 8:12] = True
+    else:
+        ks[2] = nan
+        want[:, 8:12] = True
+    out = run()
+    got = out.isnan().all(-1)
+    assert torch.equal(got, want), (int(got.sum()), int(want.sum()))
+    assert torch.equal(out[~want], clean[~want])
