@@ -510,7 +510,8 @@ __device__ __forceinline__ void flush_run(const DecodeParams& p, const Index& ix
   if (direct && QT == kF32) {
     // one rounding per output: divide, rather than multiply by 1 / l
     const int64_t orow = (int64_t)c.b * p.o_sb + (int64_t)(c.h * G + li) * p.o_sh;
-    auto nrm = [&](float a) { return lt > 0.0f ? a * vs / lt : 0.0f; };
+    // (lt NaN: so is a, and a * 0 stays NaN)
+    auto nrm = [&](float a) { return lt > 0.0f ? a * vs / lt : a * 0.0f; };
 #pragma unroll
     for (int t = 0; t < NV; ++t)
       store_out4<QT>(p.out, orow + o_chan<QUAD>(t, lq), nrm(o_elem<QUAD>(o, t, 0)), nrm(o_elem<QUAD>(o, t, 1)),
@@ -675,14 +676,16 @@ __device__ __forceinline__ void stream_f32(const DecodeParams& p, const Index& i
       for (int t = 0; t < NV; ++t) o[t] = o[t] * alpha;
       m = mnew;
     }
-    const bool live = m != -INFINITY;
+    // a column with no finite score yet has m = -inf: any finite reference
+    // gives 0 for its masked tokens and keeps the NaN of others
+    const float mref = m == -INFINITY ? 0.0f : m;
     float pr[8];
     float psum = 0.0f;
 #pragma unroll
     for (int v = 0; v < 8; ++v) {
       const float raw = s[v >> 2][v & 3];
-      const float ex = __builtin_fmaf(raw, qk_scale, __builtin_fmaf(raw, qk_lo, -m));
-      pr[v] = live && sc[v] != -INFINITY ? __builtin_amdgcn_exp2f(ex) : 0.0f;
+      const float ex = __builtin_fmaf(raw, qk_scale, __builtin_fmaf(raw, qk_lo, -mref));
+      pr[v] = sc[v] != -INFINITY ? __builtin_amdgcn_exp2f(ex) : 0.0f;
     }
     psum = ((pr[0] + pr[1]) + (pr[2] + pr[3])) + ((pr[4] + pr[5]) + (pr[6] + pr[7]));
     l += psum;
@@ -1048,6 +1051,13 @@ __device__ __forceinline__ int64_t part_row(int2 d, int k) {
   return (int64_t)(2 * (w1 + k)) * kSlotCols + col;
 }
 
+// Weight of a partial with reference m under the maximum M (log2 units).  A
+// partial without a finite score (m = -inf) has l = o = 0, or NaN where a score
+// or a V value was, which the output then is too: weight 1 keeps both.
+__device__ __forceinline__ float merge_weight(float m, float M) {
+  return m == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - M);
+}
+
 // Combines the (m, l, o) partials of each (sequence b, KV head h) that the
 // decode kernel did not write whole: its own run's and its group's prefix
 // run's, each a record or the wave slots of a split run.  NSL workgroups per
@@ -1101,7 +1111,7 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeParams p) {
 #pragma unroll
       for (int k = 0; k < KMAX; ++k) {
         if (k < nsrc) {
-          const float w = mk[k][g] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mk[k][g] - Mg[g]);
+          const float w = merge_weight(mk[k][g], Mg[g]);
           mk[k][g] = w;  // now the weight
           Lg[g] += w * lk[k][g];
         }
@@ -1127,7 +1137,7 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeParams p) {
           a += w * ov[k][i];
         }
       }
-      store_out1<QT>(p.out, out + (int64_t)(h * G + g) * p.o_sh + d, lg > 0.0f ? a / lg : 0.0f);
+      store_out1<QT>(p.out, out + (int64_t)(h * G + g) * p.o_sh + d, lg > 0.0f ? a / lg : a * 0.0f);
     }
     return;
   }
@@ -1187,7 +1197,7 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeParams p) {
       float ls = 0.0f;
       for (int k = lane; k < n; k += 64) {
         const float mk = sm[g][k];
-        const float w = mk == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mk - mnew);
+        const float w = merge_weight(mk, mnew);
         sm[g][k] = w;
         ls += w * sl[g][k];
       }
@@ -1254,7 +1264,7 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeParams p) {
   for (int j = 0; j < FPT; ++j) {
     const int g = gs[j], d = 4 * fs[j] % D;
     const float lg = run_l[g];
-    auto nrm = [&](float a) { return lg > 0.0f ? a / lg : 0.0f; };
+    auto nrm = [&](float a) { return lg > 0.0f ? a / lg : a * 0.0f; };
     store_out4<QT>(p.out, out + (int64_t)(h * G + g) * p.o_sh + d, nrm(acc[j].x), nrm(acc[j].y), nrm(acc[j].z),
                    nrm(acc[j].w));
   }

@@ -754,3 +754,43 @@ def test_full_c3_token_major(gpu):
                                [case.seq_lens[i] for i in idx], 16, case.scale, case.kv_dtype)
     ref = oracle_decode(sub, kt, vt, ks, vs)
     assert_close(out_t[idx].float().cpu().numpy(), ref, torch.bfloat16, "c3 token-major")
+
+
+@pytest.mark.parametrize("kv_dtype", [torch.float32, torch.bfloat16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("hq,hkv,d", [(32, 8, 128), (12, 12, 64)])
+@pytest.mark.parametrize("layout", ["native", "token_major"])
+@pytest.mark.parametrize("lens", [[700] * 64, [64, 40, 5000]], ids=["whole runs", "split runs"])
+def test_nan_reaches_the_output_under_fp32_queries(gpu, kv_dtype, hq, hkv, d, layout, lens):
+    """One NaN key among many finite ones makes its KV head's outputs NaN,
+    whether its run is written whole or merged; over fp32 caches also where a
+    wave, or the whole sequence, saw nothing else.  Other heads and sequences
+    are those of the call without it, bit for bit."""
+    g = torch.Generator(device=gpu).manual_seed(d)
+    blocks = [-(-n // 16) for n in lens]
+    nb = sum(blocks)
+    tables, at = [], 0
+    for n in blocks:
+        tables.append(list(range(at, at + n)))
+        at += n
+    q = torch.randn(len(lens), hq, d, generator=g, device=gpu)
+    k, v = (torch.randn(nb, 16, hkv, d, generator=g, device=gpu) for _ in range(2))
+    case = workloads.DecodeCase("nan", q, k, v, tables, lens, 16, 1 / math.sqrt(d), kv_dtype)
+    kc, vc, ks, vs = workloads.materialize(case, layout)
+    clean = _run(case, kc, vc, ks, vs, gpu)
+    assert torch.isfinite(clean).all()
+    bits = kc.view(torch.uint8) if kv_dtype == torch.float8_e4m3fn else kc
+    last, head, grp = len(lens) - 1, hkv - 1, hq // hkv
+    sequences = {last: [(2, 5)]}
+    if kv_dtype == torch.float32:
+        sequences = {last: [(j, slice(None)) for j in range(4)], 0: [(j, slice(None)) for j in range(blocks[0])]}
+    want = torch.zeros(len(lens), hq, dtype=torch.bool, device=gpu)
+    for b, cells in sequences.items():
+        for j, tok in cells:
+            bits[tables[b][j], tok, head] = 0x7F if kv_dtype == torch.float8_e4m3fn else float("nan")
+        want[b, head * grp:] = True
+    out = _run(case, kc, vc, ks, vs, gpu)
+    assert torch.equal(out.isnan().all(-1), want)
+    assert torch.equal(out[~want], clean[~want])
+    if kv_dtype == torch.float32:
+        case.q[1, 0] = float("nan")
+        assert _run(case, kc, vc, ks, vs, gpu)[1, 0].isnan().all()
