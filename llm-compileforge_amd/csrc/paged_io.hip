@@ -108,11 +108,14 @@ __device__ __forceinline__ int64_t slot_of(const PagedWriteParams& p, int64_t i)
   return ST == kI64 ? ((const int64_t*)p.slots)[i * p.slot_s] : (int64_t)((const int32_t*)p.slots)[i * p.slot_s];
 }
 
+// Workgroups of a launch in a grid of grid_of(): x first, then y.
+__device__ __forceinline__ int64_t block_index() { return (int64_t)blockIdx.y * gridDim.x + blockIdx.x; }
+
 // One thread per piece of N channels (N == 1: any strides).
 template <int XT, int ST, int CT, int N>
 __global__ __launch_bounds__(256) void paged_write_kernel(PagedWriteParams p) {
   const int np = p.D / N;
-  const int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t u = block_index() * 256 + threadIdx.x;
   const int64_t total = p.T * p.H * np;
   if (u >= total) return;
   int64_t i;
@@ -149,8 +152,9 @@ template <int XT, int ST, int CT>
 __global__ __launch_bounds__(256) void paged_write_tile_kernel(PagedWriteParams p, uint32_t chunks) {
   using X = typename Elem<XT>::T;
   using C = typename Elem<CT>::T;
-  const uint32_t g = blockIdx.x / chunks;
-  const int hd = (int)(blockIdx.x - g * chunks) * 256 + (int)threadIdx.x;
+  const uint32_t block = (uint32_t)block_index(), g = block / chunks;
+  if ((int64_t)g * 16 >= p.T) return;  // past the last group
+  const int hd = (int)(block - g * chunks) * 256 + (int)threadIdx.x;
   const bool mine = hd < p.H * p.D;
   const int h = mine ? hd / p.D : 0, d = mine ? hd % p.D : 0;
   // lane l: the slot of row g * 16 - 1 + l (-1 outside [0, T))
@@ -211,7 +215,7 @@ __global__ __launch_bounds__(256) void paged_write_tile_kernel(PagedWriteParams 
 template <int CT, int OT, int N>
 __global__ __launch_bounds__(256) void paged_gather_kernel(PagedGatherParams p) {
   const int np = p.D / N;
-  const int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t u = block_index() * 256 + threadIdx.x;
   const int64_t total = (int64_t)p.R * p.S * p.H * np;
   if (u >= total) return;
   int c, h, s, r;
@@ -260,7 +264,7 @@ __global__ __launch_bounds__(256) void paged_gather_tile_kernel(PagedGatherParam
   using C = typename Elem<CT>::T;
   using O = typename Elem<OT>::T;
   const uint32_t per = (uint32_t)(p.H * p.D / P);
-  const int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t u = block_index() * 256 + threadIdx.x;
   const int64_t total = (int64_t)p.R * blocks_per_row * per;
   if (u >= total) return;
   int64_t rb;
@@ -326,7 +330,13 @@ bool channel_tiles(const void* base, const int64_t* c_s, int bs, int eb) {
          (c_s[2] * eb) % 16 == 0;
 }
 
-int64_t grid_of(int64_t threads) { return (threads + 255) / 256; }
+// Workgroups of 256 threads for `threads`, and the grid that holds them: a
+// dimension of 2^32 threads or more is launched modulo 2^32, without an error.
+int64_t blocks_of(int64_t threads) { return (threads + 255) / 256; }
+dim3 grid_of(int64_t blocks) {
+  const int64_t rows = ceil_div(blocks, (int64_t)1 << 23);
+  return dim3((unsigned)ceil_div(blocks, rows), (unsigned)rows);
+}
 
 // Values (rows x channels) from which the channel-major write goes by whole
 // blocks.  A thread there walks 16 rows, which takes 5.4 us however few they
@@ -340,9 +350,9 @@ template <int XT, int ST, int CT>
 int32_t launch_write_t(const PagedWriteParams& p, hipStream_t stream) {
   ProfileScope prof("cf_paged_write", stream);
   if (p.T * p.H * p.D >= kTileWriteValues && channel_tiles(p.cache, p.c_s, p.bs, esize<CT>())) {
-    const int64_t chunks = grid_of((int64_t)p.H * p.D), blocks = ceil_div(p.T, 16) * chunks;
+    const int64_t chunks = blocks_of((int64_t)p.H * p.D), blocks = ceil_div(p.T, 16) * chunks;
     CF_CHECK(blocks < (int64_t)INT32_MAX, "paged write too large");
-    CF_LAUNCH((paged_write_tile_kernel<XT, ST, CT>), dim3((unsigned)blocks), dim3(256), 0, stream, p, (uint32_t)chunks);
+    CF_LAUNCH((paged_write_tile_kernel<XT, ST, CT>), grid_of(blocks), dim3(256), 0, stream, p, (uint32_t)chunks);
     CF_HIP_CHECK(hipGetLastError());
     return CF_OK;
   }
@@ -350,8 +360,8 @@ int32_t launch_write_t(const PagedWriteParams& p, hipStream_t stream) {
   const bool vec = p.D % N == 0 && rows_aligned(p.x, p.x_s, 2, p.x_s[2], esize<XT>(), N * esize<XT>()) &&
                    rows_aligned(p.cache, p.c_s, 3, p.c_s[3], esize<CT>(), N * esize<CT>());
   const int64_t threads = p.T * p.H * (vec ? p.D / N : p.D);
-  CF_CHECK(grid_of(threads) < (int64_t)INT32_MAX, "paged write too large");
-  const dim3 grid((unsigned)grid_of(threads));
+  CF_CHECK(blocks_of(threads) < (int64_t)INT32_MAX, "paged write too large");
+  const dim3 grid = grid_of(blocks_of(threads));
   if (vec) CF_LAUNCH((paged_write_kernel<XT, ST, CT, N>), grid, dim3(256), 0, stream, p);
   else CF_LAUNCH((paged_write_kernel<XT, ST, CT, 1>), grid, dim3(256), 0, stream, p);
   CF_HIP_CHECK(hipGetLastError());
@@ -390,9 +400,8 @@ int32_t launch_gather_t(const PagedGatherParams& p, hipStream_t stream) {
       rows_aligned(p.out, p.o_s, 3, p.o_s[3], esize<OT>(), P * esize<OT>())) {
     const int64_t bpr = ceil_div(p.S, 16);
     const int64_t threads = (int64_t)p.R * bpr * (p.H * p.D / P);
-    CF_CHECK(grid_of(threads) < (int64_t)INT32_MAX, "paged gather too large");
-    CF_LAUNCH((paged_gather_tile_kernel<CT, OT, P>), dim3((unsigned)grid_of(threads)), dim3(256), 0, stream, p,
-              (int)bpr);
+    CF_CHECK(blocks_of(threads) < (int64_t)INT32_MAX, "paged gather too large");
+    CF_LAUNCH((paged_gather_tile_kernel<CT, OT, P>), grid_of(blocks_of(threads)), dim3(256), 0, stream, p, (int)bpr);
     CF_HIP_CHECK(hipGetLastError());
     return CF_OK;
   }
@@ -400,8 +409,8 @@ int32_t launch_gather_t(const PagedGatherParams& p, hipStream_t stream) {
   const bool vec = p.D % N == 0 && rows_aligned(p.cache, p.c_s, 3, p.c_s[3], esize<CT>(), N * esize<CT>()) &&
                    rows_aligned(p.out, p.o_s, 3, p.o_s[3], esize<OT>(), N * esize<OT>());
   const int64_t threads = (int64_t)p.R * p.S * p.H * (vec ? p.D / N : p.D);
-  CF_CHECK(grid_of(threads) < (int64_t)INT32_MAX, "paged gather too large");
-  const dim3 grid((unsigned)grid_of(threads));
+  CF_CHECK(blocks_of(threads) < (int64_t)INT32_MAX, "paged gather too large");
+  const dim3 grid = grid_of(blocks_of(threads));
   if (vec) CF_LAUNCH((paged_gather_kernel<CT, OT, N>), grid, dim3(256), 0, stream, p);
   else CF_LAUNCH((paged_gather_kernel<CT, OT, 1>), grid, dim3(256), 0, stream, p);
   CF_HIP_CHECK(hipGetLastError());

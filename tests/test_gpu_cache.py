@@ -426,3 +426,23 @@ def test_channel_major_rows_bit_exact(gpu, rows_dtype, cache_dtype, cut, h, d):
             have = want.view(nb, 16, h, d)[torch.tensor(t)].reshape(-1, h, d)[:seq]
             full[: have.shape[0]] = have * scale.cpu()[:, None] if fp8 else have
             assert torch.equal(got[r], full), (seq, r)
+
+
+def test_rows_of_more_than_two_to_the_32_elements(gpu):
+    """Writes and gathers that take a thread per element (rows that are not
+    16-byte aligned) and hold more than 2^32 of them: the last rows too."""
+    t, h, d = (1 << 14) + 16, 64, 4096
+    x = torch.randn(1, h, d, device=gpu).to(torch.float16)
+    cache = torch.zeros(2, 16, h, d + 1, dtype=torch.float16, device=gpu)[..., :d]
+    slots = torch.full((t,), -1, dtype=torch.int64, device=gpu)
+    slots[0], slots[-1] = 3, 17
+    ops.paged_write(x.expand(t, h, d), slots, cache)
+    want = torch.zeros(2, 16, h, d, dtype=torch.float16, device=gpu)
+    want[0, 3], want[1, 1] = x[0], x[0]
+    assert torch.equal(cache, want)
+    tables = torch.zeros(1, t // 16, dtype=torch.int32, device=gpu)
+    tables[0, -1] = 1
+    out = torch.full((1, t, h, d), float("nan"), dtype=torch.float16, device=gpu)
+    ops.paged_gather(cache, tables, t, out=out)
+    rows = out.view(t // 16, 16, h, d)
+    assert torch.equal(rows[-1], want[1]) and all(torch.equal(rows[i], want[0]) for i in range(0, t // 16 - 1, 97))
