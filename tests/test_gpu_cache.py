@@ -383,7 +383,7 @@ def test_channel_major_rows_bit_exact(gpu, rows_dtype, cache_dtype, cut, h, d):
     channel-major cache and back, against torch's indexing and casts; one row
     below and at the size from which the write goes by blocks, and above it
     with ragged runs."""
-    at_size = (3 << 18) // (h * d) + 1
+    at_size = ((5 if cache_dtype == torch.float8_e4m3fn else 1) << 17) // (h * d) + 1
     lens = [n for n in cut if n > 0] if len(cut) > 1 else []
     lens = lens[:3] + [at_size - min(cut)] + lens[3:]
     g = torch.Generator(device=gpu).manual_seed(sum(lens) + d)
@@ -446,3 +446,43 @@ def test_rows_of_more_than_two_to_the_32_elements(gpu):
     ops.paged_gather(cache, tables, t, out=out)
     rows = out.view(t // 16, 16, h, d)
     assert torch.equal(rows[-1], want[1]) and all(torch.equal(rows[i], want[0]) for i in range(0, t // 16 - 1, 97))
+
+
+@pytest.mark.parametrize("rows_dtype,cache_dtype", [
+    (torch.float32, torch.float32), (torch.float16, torch.float16), (torch.bfloat16, torch.float8_e4m3fn),
+    (torch.float32, torch.float8_e4m3fn)])
+@pytest.mark.parametrize("layout", ["channel-major 32", "channel-major 8", "unaligned", "rows", "strided rows"])
+def test_rows_bit_exact_where_the_launch_changes(gpu, rows_dtype, cache_dtype, layout):
+    """Writes and gathers one value row below and at each size from which they
+    go another way, for every form of cache and row strides that has one."""
+    h, d = 4, 64
+    bs = int(layout.split()[1]) if "channel" in layout else 16
+    fp8 = cache_dtype == torch.float8_e4m3fn
+    g = torch.Generator(device=gpu).manual_seed(bs)
+    scale = torch.rand(h, generator=g, device=gpu) + 0.01 if fp8 else None
+    for values in (1 << 17, 1 << 18, 7 << 16, 1 << 19, 5 << 17, 7 << 17, 1 << 21):
+        for t in (values // (h * d) - 1, values // (h * d)):
+            nb = t // bs + 2
+            raw = torch.uint8 if fp8 else cache_dtype
+            if "channel" in layout:
+                cache = torch.zeros(nb, h, d, bs, dtype=raw, device=gpu).view(cache_dtype).permute(0, 3, 1, 2)
+            elif layout == "unaligned":
+                cache = torch.zeros(nb, bs, h, d + 1, dtype=raw, device=gpu).view(cache_dtype)[..., :d]
+            else:
+                cache = torch.zeros(nb, bs, h, d, dtype=raw, device=gpu).view(cache_dtype)
+            x = torch.randn(t, h, d, generator=g, device=gpu).to(rows_dtype)
+            if layout == "strided rows":
+                x = x.transpose(1, 2).contiguous().transpose(1, 2)
+            slots = torch.randperm(nb * bs, generator=g, device=gpu)[:t]
+            slots[: t // 2] = slots[: t // 2].sort().values  # runs, and rows on their own
+            slots[1] = -1
+            ops.paged_write(x, slots, cache, scale)
+            val = (x.float() / scale[:, None] if fp8 else x).to(cache_dtype).float()
+            want = torch.zeros(nb * bs, h, d, device=gpu)
+            keep = slots >= 0
+            want[slots[keep]] = val[keep]
+            assert torch.equal(cache.float().reshape(nb * bs, h, d), want), (values, t)
+            table = torch.randperm(nb, generator=g, device=gpu).to(torch.int32)
+            got = ops.paged_gather(cache, table.view(1, nb), t, scale=scale)
+            ref = want.view(nb, bs, h, d)[table.long()].reshape(-1, h, d)[:t]
+            assert torch.equal(got[0].float(), ref * scale[:, None] if fp8 else ref), (values, t)
