@@ -205,13 +205,13 @@ __global__ __launch_bounds__(256) void paged_write_tile_kernel(PagedWriteParams 
   const int64_t up = __shfl_up(sl, 1, 64);
   const bool cont = valid && lane > 0 && sl == up + 1 && (sl & 15) != 0;
   const uint32_t vm = (uint32_t)__ballot(valid), cm = (uint32_t)__ballot(cont);
-  // lane 1 + e <-> row e of the group
-  // (computed before any lane leaves: rows are read from lanes whose channel
-  // is past the last one too)
+  // lane 1 + e <-> row e of the group.  Rows are read from lanes whose channel
+  // is past the last one too, so no lane leaves on its own from here on: only
+  // the stores ask whether the channel is there.
   const int64_t blk = p.bs == 16 ? sl >> 4 : sl / p.bs;
   const int64_t dst = valid ? blk * p.c_s[0] + (sl - blk * p.bs) : 0;
   const uint32_t starts = vm & ~cm & 0x1FFFEu;
-  if (!mine || starts == 0u) return;
+  if (starts == 0u) return;  // uniform
   const int e0 = __builtin_ctz(starts) - 1;    // first owned row, 0..15
   const int ext = __builtin_ctz(~(cm >> 17));  // rows past the group that continue its last run, <= 15
   const uint32_t own = ((vm & 0x1FFFEu & ~((2u << e0) - 1u)) >> 1) | (((1u << ext) - 1u) << 16);
@@ -235,14 +235,20 @@ __global__ __launch_bounds__(256) void paged_write_tile_kernel(PagedWriteParams 
         for (int j = 0; j < 16; ++j) out.c[j] = encode<CT>(Elem<XT>::load(&raw[k + j]), qz);
       }
     }
-    uint4* to = (uint4*)(chan + dst_of(e0));
+    const int64_t at = dst_of(e0);
+    if (mine) {
 #pragma unroll
-    for (int q = 0; q < esize<CT>(); ++q) to[q] = out.q[q];
+      for (int q = 0; q < esize<CT>(); ++q) ((uint4*)(chan + at))[q] = out.q[q];
+    }
     return;
   }
 #pragma unroll
-  for (int e = 0; e < 31; ++e)
-    if ((own >> e) & 1u) chan[dst_of(e)] = encode<CT>(Elem<XT>::load(&raw[e]), qz);
+  for (int e = 0; e < 31; ++e) {
+    if ((own >> e) & 1u) {
+      const int64_t at = dst_of(e);
+      if (mine) chan[at] = encode<CT>(Elem<XT>::load(&raw[e]), qz);
+    }
+  }
 }
 
 template <int CT, int OT, int N, bool VEC>
