@@ -382,16 +382,13 @@ dim3 grid_of(int64_t blocks) {
 
 // Values (rows x channels) from which channel-major blocks are written by whole
 // 16-token pieces.  A thread there walks 16 rows, which takes 3.0-3.6 us (4.4-5.4
-// into e4m3fn) however few they are; a thread per element is done in 2.5 us for
-// a decode step, but writes 1 to 4 bytes of every 16 to 64.  By element / by
-// piece: 128,000 fp16 values 3.0 / 3.0 us, 196,608 fp32 values 4.2 / 3.4 us,
-// 512,000 fp16 values 4.2 / 3.3 us; into e4m3fn 512,000 values 4.4 / 5.3 us,
-// 768,000 6.3 / 5.4 us.
-template <int CT>
-constexpr int64_t tile_write_values() {
-  return CT == kE4M3 ? 5 << 17 : 1 << 17;
-}
-// The same for gathers (3.3 us at 16-token pieces, 4.7 from e4m3fn): 256,000
+// into e4m3fn) where runs fill their pieces and 5.5 us where they do not,
+// however few they are; a thread per element is done in 2.5 us for a decode
+// step, but writes 1 to 4 bytes of every 16 to 64.  By element / by piece, whole
+// runs / short ones: 512,000 fp16 values 4.2 / 3.3 / 5.5 us, 768,000 6.8 / 3.7 /
+// 5.5 us; into e4m3fn 512,000 values 4.4 / 5.3 us, 768,000 6.3 / 5.4 us.
+constexpr int64_t kTileWriteValues = 5 << 17;
+// The same for gathers (3.3 us by pieces, 4.7 from e4m3fn): 256,000
 // fp32 values 3.2 / 3.4 us, 384,000 3.8 / 3.5 us; e4m3fn 384,000 3.9 / 4.8 us,
 // 768,000 5.7 / 4.9 us.
 template <int CT>
@@ -410,10 +407,11 @@ constexpr int64_t kWholePieceValues = 1 << 21;
 // Rows with a channel stride on either side: 16 (gathers: 8) channels a thread
 // put several tokens, which such layouts keep side by side, in a wave.  New rows
 // with one: 4,000 fp16 rows of 8 heads of 128 15.4 us by element, 7.9 us; 500
-// rows into e4m3fn 3.9, 5.9 us.  Caches with one (blocks of 8 tokens), heads x
-// head_dim below 1,024: 4,000 fp32 rows of 4 heads of 64 10.9, 4.5 us.
+// rows into e4m3fn 3.9, 5.9 us.  Caches with one, heads x head_dim below 1,024:
+// fp32 rows of 4 heads of 64, 500 of them 3.5, 4.0 us, 1,000 4.8, 4.1, 2,000 7.3,
+// 4.2; with 8 heads of 128 a wave holds one token either way.
 constexpr int64_t kStridedRowValues = 7 << 17;
-constexpr int64_t kStridedCacheValues = 7 << 16;
+constexpr int64_t kStridedCacheValues = 7 << 15;
 constexpr int64_t kStridedGatherValues = 5 << 17;
 
 template <int XT, int ST, int CT, int N, bool VEC>
@@ -431,7 +429,7 @@ template <int XT, int ST, int CT>
 int32_t launch_write_t(const PagedWriteParams& p, hipStream_t stream) {
   ProfileScope prof("cf_paged_write", stream);
   const int64_t values = p.T * p.H * p.D;
-  if (values >= tile_write_values<CT>() && channel_tiles(p.cache, p.c_s, p.bs, esize<CT>())) {
+  if (values >= kTileWriteValues && channel_tiles(p.cache, p.c_s, p.bs, esize<CT>())) {
     const int64_t chunks = blocks_of((int64_t)p.H * p.D), blocks = ceil_div(p.T, 16) * chunks;
     CF_CHECK(blocks < (int64_t)INT32_MAX, "paged write too large");
     CF_LAUNCH((paged_write_tile_kernel<XT, ST, CT>), grid_of(blocks), dim3(256), 0, stream, p, (uint32_t)chunks);
