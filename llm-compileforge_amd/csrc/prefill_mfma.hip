@@ -1170,8 +1170,9 @@ int32_t launch_direct(PrefillParams& p, hipStream_t stream) {
 
 template <int QT, int KT, int D, int G, bool VTOK>
 int32_t launch_t(PrefillParams& p, hipStream_t stream) {
-  p.workers = item_workers<QT, KT, D, G, VTOK, true>();
-  if (p.max_items <= std::min(p.workers, p.split_slots)) return launch_direct<QT, KT, D, G, VTOK>(p, stream);
+  // a piece's workgroup is its workspace slot, so no more of them than slots
+  p.workers = std::min(item_workers<QT, KT, D, G, VTOK, true>(), p.split_slots);
+  if (p.max_items <= p.workers) return launch_direct<QT, KT, D, G, VTOK>(p, stream);
   {
     ProfileScope prof("cf_prefill_plan", stream);
     CF_LAUNCH(prefill_plan_kernel, dim3(1), dim3(kPlanThreads), 0, stream, p);

@@ -36,7 +36,7 @@ struct PrefillParams {
   float2* ws_ml;  // [split_slots][128] a piece's (m in log2 units, l) per column
   float4* ws_o;   // [split_slots][128 * D / 4] its un-normalized output
   int split_slots;  // slots for pieces (0: the call may hold more items than workgroups)
-  int workers;      // direct launches: resident workgroups of the item kernel
+  int workers;      // direct launches: resident workgroups of the item kernel, at most the slots
 };
 
 // Query rows per work item for GQA group G.
