@@ -175,9 +175,15 @@ int32_t cf_paged_decode_shared_noalloc(const CfTensor* q, const CfTensor* k_cach
                                        int32_t partition_tokens, CfTensor* out,
                                        void* stream);
 
-/* Workspace needed by cf_prefill_chunk_fp8 (on the current device) for
- * num_q_tokens query rows in num_chunks chunks.  Grows with the query
- * rows (one small record per query block), not with the cached context. */
+/* Workspace with which cf_prefill_chunk_fp8 runs num_q_tokens query rows in
+ * num_chunks chunks best (on the current device): small records that grow with
+ * the chunks and the query blocks, not with the cached context, and, for calls
+ * of at most one work item (128 / group query rows of one KV head) per resident
+ * workgroup, a fixed 25 MB (head_dim 64) or 34 MB (head_dim 128) for the partial
+ * outputs of long items cut along their KV range.  So a small call's answer can
+ * be above a large one's.  The records alone are enough for any call: a
+ * workspace sized for the largest step serves all smaller ones, without the
+ * cuts where it lacks the room for them. */
 int32_t cf_prefill_chunk_workspace_bytes(int64_t num_q_tokens, int64_t num_chunks,
                                          int64_t num_q_heads, int64_t num_kv_heads,
                                          int64_t head_dim, int32_t block_size,

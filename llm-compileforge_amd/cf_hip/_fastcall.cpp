@@ -152,16 +152,21 @@ at::Tensor new_tensor(at::IntArrayRef sizes, at::ScalarType dtype, const at::Ten
 }
 
 // A workspace of `need` bytes for this device and stream: the caller's, or
-// ops.py's cached one (held by a new reference while the call runs).
+// ops.py's cached one (held by a new reference while the call runs).  `any`: the
+// caller's may be of another size, for the library to judge.
 struct Workspace {
   PyObject* held = nullptr;
   void* ptr = nullptr;
+  uint64_t bytes = 0;
 
-  Workspace(PyObject* given, uint64_t need, const Call& call, PyObject* tensor_on_device) {
+  Workspace(PyObject* given, uint64_t need, const Call& call, PyObject* tensor_on_device, bool any = false) {
     if (need == 0) return;
+    bytes = need;
     if (given != Py_None) {
       const at::Tensor& t = tensor_of(given);
-      if ((uint64_t)(t.numel() * t.element_size()) < need) throw Slow{};
+      const uint64_t has = (uint64_t)(t.numel() * t.element_size());
+      if (any) bytes = has;
+      else if (has < need) throw Slow{};
       ptr = t.data_ptr();
       return;
     }
@@ -272,7 +277,7 @@ PyObject* prefill_chunk(PyObject*, PyObject* const* args, Py_ssize_t n) {
     uint64_t need = 0;
     if (g_lib.prefill_ws(q.size(0), bt.size(0), q.size(1), k.size(2), q.size(2), (int32_t)bs, &need) != CF_OK)
       throw Slow{};
-    const Workspace ws(a[11], need, call, a[0]);
+    const Workspace ws(a[11], need, call, a[0], true);
     at::Tensor fresh;
     CfTensor dout;
     if (a[10] == Py_None) {
@@ -283,7 +288,7 @@ PyObject* prefill_chunk(PyObject*, PyObject* const* args, Py_ssize_t n) {
     }
     const int32_t rc = without_gil([&] {
       return g_lib.prefill(&dq, &dk, &dv, &dt, &dl, &ds, opt(a[8], dks), opt(a[9], dvs), (float)scale, (int32_t)bs,
-                           &dout, ws.ptr, need, call.stream);
+                           &dout, ws.ptr, ws.bytes, call.stream);
     });
     if (rc != CF_OK) return PyLong_FromLong(rc);
     if (a[10] == Py_None) return THPVariable_Wrap(fresh);

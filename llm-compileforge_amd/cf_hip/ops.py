@@ -280,6 +280,9 @@ def prefill_chunk(
     bf16 q, fp16 or e4m3fn under fp16 q, block_size 16, in the native or
     paired tile layout or the reference's token-major rows ([NB, 16, Hkv,
     D] contiguous).
+
+    workspace: optional buffer, by default a cached one per (device, stream);
+    prefill_workspace_bytes() of this call or of a larger one.
     """
     if _on_gpu(q):
         r = _fast().prefill_chunk(q, k_cache, v_cache, block_tables, seq_lens, q_start, float(scale), int(block_size),
@@ -296,8 +299,8 @@ def prefill_chunk(
                                    block_size)
     if workspace is None:
         workspace = _cached_workspace(need, dev)
-    elif workspace.numel() * workspace.element_size() < need:
-        raise ValueError(f"workspace of {need} bytes needed, {workspace.numel() * workspace.element_size()} given")
+    else:  # of another call's size, it may be: the library takes less than `need`, too
+        need = workspace.numel() * workspace.element_size()
     ks = descriptor(k_scale) if k_scale is not None else None
     vs = descriptor(v_scale) if v_scale is not None else None
     d = [descriptor(t) for t in (q, k_cache, v_cache, block_tables, seq_lens, q_start)]

@@ -577,14 +577,13 @@ int32_t cf_prefill_chunk_fp8(const CfTensor* q, const CfTensor* k_cache, const C
   p.RB = prefill_rows_per_item(p.G);
   CF_CHECK((Tq / p.RB + N) * Hkv < (int64_t)INT32_MAX / 2, "too many prefill work items");
   p.max_items = (int)((Tq / p.RB + N) * Hkv);
-  const uint64_t need = prefill_workspace_bytes(Tq, N, Hq, Hkv, D);
-  if (workspace == nullptr || workspace_bytes < need) {
+  const uint64_t need = prefill_bind_workspace(p, workspace, workspace != nullptr ? workspace_bytes : 0);
+  if (need > 0) {
     set_error("workspace of %llu bytes needed, %llu given", (unsigned long long)need,
               (unsigned long long)workspace_bytes);
     return CF_ERR_WORKSPACE;
   }
   CF_CHECK(((uintptr_t)workspace & 255) == 0, "workspace must be 256-byte aligned");
-  prefill_bind_workspace(p, workspace);
   return launch_prefill(p, vq.dtype, vk.dtype, as_stream(stream));
 }
 

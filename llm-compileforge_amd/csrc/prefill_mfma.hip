@@ -1142,15 +1142,20 @@ int item_workers() {
   return prefill_cus() * per_cu;
 }
 
+// No item is longer than the tables' capacity, so short tables bound the
+// pieces of one; 1: too short for a cut.
+int64_t most_pieces(const PrefillParams& p) {
+  const int64_t tiles = ceil_div((int64_t)p.Mb * 16, 32);
+  return tiles > kMinPieceTiles + kCutTiles ? ceil_div(tiles, kMinPieceTiles) : 1;
+}
+
 // Calls of at most one item per resident workgroup: one piece per workgroup
 // (direct_piece), and the merge of the cut items.
 template <int QT, int KT, int D, int G, bool VTOK>
 int32_t launch_direct(PrefillParams& p, hipStream_t stream) {
-  // no item is longer than the tables' capacity, so short tables bound the
-  // pieces, and where no item is long enough for a cut there is nothing to merge
-  // (an empty merge launch is 2 us: 256 rows, 8 heads of 128, 15.2 -> 13.3 us)
-  const int64_t tiles = ceil_div((int64_t)p.Mb * 16, 32);
-  const int64_t most = tiles > kMinPieceTiles + kCutTiles ? ceil_div(tiles, kMinPieceTiles) : 1;
+  // nothing is cut: nothing to merge (an empty merge launch is 2 us: 256 rows, 8
+  // heads of 128, 15.2 -> 13.3 us)
+  const int64_t most = most_pieces(p);
   if (most == 1) p.splits = nullptr;
   {
     ProfileScope prof("cf_prefill_mfma", stream);
@@ -1171,7 +1176,8 @@ int32_t launch_direct(PrefillParams& p, hipStream_t stream) {
 template <int QT, int KT, int D, int G, bool VTOK>
 int32_t launch_t(PrefillParams& p, hipStream_t stream) {
   // a piece's workgroup is its workspace slot, so no more of them than slots
-  p.workers = std::min(item_workers<QT, KT, D, G, VTOK, true>(), p.split_slots);
+  // where an item may be cut (none: the workspace is one of a larger call)
+  p.workers = std::min(item_workers<QT, KT, D, G, VTOK, true>(), most_pieces(p) > 1 ? p.split_slots : kDirectItems);
   if (p.max_items <= p.workers) return launch_direct<QT, KT, D, G, VTOK>(p, stream);
   {
     ProfileScope prof("cf_prefill_plan", stream);
@@ -1258,20 +1264,31 @@ int64_t split_slots_of(int64_t max_items, int64_t D) {
 }
 
 // Workspace: [chunks int4 x N][items int4 x max_items][header 12 int], and
-// for direct launches [merge records 2 int4 x max_items][(m, l) float2 x 128
-// per slot][o float x 128 x D per slot]
+// for direct launches that cut items [merge records 2 int4 x max_items][(m, l)
+// float2 x 128 per slot][o float x 128 x D per slot].  A workspace that ends
+// with the header serves every call: it is then queued.
+uint64_t queue_workspace_bytes(int64_t N, int64_t max_items) {
+  return pad256((uint64_t)N * 16) + pad256((uint64_t)max_items * 16) + 256;
+}
+
+uint64_t slot_workspace_bytes(int64_t max_items, int64_t D, uint64_t slots) {
+  if (slots == 0) return 0;
+  return pad256((uint64_t)max_items * 32) + pad256(slots * kCols * 8) + slots * kCols * (uint64_t)D * 4;
+}
+
 uint64_t prefill_workspace_bytes(int64_t Tq, int64_t N, int64_t Hq, int64_t Hkv, int64_t D) {
   const int64_t G = Hkv > 0 ? Hq / Hkv : 1;
   const int64_t RB = std::max<int64_t>(G > 0 ? kCols / G : 1, 1);
   const int64_t max_items = (Tq / RB + N) * Hkv;
-  const uint64_t slots = (uint64_t)split_slots_of(max_items, D);
-  const uint64_t base = pad256((uint64_t)N * 16) + pad256((uint64_t)max_items * 16) + 256;
-  if (slots == 0) return base;
-  return base + pad256((uint64_t)max_items * 32) + pad256(slots * kCols * 8) + slots * kCols * (uint64_t)D * 4;
+  return queue_workspace_bytes(N, max_items) +
+         slot_workspace_bytes(max_items, D, (uint64_t)split_slots_of(max_items, D));
 }
 
-void prefill_bind_workspace(PrefillParams& p, void* workspace) {
-  const uint64_t slots = (uint64_t)split_slots_of(p.max_items, p.D);
+uint64_t prefill_bind_workspace(PrefillParams& p, void* workspace, uint64_t bytes) {
+  const uint64_t base = queue_workspace_bytes(p.N, p.max_items);
+  if (bytes < base) return base;
+  uint64_t slots = (uint64_t)split_slots_of(p.max_items, p.D);
+  if (bytes - base < slot_workspace_bytes(p.max_items, p.D, slots)) slots = 0;
   p.split_slots = (int)slots;
   char* w = (char*)workspace;
   p.chunks = (int4*)w;
@@ -1279,12 +1296,18 @@ void prefill_bind_workspace(PrefillParams& p, void* workspace) {
   p.items = (int4*)w;
   w += pad256((uint64_t)p.max_items * 16);
   p.header = (int*)w;
-  w += 256;
-  p.splits = (int4*)w;
-  w += pad256((uint64_t)p.max_items * 32);
-  p.ws_ml = (float2*)w;
-  w += pad256(slots * kCols * 8);
-  p.ws_o = (float4*)w;
+  p.splits = nullptr;
+  p.ws_ml = nullptr;
+  p.ws_o = nullptr;
+  if (slots > 0) {
+    w += 256;
+    p.splits = (int4*)w;
+    w += pad256((uint64_t)p.max_items * 32);
+    p.ws_ml = (float2*)w;
+    w += pad256(slots * kCols * 8);
+    p.ws_o = (float4*)w;
+  }
+  return 0;
 }
 
 int32_t launch_prefill(PrefillParams& p, int q_dt, int kv_dt, hipStream_t stream) {

@@ -494,3 +494,35 @@ def test_nan_reaches_the_output_of_a_cut_item(gpu, q_dtype, kv_dtype, where):
     got = out.isnan().all(-1)
     assert torch.equal(got, want), (int(got.sum()), int(want.sum()))
     assert torch.equal(out[~want], clean[~want])
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(32, 8, 128), (12, 12, 64)])
+def test_one_workspace_for_steps_of_all_sizes(gpu, hq, hkv, d):
+    """A workspace sized for the largest step serves the smaller ones, which ask
+    for more of their own: the same rows, queued instead of cut (or, where the
+    tables are too short for a cut, direct); one byte less than the records is
+    refused."""
+    rows = 4096 if hkv == 8 else 16384
+    large = ops.prefill_workspace_bytes(rows, 8, hq, hkv, d)
+    assert large < 1 << 20 < ops.prefill_workspace_bytes(1, 1, hq, hkv, d)
+    ws = torch.empty(large, dtype=torch.uint8, device=gpu)
+    for cached, n in ((0, 1), (100, 60), (4000, 40), (2000, 500)):
+        q, kc, vc, _, _, tables, lens, q_start = _cut_call(gpu, torch.bfloat16, torch.bfloat16, hq, hkv, d, cached, n)
+
+        def run(workspace):
+            return chunked_prefill_attention(q, kc, vc, tables, lens, q_start, workspace=workspace)
+
+        want = run(None)
+        with ops.KernelTimer() as timer:
+            got = run(ws)
+            torch.cuda.synchronize()
+            assert timer.query("cf_prefill_plan")[1] == int(cached >= 2000)
+            assert timer.query("cf_prefill_merge")[1] == 0
+        # sums in another order, rounded to bf16 once each: a unit (2^-7) apart
+        # at most, small values by what the sums' own rounding leaves
+        assert torch.allclose(got.float(), want.float(), rtol=2.0**-7, atol=2.0**-9 * want.float().abs().mean().item())
+        items = (n // (128 * hkv // hq) + 1) * hkv
+        least = 256 * (1 + -(-16 * items // 256)) + 256
+        assert torch.equal(run(ws[:least]), got)
+        with pytest.raises(ValueError, match="workspace of"):
+            run(ws[:least - 1])
