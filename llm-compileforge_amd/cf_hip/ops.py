@@ -445,7 +445,7 @@ def fp8_scale_quantize(*xs: torch.Tensor, per_head: bool) -> list[tuple[torch.Te
             x.is_cuda and x.is_contiguous() and x.shape == x0.shape and x.dtype == x0.dtype and x.device == x0.device
             for x in xs):
         return None
-    if per_head and (x0.dim() < 2 or x0.shape[-1] % 16):
+    if per_head and (x0.dim() < 3 or x0.shape[-1] % 16):  # 2-D: one head (see _as3)
         return None
     heads = x0.shape[-2] if per_head else 1
     shape = (-1, heads, x0.shape[-1] if per_head else 16)

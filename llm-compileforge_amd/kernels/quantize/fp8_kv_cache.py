@@ -136,7 +136,8 @@ class FP8KVCacheQuantizer:
         """Quantizes x [..., H, D] with one scale per head h (axis -2).
 
         scales[h] applies quantize_block's rule to x[..., h, :]; returns
-        (codes of x's shape, float32 scales [H]).
+        (codes of x's shape, float32 scales [H]).  A two-dimensional x is the
+        rows of one head, as for fp8_amax_scale: scales [1].
         """
         self._check_device("x", x)
         if x.dim() < 2:

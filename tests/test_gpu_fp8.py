@@ -368,3 +368,13 @@ def test_paged_write_of_channels_that_do_not_fill_a_wave(gpu, h, d):
         for i in range(h):
             want[37:37 + n, i] = ofp8.quantize(x[:, i].float().cpu().numpy(), float(sc[i]))
         assert np.array_equal(codes(c).reshape(nb * 16, h, d), want)
+
+
+@pytest.mark.parametrize("shape", [(8, 128), (8, 24), (200, 64)])
+def test_a_two_dimensional_block_is_one_head(gpu, shape):
+    """Whatever its sizes: one scale, the codes of the separate calls."""
+    x = torch.randn(shape, device=gpu)
+    x[0] *= 3
+    q, s = FP8KVCacheQuantizer().quantize_per_head(x)
+    assert torch.equal(s, ops.fp8_amax_scale(x)) and s.shape == (1,)
+    assert np.array_equal(codes(q), codes(ops.fp8_quantize(x, s)))
