@@ -381,7 +381,8 @@ PyObject* scale_quantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const at::Tensor& x0 = tensor_of(a[0]);
     const int64_t total = x0.numel();
     if (total == 0 || total % 16 != 0) throw Slow{};
-    if (per_head && (x0.dim() < 3 || x0.size(-1) % 16 != 0)) throw Slow{};  // 2-D: one head
+    // (2-D: one head; the library takes 64 heads, and its workspace grows with them)
+    if (per_head && (x0.dim() < 3 || x0.size(-1) % 16 != 0 || x0.size(-2) > 64)) throw Slow{};
     const Call call(x0);
     const int64_t heads = per_head ? x0.size(-2) : 1, row = per_head ? x0.size(-1) : 16;
     at::Tensor codes[2], scales[2];

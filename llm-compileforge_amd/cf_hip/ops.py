@@ -431,6 +431,9 @@ def fp8_quantize_kv(k: torch.Tensor, v: torch.Tensor, k_scales: torch.Tensor, v_
     return k_out, v_out
 
 
+_DENSE_HEADS = 64  # most heads cf_fp8_scale_quantize takes (its workspace grows with them)
+
+
 def fp8_scale_quantize(*xs: torch.Tensor, per_head: bool) -> list[tuple[torch.Tensor, torch.Tensor]] | None:
     """(codes, scales) of one or two tensors in at most two launches: the
     results of fp8_amax_scale and fp8_quantize with one scale per head (axis
@@ -445,7 +448,7 @@ def fp8_scale_quantize(*xs: torch.Tensor, per_head: bool) -> list[tuple[torch.Te
             x.is_cuda and x.is_contiguous() and x.shape == x0.shape and x.dtype == x0.dtype and x.device == x0.device
             for x in xs):
         return None
-    if per_head and (x0.dim() < 3 or x0.shape[-1] % 16):  # 2-D: one head (see _as3)
+    if per_head and (x0.dim() < 3 or x0.shape[-1] % 16 or x0.shape[-2] > _DENSE_HEADS):  # 2-D: one head (see _as3)
         return None
     heads = x0.shape[-2] if per_head else 1
     shape = (-1, heads, x0.shape[-1] if per_head else 16)

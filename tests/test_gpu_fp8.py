@@ -378,3 +378,16 @@ def test_a_two_dimensional_block_is_one_head(gpu, shape):
     q, s = FP8KVCacheQuantizer().quantize_per_head(x)
     assert torch.equal(s, ops.fp8_amax_scale(x)) and s.shape == (1,)
     assert np.array_equal(codes(q), codes(ops.fp8_quantize(x, s)))
+
+
+def test_many_heads_take_no_workspace(gpu):
+    """More heads than the one-call kernels take: the separate calls, and no
+    memory beyond the outputs."""
+    x = torch.randn(1, 60000, 16, device=gpu)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    q, s = FP8KVCacheQuantizer().quantize_per_head(x)
+    torch.cuda.synchronize()
+    assert torch.cuda.max_memory_allocated() - before <= 4 * (q.numel() + 4 * s.numel())
+    assert torch.equal(s, ops.fp8_amax_scale(x))
