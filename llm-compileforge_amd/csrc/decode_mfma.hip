@@ -450,9 +450,6 @@ __device__ __forceinline__ void store_out4(void* out, int64_t off, float a, floa
   }
 }
 
-// Writes out a finished run (normalized output, record or wave-slot
-// partial) and, from the wave holding the run's first tile, the merge
-// descriptors of the sequences it covers.
 // The four consecutive channels of store t that a lane holds of its column:
 // channels 16 t + 4 lq .. + 3 of O tile t, or (QUAD: fp32 token-major V) the
 // t-th four of its 16 channels 64 u + 16 lq, spread over O tiles 4 u .. 4 u + 3.
@@ -465,6 +462,9 @@ __device__ __forceinline__ float o_elem(const f32x4_t* o, int t, int e) {
   return QUAD ? o[4 * (t >> 2) + e][t & 3] : o[t][e];
 }
 
+// Writes out a finished run (normalized output, record or wave-slot
+// partial) and, from the wave holding the run's first tile, the merge
+// descriptors of the sequences it covers.
 template <int QT, bool PL, int D, bool QUAD = false>
 __device__ __forceinline__ void flush_run(const DecodeParams& p, const Index& ix, const Plan* pl, const Coord& c,
                                           const f32x4_t* o, float m, float l, int run_j0, bool first_run,
@@ -606,29 +606,44 @@ __device__ __forceinline__ void stream_f32(const DecodeParams& p, const Index& i
   int run_j0 = c0.j;
   bool first_run = true;
   // Scores in log2 units, scale * log2(e) = qk_scale + qk_lo to twice the
-  // precision: p = 2^(s * scale * log2(e) - m) is formed in one rounding of
-  // the exponent.
+  // precision.  The reference m is a whole number, and a score's exponent is
+  // split into its nearest whole number e and the rest, which is then held to
+  // full precision (|rest| <= 1/2): p = 2^rest * 2^(e - m), so that neither the
+  // exponent's size nor the distance to the reference, nor a rescale or a merge
+  // of partials (powers of two), rounds anything.
   const float qk_scale = p.scale * kLog2e;
   const float qk_lo = __builtin_fmaf(p.scale, kLog2e, -qk_scale) + p.scale * kLog2eLo;
   for (;;) {
     const bool run_ends = !has1 || c1.b != c0.b || c1.h != c0.h || c1.kind != c0.kind;
-    // four partial sums per score: a short chain rounds less (and the MFMAs
-    // of a chain wait on each other)
-    f32x4_t se[2][4];
-#pragma unroll
-    for (int x = 0; x < 2; ++x)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) se[x][e] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int c = 0; c < NC; ++c)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int x = 0; x < 2; ++x)
-          se[x][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(elem4(r.k[x][c], e), elem4(q[c], e), se[x][e], 0, 0, 0);
+    // A score's channels in sums of kChain MFMAs (4 channels each), added in a
+    // tree: a sum in one chain rounds in proportion to its length.  With the
+    // exponent above and the sums of P.V below, the error against 64 bits over
+    // contexts of 50 to 3,000 tokens is 1.3e-7 to 1.7e-7 (four chains of a
+    // score's channels, one rounding of the exponent and one sum a block: 1.5e-7
+    // to 2.0e-7; the generic kernel 1.5e-7 to 2.3e-7), and 2.0e-7 to 4.0e-7 with
+    // four times the scores (2.4e-7 to 5.3e-7; 2.2e-7 to 4.5e-7).  8 sequences of
+    // 1,000 tokens, 32 / 8 heads of 128: 26.5 -> 25.8 us; 4 of 64 tokens 10.7 ->
+    // 11.3 us.
+    constexpr int kChain = D == 64 ? 1 : 2, kSums = 4 * NC / kChain;
     f32x4_t s[2];
 #pragma unroll
-    for (int x = 0; x < 2; ++x) s[x] = (se[x][0] + se[x][1]) + (se[x][2] + se[x][3]);
+    for (int x = 0; x < 2; ++x) {
+      f32x4_t se[kSums];
+#pragma unroll
+      for (int i = 0; i < kSums; ++i) {
+        se[i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int u = 0; u < kChain; ++u) {
+          const int c = (i * kChain + u) >> 2, e = (i * kChain + u) & 3;
+          se[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(elem4(r.k[x][c], e), elem4(q[c], e), se[i], 0, 0, 0);
+        }
+      }
+#pragma unroll
+      for (int w = kSums / 2; w > 0; w /= 2)
+#pragma unroll
+        for (int i = 0; i < w; ++i) se[i] = se[2 * i] + se[2 * i + 1];
+      s[x] = se[0];
+    }
     // (the last iteration reloads its own tile, so every path has the same
     // number of loads in flight)
     load_k_f32<D, VTOK>(r, kv, c1.blkA, c1.blkB, li, lq, c1.h);
@@ -669,7 +684,7 @@ __device__ __forceinline__ void stream_f32(const DecodeParams& p, const Index& i
     if (__any(mt > m + 8.0f)) {
       mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
       mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-      const float mnew = mt > m + 8.0f ? mt : m;
+      const float mnew = mt > m + 8.0f ? __builtin_rintf(mt) : m;
       const float alpha = mnew == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mnew);
       l *= alpha;
 #pragma unroll
@@ -683,37 +698,38 @@ __device__ __forceinline__ void stream_f32(const DecodeParams& p, const Index& i
     float psum = 0.0f;
 #pragma unroll
     for (int v = 0; v < 8; ++v) {
-      const float raw = s[v >> 2][v & 3];
-      const float ex = __builtin_fmaf(raw, qk_scale, __builtin_fmaf(raw, qk_lo, -mref));
-      pr[v] = sc[v] != -INFINITY ? __builtin_amdgcn_exp2f(ex) : 0.0f;
+      const float raw = s[v >> 2][v & 3], t = raw * qk_scale, e = __builtin_rintf(t);
+      // (past 2^24 the rest is below the score's own last bit)
+      const float lo = __builtin_amdgcn_fmed3f(__builtin_fmaf(raw, qk_lo, __builtin_fmaf(raw, qk_scale, -t)), -0.5f, 0.5f);
+      const int sh = (int)__builtin_amdgcn_fmed3f(e - mref, -300.0f, 300.0f);
+      pr[v] = sc[v] != -INFINITY ? __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((t - e) + lo), sh) : 0.0f;
     }
     psum = ((pr[0] + pr[1]) + (pr[2] + pr[3])) + ((pr[4] + pr[5]) + (pr[6] + pr[7]));
     l += psum;
-    // Step s of block x: tokens 4 lq + s, this lane's own p.  Each block's sum
-    // is formed apart and the tile's added to O once, so a sum over n tokens
-    // is a chain of n / 32 additions instead of n / 4 (the error against 64
-    // bits over contexts of 16 to 10,000 tokens: 1.5e-7 to 2.2e-7, where one
-    // running sum gave up to 4.7e-7 and the generic kernel up to 3.2e-7).
+    // Step s of block x: tokens 4 lq + s, this lane's own p.  Every two steps'
+    // sum is formed apart and the tile's added to O once, so a sum over n tokens
+    // is a chain of n / 32 additions instead of n / 4 (one running sum: errors
+    // of up to 4.7e-7).
     constexpr int kOT = 2;  // O tiles at a time
 #pragma unroll
     for (int t0 = 0; t0 < NV; t0 += kOT) {
-      f32x4_t ot[2][kOT];
+      f32x4_t ot[4][kOT];
 #pragma unroll
-      for (int x = 0; x < 2; ++x)
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int t = 0; t < kOT; ++t) ot[x][t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int t = 0; t < kOT; ++t) ot[i][t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int st = 0; st < 4; ++st)
 #pragma unroll
         for (int x = 0; x < 2; ++x)
 #pragma unroll
           for (int t = 0; t < kOT; ++t) {
-            const int ti = t0 + t;
+            const int ti = t0 + t, i = 2 * x + (st >> 1);
             const float a = VTOK ? elem4(r.v[x][(ti & ~3) + st], ti & 3) : elem4(r.v[x][ti], st);
-            ot[x][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, pr[4 * x + st], ot[x][t], 0, 0, 0);
+            ot[i][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, pr[4 * x + st], ot[i][t], 0, 0, 0);
           }
 #pragma unroll
-      for (int t = 0; t < kOT; ++t) o[t0 + t] = o[t0 + t] + (ot[0][t] + ot[1][t]);
+      for (int t = 0; t < kOT; ++t) o[t0 + t] = o[t0 + t] + ((ot[0][t] + ot[1][t]) + (ot[2][t] + ot[3][t]));
     }
     load_v_f32<D, VTOK>(r, kv, c1.blkA, c1.blkB, li, lq, c1.h);
     if (run_ends) {

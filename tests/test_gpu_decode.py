@@ -794,3 +794,42 @@ def test_nan_reaches_the_output_under_fp32_queries(gpu, kv_dtype, hq, hkv, d, la
     if kv_dtype == torch.float32:
         case.q[1, 0] = float("nan")
         assert _run(case, kc, vc, ks, vs, gpu)[1, 0].isnan().all()
+
+
+@pytest.mark.parametrize("lens,hq,hkv,d", [
+    ([100] * 32, 32, 8, 128), ([64] * 32, 32, 8, 128), ([1000] * 8, 64, 8, 128), ([90] * 64, 16, 1, 128),
+    ([3000] * 4, 32, 8, 128), ([1000] * 8, 32, 4, 64), ([50] * 64, 32, 4, 64), ([2000] * 8, 16, 4, 64),
+    ([700] * 64, 12, 12, 64)])
+@pytest.mark.parametrize("spread", [1.0, 4.0])
+def test_fp32_error_is_not_above_the_partitioned_kernels(gpu, lens, hq, hkv, d, spread):
+    """Over fp32 caches the MFMA kernel's error against 64 bits (2-norm, over
+    some 1,000 heads in four draws, as a head's error goes with its few largest
+    weights) is at most that of the partitioned kernel, also where the scores
+    spread widely and so their own rounding and the exponent's weigh most."""
+    sums = {512: 0.0, 256: 0.0}
+    for seed in range(4):
+        g = torch.Generator(device=gpu).manual_seed(seed)
+        blocks = [-(-n // 16) for n in lens]
+        nb = sum(blocks)
+        perm = torch.randperm(nb, generator=torch.Generator().manual_seed(seed)).tolist()
+        tables, at = [], 0
+        for n in blocks:
+            tables.append(perm[at:at + n])
+            at += n
+        q = torch.randn(len(lens), hq, d, generator=g, device=gpu) * spread
+        k, v = (torch.randn(nb, 16, hkv, d, generator=g, device=gpu) for _ in range(2))
+        case = workloads.DecodeCase("error", q, k, v, tables, lens, 16, 1 / math.sqrt(d), torch.float32)
+        kc, vc, _, _ = workloads.materialize(case, "native")
+        ref = torch.zeros(q.shape, dtype=torch.float64, device=gpu)
+        for b, n in enumerate(lens):
+            kk, vv = (x[torch.tensor(tables[b], device=gpu)].reshape(-1, hkv, d)[:n].double().repeat_interleave(
+                hq // hkv, 1) for x in (k, v))
+            w = torch.softmax((q[b].double() * kk).sum(-1) * case.scale, 0)
+            ref[b] = (w.unsqueeze(-1) * vv).sum(0)
+        for pt in sums:  # 256: a partition length of the caller's own
+            with ops.KernelTimer() as timer:
+                out = _run(case, kc, vc, None, None, gpu, pt=pt)
+                assert timer.query("cf_decode_mfma")[1] == int(pt == 512)
+            sums[pt] += float((out.double() - ref).norm() / ref.norm())
+    print(f"[error] mfma {sums[512] / 4:.3e} partitioned {sums[256] / 4:.3e}", flush=True)
+    assert sums[512] <= sums[256]
