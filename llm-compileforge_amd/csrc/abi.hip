@@ -276,6 +276,29 @@ static int32_t generic_partition(int64_t batch, int64_t num_q_heads, int64_t num
   return (int32_t)t;
 }
 
+// Whether fp32 caches under fp32 queries, in a layout that the MFMA kernel
+// takes, are better off on the generic kernel: where few query heads share a KV
+// head, and so few of the MFMA's 16 columns are used, as long as the call is
+// bound by its launches' latency rather than by its bytes, and a sequence does
+// not leave its reduce hundreds of partitions.  Generic / MFMA, in us, with
+// tables of `capacity` tokens all in use:
+//   group 1, 12 heads of 64:  1 x 16 5.9 / 8.6, 4 x 512 11.8 / 13.5, 64 x 128
+//     22.7 / 23.5, 256 x 64 34 / 32, 64 x 512 59 / 49, 1 x 8,000 23.1 / 18.8;
+//   group 1, 32 heads of 128: 4 x 512 22.4 / 26.8, 16 x 256 36.8 / 36.4, 64 x 128
+//     59 / 54;
+//   group 2, 8 KV heads of 128: 1 x 64 12.6 / 10.7, 16 x 256 18.6 / 20.6, 16 x 512
+//     25.7 / 25.7, 64 x 256 43 / 36; of 64: 4 x 1,024 14.2 / 16.5, 64 x 128 22 / 19,
+//     1 x 4,096 16.2 / 15.0;
+//   group 4, 8 KV heads of 128: 1 x 16 9.1 / 10.3, 256 x 16 23.6 / 25.4, 1 x 32
+//     13.5 / 10.2;
+//   group 8, 4 KV heads of 64: 1 x 16 10.7 / 8.2.
+static bool f32_generic_faster(int64_t batch, int64_t num_kv_heads, int64_t group, int64_t capacity) {
+  const int64_t rows = batch * num_kv_heads * capacity;  // K rows of one head
+  if (group == 1) return rows <= 1 << 17 && capacity <= 4096;
+  if (group == 2) return rows <= 1 << 15 && capacity <= 2048;
+  return group == 4 && capacity <= 16;
+}
+
 // Generic-path layout: [o partials, 256-byte padded] [(m, l)].
 static uint64_t generic_workspace_bytes(int64_t batch, int64_t num_q_heads, int64_t head_dim, int64_t parts) {
   if (parts <= 1) return 0;
@@ -412,12 +435,13 @@ int32_t cf_paged_decode_shared(const CfTensor* q, const CfTensor* k_cache, const
   if (B == 0) return CF_OK;
 
   bool mfma = decode_mfma_supported(p, vq.dtype, vk.dtype);
-  // fp32 caches also run on the generic kernel.  It takes the calls that ask
-  // for a partition length of their own (the MFMA kernel has no partitions),
-  // and those whose workspace, or the fixed scratch, holds its partials
-  // (none for short tables) but not the MFMA kernel's rows.
+  // fp32 caches also run on the generic kernel.  It takes the calls that it is
+  // faster for, those that ask for a partition length of their own (the MFMA
+  // kernel has no partitions), and those whose workspace, or the fixed scratch,
+  // holds its partials (none for short tables) but not the MFMA kernel's rows.
   if (mfma && vk.dtype == CF_F32 &&
-      (partition_tokens != kDefaultPartitionTokens ||
+      (f32_generic_faster(B, Hkv, p.G, vt.size[1] * (int64_t)bs) ||
+       partition_tokens != kDefaultPartitionTokens ||
        workspace_bytes < decode_mfma_workspace_bytes(B, Hq, Hkv, D)))
     mfma = false;
   const uint64_t need = mfma ? decode_mfma_workspace_bytes(B, Hq, Hkv, D)

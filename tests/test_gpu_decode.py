@@ -833,3 +833,25 @@ def test_fp32_error_is_not_above_the_partitioned_kernels(gpu, lens, hq, hkv, d, 
             sums[pt] += float((out.double() - ref).norm() / ref.norm())
     print(f"[error] mfma {sums[512] / 4:.3e} partitioned {sums[256] / 4:.3e}", flush=True)
     assert sums[512] <= sums[256]
+
+
+@pytest.mark.parametrize("hq,hkv,d,batch,capacity,mfma", [
+    (4, 4, 64, 16, 2048, False), (4, 4, 64, 16, 2064, True), (1, 1, 64, 1, 4096, False), (1, 1, 128, 1, 4112, True),
+    (4, 2, 128, 16, 1024, False), (4, 2, 64, 16, 1040, True), (2, 1, 128, 1, 2048, False), (2, 1, 64, 1, 2064, True),
+    (8, 2, 128, 300, 16, False), (8, 2, 128, 2, 32, True), (8, 1, 64, 1, 16, True)])
+def test_fp32_kernel_choice(gpu, hq, hkv, d, batch, capacity, mfma):
+    """Both sides of the lines by which a call over an fp32 cache goes to the
+    partitioned kernel or to the MFMA kernel."""
+    g = torch.Generator(device=gpu).manual_seed(capacity)
+    per = capacity // 16
+    lens = [max(1, capacity - 37 * (i % 8)) for i in range(batch)]
+    nb = min(batch * per, 600)
+    tables = [[(i * 7 + j) % nb for j in range(per)] for i in range(batch)]
+    q = torch.randn(batch, hq, d, generator=g, device=gpu)
+    k, v = (torch.randn(nb, 16, hkv, d, generator=g, device=gpu) for _ in range(2))
+    case = workloads.DecodeCase("route", q, k, v, tables, lens, 16, 1 / math.sqrt(d), torch.float32)
+    kc, vc, ks, vs = workloads.materialize(case, "native")
+    with ops.KernelTimer() as timer:
+        out = _run(case, kc, vc, ks, vs, gpu)
+        assert timer.query("cf_decode_mfma")[1] == int(mfma) and timer.query("cf_decode_generic")[1] == int(not mfma)
+    assert_close(out.cpu().numpy(), oracle_decode(case, kc, vc, ks, vs), torch.float32, "choice")
