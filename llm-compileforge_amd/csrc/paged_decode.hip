@@ -135,9 +135,11 @@ __global__ __launch_bounds__(kGenericThreads) void decode_generic_kernel(DecodeP
     float m = -INFINITY;
     for (int i = lane; i < count; i += 64) m = fmaxf(m, sc[g * PT + i]);
     m = wave_max(m);
+    // no finite score: masked tokens get 0, NaN ones keep it
+    const float mref = m == -INFINITY ? 0.0f : m;
     float l = 0.0f;
     for (int i = lane; i < count; i += 64) {
-      const float e = m == -INFINITY ? 0.0f : expf(sc[g * PT + i] - m);
+      const float e = expf(sc[g * PT + i] - mref);
       sc[g * PT + i] = e;
       l += e;
     }
@@ -179,7 +181,8 @@ __global__ __launch_bounds__(kGenericThreads) void decode_generic_kernel(DecodeP
       }
     } else if (active) {
       // kU tokens per step, their loads issued together (an invalid block
-      // reads block 0 and gets weight 0; a cache without blocks is not read)
+      // reads block 0, and zeros take its place; a cache without blocks is not
+      // read)
       constexpr int kU = 8;
       for (int t0 = grp; p.NB > 0 && t0 < count; t0 += kU * ng) {
         float vv[kU], ww[kU];
@@ -191,7 +194,8 @@ __global__ __launch_bounds__(kGenericThreads) void decode_generic_kernel(DecodeP
           const bool ok = t < count && (uint64_t)blk < (uint64_t)p.NB;
           const typename KE::T* vrow = vbase + (ok ? blk : 0) * p.v_s[0] + (int64_t)((start + tt) % bs) * p.v_s[1] +
                                        (int64_t)h * p.v_s[2];
-          vv[u] = KE::load(vrow + (int64_t)d * p.v_s[3]);
+          const float x = KE::load(vrow + (int64_t)d * p.v_s[3]);
+          vv[u] = ok ? x : 0.0f;
           ww[u] = ok ? sc[g * PT + tt] : 0.0f;
         }
 #pragma unroll
@@ -212,7 +216,7 @@ __global__ __launch_bounds__(kGenericThreads) void decode_generic_kernel(DecodeP
     if (DIRECT) {
       const float l = sml[2 * g + 1];
       OutE::store((typename OutE::T*)p.out + (int64_t)b * p.o_sb + (int64_t)hq * p.o_sh + d,
-                  l > 0.0f ? acc / l : 0.0f);
+                  l > 0.0f ? acc / l : acc * 0.0f);  // (l NaN: so is acc)
     } else {
       const int64_t row = ((int64_t)b * p.Hq + hq) * p.max_parts + part;
       p.ws_o[row * D + d] = acc;
@@ -252,12 +256,11 @@ __global__ __launch_bounds__(256) void decode_reduce_kernel(DecodeParams p) {
   if (lane == 0) red[wave] = mloc;
   __syncthreads();
   const float M = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-  // A partition whose blocks were all invalid has m = -inf and l = 0.
+  // A partition without a finite score has m = -inf and l = o = 0, or NaN where
+  // a score or a V value was: weight 1 keeps both.
+  auto weight = [&](float m) { return m != -INFINITY ? expf(m - M) : 1.0f; };
   float lloc = 0.0f;
-  for (int i = tid; i < nparts; i += 256) {
-    const float m = ml[i * 2];
-    if (m != -INFINITY) lloc += ml[i * 2 + 1] * expf(m - M);
-  }
+  for (int i = tid; i < nparts; i += 256) lloc += ml[i * 2 + 1] * weight(ml[i * 2]);
   lloc = wave_sum(lloc);
   if (lane == 0) red[4 + wave] = lloc;
   __syncthreads();
@@ -267,8 +270,7 @@ __global__ __launch_bounds__(256) void decode_reduce_kernel(DecodeParams p) {
     for (int d = tid; d < p.D; d += 256) {
       float acc = 0.0f;
       for (int i = 0; i < nparts; ++i) {
-        const float m = ml[i * 2];
-        if (m != -INFINITY) acc = fmaf(expf(m - M), po[(int64_t)i * p.D + d], acc);
+        acc = fmaf(weight(ml[i * 2]), po[(int64_t)i * p.D + d], acc);
       }
       OutE::store(o + d, acc * inv);
     }
@@ -280,9 +282,7 @@ __global__ __launch_bounds__(256) void decode_reduce_kernel(DecodeParams p) {
   if (grp < ng) {
 #pragma unroll 4
     for (int i = grp; i < nparts; i += ng) {
-      const float m = ml[i * 2];
-      const float w = m != -INFINITY ? expf(m - M) : 0.0f;
-      acc = fmaf(w, po[(int64_t)i * p.D + d], acc);
+      acc = fmaf(weight(ml[i * 2]), po[(int64_t)i * p.D + d], acc);
     }
   }
   part_acc[tid] = acc;

@@ -759,7 +759,8 @@ def test_full_c3_token_major(gpu):
 @pytest.mark.parametrize("kv_dtype", [torch.float32, torch.bfloat16, torch.float8_e4m3fn])
 @pytest.mark.parametrize("hq,hkv,d", [(32, 8, 128), (12, 12, 64)])
 @pytest.mark.parametrize("layout", ["native", "token_major"])
-@pytest.mark.parametrize("lens", [[700] * 64, [64, 40, 5000]], ids=["whole runs", "split runs"])
+@pytest.mark.parametrize("lens", [[700] * 64, [64, 40, 5000], [64, 40], [14, 16]],
+                         ids=["whole runs", "split runs", "partitions", "one partition"])
 def test_nan_reaches_the_output_under_fp32_queries(gpu, kv_dtype, hq, hkv, d, layout, lens):
     """One NaN key among many finite ones makes its KV head's outputs NaN,
     whether its run is written whole or merged; over fp32 caches also where a
@@ -780,9 +781,10 @@ def test_nan_reaches_the_output_under_fp32_queries(gpu, kv_dtype, hq, hkv, d, la
     assert torch.isfinite(clean).all()
     bits = kc.view(torch.uint8) if kv_dtype == torch.float8_e4m3fn else kc
     last, head, grp = len(lens) - 1, hkv - 1, hq // hkv
-    sequences = {last: [(2, 5)]}
+    sequences = {last: [(blocks[last] - 1, 5)]}
     if kv_dtype == torch.float32:
-        sequences = {last: [(j, slice(None)) for j in range(4)], 0: [(j, slice(None)) for j in range(blocks[0])]}
+        sequences = {last: [(j, slice(None)) for j in range(min(4, blocks[last]))],
+                     0: [(j, slice(None)) for j in range(blocks[0])]}
     want = torch.zeros(len(lens), hq, dtype=torch.bool, device=gpu)
     for b, cells in sequences.items():
         for j, tok in cells:
