@@ -32,6 +32,10 @@ extern "C" {
 
 #define CF_ABI_VERSION 1
 
+/* partition_tokens of a decode call that leaves the choice of kernel to the
+ * library (see cf_paged_decode). */
+#define CF_DEFAULT_PARTITION_TOKENS 512
+
 /* dtype codes: 0..6 follow the reference's SfaConstant.dtype_code numbering
  * (reference include/sfa_abi.proto:86); 7 is added for OCP FP8 e4m3fn. */
 typedef enum {
@@ -103,14 +107,21 @@ int32_t cf_paged_decode_workspace_bytes(int64_t batch, int64_t num_q_heads,
  * contributes no tokens (the dict-based Python API rejects such tables
  * before the call, as the reference's indexing would).
  *
- * With bf16 q, bf16/e4m3fn caches, bs = 16, head_dim 64 or 128, G <= 16,
- * K rows with unit channel stride and V stored channel-major inside a
- * block (token stride 1: the layout cf_hip.layout calls "native"), one
- * MFMA kernel balances 32-token tiles evenly over all waves of the GPU and
- * a merge kernel combines the sequences split between waves;
- * partition_tokens is unused there.  Other inputs run a generic kernel that
- * splits sequences into partition_tokens partitions (multiple of bs)
- * merged by a log-sum-exp reduce.
+ * Two kernels.  One, on the matrix cores, balances 32-token tiles evenly over
+ * all waves of the GPU, and a merge kernel combines the sequences split between
+ * waves.  It takes bs = 16, head_dim 64 or 128, Hq/Hkv of 1, 2, 4, 8 or 16, K
+ * rows with unit channel stride and V stored channel-major inside a block
+ * (token stride 1: the layout cf_hip.layout calls "native") or token-major, all
+ * 16-byte aligned, with
+ *     q bf16 over bf16 or e4m3fn caches,   q f16 over f16 or e4m3fn caches,
+ *     q f32 over bf16, e4m3fn or f32 caches.
+ * The other, for every other input, splits sequences into partitions of
+ * partition_tokens tokens (a multiple of bs; shortened where the call is small)
+ * merged by a log-sum-exp reduce.  partition_tokens is unused by the first, with
+ * one exception: a call over f32 caches with another value than
+ * CF_DEFAULT_PARTITION_TOKENS asks for partitions of that length, and so for the
+ * second kernel.  f32 caches also go there in small calls with Hq/Hkv of at most
+ * 4, which it is faster for, and where the workspace is too small for the first.
  *
  * workspace: cf_paged_decode_workspace_bytes() bytes, 256-byte aligned;
  * calls that share a workspace must not overlap. */

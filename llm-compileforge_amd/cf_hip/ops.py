@@ -15,7 +15,7 @@ import torch
 from . import _abi
 from ._abi import check, descriptor, lib, ref, stream_handle
 
-DEFAULT_PARTITION_TOKENS = 512
+DEFAULT_PARTITION_TOKENS = 512  # CF_DEFAULT_PARTITION_TOKENS
 
 
 def _require_device(name: str, t: torch.Tensor) -> None:
@@ -159,6 +159,10 @@ def paged_decode(
     block_tables: int32 [B, Mb]; seq_lens: int32 [B]; caches [NB, bs, Hkv, D]
     with any strides (f32/f16/bf16/e4m3fn); e4m3fn caches need per-KV-head
     fp32 k_scale/v_scale of shape [Hkv] or [1].
+
+    partition_tokens: partition length of the calls that the partitioned kernel
+    takes.  Over float32 caches any other value than the default asks for that
+    kernel (2 to 4 times as long on large calls).
     """
     if _on_gpu(q):
         r = _fast().paged_decode(q, k_cache, v_cache, block_tables, seq_lens, float(scale), int(block_size), k_scale,

@@ -251,8 +251,6 @@ int32_t cf_last_error(char* buf, uint64_t len) {
   return (int32_t)e.size();
 }
 
-constexpr int32_t kDefaultPartitionTokens = 512;  // the binding's default
-
 static int64_t decode_max_parts(int64_t max_blocks, int32_t bs, int32_t pt) {
   return std::max<int64_t>(1, ceil_div(max_blocks * (int64_t)bs, pt));
 }
@@ -441,7 +439,7 @@ int32_t cf_paged_decode_shared(const CfTensor* q, const CfTensor* k_cache, const
   // holds its partials (none for short tables) but not the MFMA kernel's rows.
   if (mfma && vk.dtype == CF_F32 &&
       (f32_generic_faster(B, Hkv, p.G, vt.size[1] * (int64_t)bs) ||
-       partition_tokens != kDefaultPartitionTokens ||
+       partition_tokens != CF_DEFAULT_PARTITION_TOKENS ||
        workspace_bytes < decode_mfma_workspace_bytes(B, Hq, Hkv, D)))
     mfma = false;
   const uint64_t need = mfma ? decode_mfma_workspace_bytes(B, Hq, Hkv, D)

@@ -1,7 +1,8 @@
 // Paged decode attention: generic VALU kernel (any dtype, any block size,
 // any strides) and the log-sum-exp partition reduce.  It takes the calls that
 // decode_mfma.hip does not (other head dims, block sizes, groups, strides or
-// dtype pairs) and fp32 caches with a partition length of the caller's own.
+// dtype pairs), small calls over fp32 caches, and those with a partition length
+// of the caller's own.
 //
 // Semantics follow the reference CPU path (kernels/paged_attention.py:21-73):
 // sequence b attends non-causally to its first min(seq_len, Mb*bs) cached

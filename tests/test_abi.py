@@ -301,3 +301,10 @@ def test_prefill_cache_layout_checks():
     ds, run = call(cache, cache)
     ds[2].t.r4.strides[1] = 1
     assert run() == _abi.CF_ERR_UNSUPPORTED
+
+
+def test_the_default_partition_length_is_the_headers():
+    from cf_hip import ops
+
+    text = (ROOT / "include" / "cf_hip.h").read_text()
+    assert int(re.search(r"#define CF_DEFAULT_PARTITION_TOKENS (\d+)", text).group(1)) == ops.DEFAULT_PARTITION_TOKENS
