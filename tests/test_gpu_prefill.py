@@ -526,3 +526,28 @@ def test_one_workspace_for_steps_of_all_sizes(gpu, hq, hkv, d):
         assert torch.equal(run(ws[:least]), got)
         with pytest.raises(ValueError, match="workspace of"):
             run(ws[:least - 1])
+
+
+@pytest.mark.parametrize("q_dtype,kv_dtype", [
+    (torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float8_e4m3fn), (torch.float16, torch.float16),
+    (torch.float16, torch.float8_e4m3fn)])
+@pytest.mark.parametrize("hq,hkv,d", [(32, 8, 128), (12, 12, 64)])
+@pytest.mark.parametrize("scale", [1.0, -1.0, 0.0])
+def test_relative_error_of_cut_items(gpu, q_dtype, kv_dtype, hq, hkv, d, scale):
+    """Cut items against the float64 oracle by their 2-norm, as outputs behind
+    thousands of tokens are far below the absolute bound of assert_close: the
+    output's rounding (half a unit, 2^-9 bf16, 2^-12 fp16) and P's (2^-12 as one
+    fp16 term) at their largest, and as much again for the sums.  Any scale sign."""
+    q, kc, vc, ks, vs, tables, lens, q_start = _cut_call(gpu, q_dtype, kv_dtype, hq, hkv, d, 3000, 33)
+    scale /= d**0.5
+    with ops.KernelTimer() as timer:
+        out = chunked_prefill_attention(q, kc, vc, tables, lens, q_start, 16, scale, k_scale=ks, v_scale=vs)
+        torch.cuda.synchronize()
+        assert timer.query("cf_prefill_merge")[1] == 1
+    k, v = _cache_values(kc, vc, list(range(kc.shape[0])))
+    ref, _ = paged_prefill_fp64(q.float().cpu().numpy(), k, v, tables.tolist(), lens.tolist(), q_start.tolist(), 16, scale,
+                                *(x.cpu().numpy() if x is not None else None for x in (ks, vs)))
+    got = out.double().cpu().numpy()
+    err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    print(f"[error] {q_dtype} over {kv_dtype}, scale {scale:.3f}: {err:.2e}", flush=True)
+    assert err <= 2 * (2.0**-9 if q_dtype == torch.bfloat16 else 2.0**-12 + 2.0**-12)
