@@ -232,9 +232,13 @@ __global__ __launch_bounds__(256) void kv_write_native_kernel(KvWriteParams p, u
   }
   const uint32_t vb = blockIdx.x - k_blocks;
   const uint32_t g = vb / v_chunks;
-  const int hd = (int)(vb - g * v_chunks) * 256 + (int)threadIdx.x;
-  const bool mine = hd < p.H * p.D;
-  const int h = mine ? hd / p.D : 0, d = mine ? hd % p.D : 0;
+  // Rows are read from lanes by their number, so no lane of a wave may leave on
+  // its own: lanes past the last channel repeat it (the same bytes to the same
+  // place), and only whole waves past it leave.
+  const int hd0 = (int)(vb - g * v_chunks) * 256 + (int)threadIdx.x;
+  if (hd0 - (int)(threadIdx.x & 63) >= p.H * p.D) return;
+  const int hd = min(hd0, p.H * p.D - 1);
+  const int h = hd / p.D, d = hd % p.D;
   // lane l holds the slot of row g * 16 - 1 + l (-1 outside [0, T)): the
   // row before the group, the group's 16 rows and the 15 after them (a run
   // starting in the group ends within 16 rows)
@@ -259,9 +263,7 @@ __global__ __launch_bounds__(256) void kv_write_native_kernel(KvWriteParams p, u
   // Lane 1 + e <-> row e of the group.  Runs start at valid rows that do not
   // continue the previous one; the group owns the valid rows 0..15 from its
   // first run start on, and rows 16..30 that continue its last run.
-  // each row's destination (block row base + token offset), per lane.  Rows are
-  // read from lanes whose channel is past the last one too, so no lane leaves
-  // on its own from here on: only the stores ask whether the channel is there.
+  // each row's destination (block row base + token offset), per lane
   const int64_t dst = valid ? (sl >> 4) * p.vc_s[0] + (sl & 15) : 0;
   const uint32_t starts = vm & ~cm & 0x1FFFEu;
   if (starts == 0u) return;  // uniform
@@ -292,29 +294,20 @@ __global__ __launch_bounds__(256) void kv_write_native_kernel(KvWriteParams p, u
     if (ow == 0xFFFFu && ((cm >> (e0 + 2)) & 0x7FFFu) == 0x7FFFu) {
       // a run of 16 rows fills one block's channel row (its start is at
       // token 0 of the block)
-      uint8_t* to = vcache + dst_of(e0);
-      if (mine) *(uint4*)(to + chan) = c4;
+      *(uint4*)(vcache + dst_of(e0) + chan) = c4;
       return;
     }
     const uint32_t cw[4] = {c4.x, c4.y, c4.z, c4.w};
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      if ((ow >> j) & 1u) {
-        uint8_t* to = vcache + dst_of(e0 + j);
-        if (mine) to[chan] = (uint8_t)(cw[j >> 2] >> (8 * (j & 3)));
-      }
-    }
+    for (int j = 0; j < 16; ++j)
+      if ((ow >> j) & 1u) vcache[dst_of(e0 + j) + chan] = (uint8_t)(cw[j >> 2] >> (8 * (j & 3)));
     return;
   }
   // owned rows spread over more than 16 (a short run, then a run reaching
   // past the group): byte by byte
 #pragma unroll
-  for (int e = 0; e < 31; ++e) {
-    if ((own >> e) & 1u) {
-      uint8_t* to = vcache + dst_of(e);
-      if (mine) to[chan] = qv(XE::load(&raw[e]));
-    }
-  }
+  for (int e = 0; e < 31; ++e)
+    if ((own >> e) & 1u) vcache[dst_of(e) + chan] = qv(XE::load(&raw[e]));
 }
 
 // Whether kv_write_native_kernel applies: native cache layout with block

@@ -185,9 +185,13 @@ __global__ __launch_bounds__(256) void paged_write_tile_kernel(PagedWriteParams 
   using C = typename Elem<CT>::T;
   const uint32_t block = (uint32_t)block_index(), g = block / chunks;
   if ((int64_t)g * 16 >= p.T) return;  // past the last group
-  const int hd = (int)(block - g * chunks) * 256 + (int)threadIdx.x;
-  const bool mine = hd < p.H * p.D;
-  const int h = mine ? hd / p.D : 0, d = mine ? hd % p.D : 0;
+  // Rows are read from lanes by their number, so no lane of a wave may leave on
+  // its own: lanes past the last channel repeat it (the same bytes to the same
+  // place), and only whole waves past it leave.
+  const int hd0 = (int)(block - g * chunks) * 256 + (int)threadIdx.x;
+  if (hd0 - (int)(threadIdx.x & 63) >= p.H * p.D) return;
+  const int hd = min(hd0, p.H * p.D - 1);
+  const int h = hd / p.D, d = hd % p.D;
   // lane l: the slot of row g * 16 - 1 + l (-1 outside [0, T))
   const int lane = (int)(threadIdx.x & 63);
   const int64_t r = (int64_t)g * 16 - 1 + lane;
@@ -205,9 +209,7 @@ __global__ __launch_bounds__(256) void paged_write_tile_kernel(PagedWriteParams 
   const int64_t up = __shfl_up(sl, 1, 64);
   const bool cont = valid && lane > 0 && sl == up + 1 && (sl & 15) != 0;
   const uint32_t vm = (uint32_t)__ballot(valid), cm = (uint32_t)__ballot(cont);
-  // lane 1 + e <-> row e of the group.  Rows are read from lanes whose channel
-  // is past the last one too, so no lane leaves on its own from here on: only
-  // the stores ask whether the channel is there.
+  // lane 1 + e <-> row e of the group
   const int64_t blk = p.bs == 16 ? sl >> 4 : sl / p.bs;
   const int64_t dst = valid ? blk * p.c_s[0] + (sl - blk * p.bs) : 0;
   const uint32_t starts = vm & ~cm & 0x1FFFEu;
@@ -235,20 +237,14 @@ __global__ __launch_bounds__(256) void paged_write_tile_kernel(PagedWriteParams 
         for (int j = 0; j < 16; ++j) out.c[j] = encode<CT>(Elem<XT>::load(&raw[k + j]), qz);
       }
     }
-    const int64_t at = dst_of(e0);
-    if (mine) {
+    uint4* to = (uint4*)(chan + dst_of(e0));
 #pragma unroll
-      for (int q = 0; q < esize<CT>(); ++q) ((uint4*)(chan + at))[q] = out.q[q];
-    }
+    for (int q = 0; q < esize<CT>(); ++q) to[q] = out.q[q];
     return;
   }
 #pragma unroll
-  for (int e = 0; e < 31; ++e) {
-    if ((own >> e) & 1u) {
-      const int64_t at = dst_of(e);
-      if (mine) chan[at] = encode<CT>(Elem<XT>::load(&raw[e]), qz);
-    }
-  }
+  for (int e = 0; e < 31; ++e)
+    if ((own >> e) & 1u) chan[dst_of(e)] = encode<CT>(Elem<XT>::load(&raw[e]), qz);
 }
 
 template <int CT, int OT, int N, bool VEC>
@@ -318,8 +314,8 @@ __global__ __launch_bounds__(256) void paged_gather_tile_kernel(PagedGatherParam
     r = (int)(rb / blocks_per_row);
   }
   const int hd = (int)(u - rb * per) * P;
-  const int s0 = (int)(rb - (int64_t)r * blocks_per_row) * 16;  // first token
-  const int jb = s0 / p.bs;
+  const int piece = (int)(rb - (int64_t)r * blocks_per_row), s0 = piece * 16;  // first token
+  const int jb = p.bs == 16 ? piece : (int)((uint32_t)s0 / (uint32_t)p.bs);
   const int h = hd / p.D, d = hd - h * p.D;
   int64_t blk = -1;
   if (jb < p.Mb) {
