@@ -1103,8 +1103,9 @@ int32_t launch_scale_quantize(const Rank4* x, const Rank4* out, float* const* sc
   CF_HIP_CHECK(hipGetLastError());
   {
     // 16 workgroups per CU at most, as each reduces the maxima (2 x 33.5 MB of
-    // bf16: 19-23 us, 4.4-5.3 TB/s; 4 to 32 per CU lie within the spread that
-    // the buffers' placement gives)
+    // bf16: 27-32 us, 3.1-3.7 TB/s, behind the first pass over other buffers than
+    // the call before; 19-23 us where the same call repeats.  4 to 32 per CU lie
+    // within the spread that the buffers' placement gives)
     const int blocks = (int)std::min<int64_t>(16 * (int64_t)device_cu_count() / count, ceil_div(p.n, 256 * kDenseBatch));
     ProfileScope prof("cf_fp8_quantize", stream);
     CF_SQ(quantize_parts_kernel, dim3(blocks, count), dim3(256), 0, stream, p, wgs)
