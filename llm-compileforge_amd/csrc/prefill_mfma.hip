@@ -438,8 +438,8 @@ __device__ __forceinline__ TileIds tile_resolve(int ia, int ib, int NB) {
 // Block ids of tile j from the item's table row (`trow`, stride t_sm).
 __device__ __forceinline__ TileIds tile_ids(const PrefillParams& p, const int32_t* __restrict__ trow, int j,
                                             int kvlen) {
-  const int nblk = (kvlen + 15) >> 4;
-  const int ia = trow[(int64_t)(2 * j) * p.t_sm];
+  const int nblk = (kvlen + 15) >> 4;  // 0: no table entry is read (the table may have none)
+  const int ia = 2 * j < nblk ? trow[(int64_t)(2 * j) * p.t_sm] : -1;
   const int ib = 2 * j + 1 < nblk ? trow[(int64_t)(2 * j + 1) * p.t_sm] : -1;
   return tile_resolve(ia, ib, p.NB);
 }

@@ -551,3 +551,15 @@ def test_relative_error_of_cut_items(gpu, q_dtype, kv_dtype, hq, hkv, d, scale):
     err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
     print(f"[error] {q_dtype} over {kv_dtype}, scale {scale:.3f}: {err:.2e}", flush=True)
     assert err <= 2 * (2.0**-9 if q_dtype == torch.bfloat16 else 2.0**-12 + 2.0**-12)
+
+
+@pytest.mark.parametrize("chunks", [1, 700])
+def test_tables_without_blocks_give_zero_rows(gpu, chunks):
+    """Block tables of no columns (direct and queued calls): nothing is visible."""
+    q, kc, vc, ks, vs, _, _, _ = _cut_call(gpu, torch.bfloat16, torch.bfloat16, 8, 8, 64, 0, 16)
+    q = q.repeat(chunks, 1, 1)
+    tables = torch.empty(chunks, 0, dtype=torch.int32, device=gpu)
+    lens = torch.full((chunks,), 16, dtype=torch.int32, device=gpu)
+    starts = torch.arange(chunks + 1, dtype=torch.int32, device=gpu) * 16
+    out = chunked_prefill_attention(q, kc, vc, tables, lens, starts, out=torch.full_like(q, float("nan")))
+    assert torch.equal(out, torch.zeros_like(q))
