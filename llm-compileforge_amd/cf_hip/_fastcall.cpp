@@ -191,12 +191,14 @@ struct Workspace {
   Workspace& operator=(const Workspace&) = delete;
 };
 
+// Runs f with the GIL released; held again also where f throws.
 template <class F>
 int32_t without_gil(F f) {
-  PyThreadState* st = PyEval_SaveThread();
-  const int32_t rc = f();
-  PyEval_RestoreThread(st);
-  return rc;
+  struct Release {
+    PyThreadState* st = PyEval_SaveThread();
+    ~Release() { PyEval_RestoreThread(st); }
+  } release;
+  return f();
 }
 
 // Runs a call body: Slow, torch's exceptions and Python errors become None.
